@@ -29,7 +29,7 @@ MIN_LOG_N, MAX_LOG_N = 7, 17
 MIN_BITS, MAX_BITS = 128, 55904
 MIX_LOG_N = {"batch": (10, 13), "served": (12, 15)}
 MIX_LIMBS = {"batch": (8, 128), "served": (16, 512)}
-SERVED_BUDGET = 8 << 30  # device bytes of the temporary server
+SERVED_BUDGET = 2 << 30  # device bytes of the temporary server
 
 
 def listed():
