@@ -378,8 +378,8 @@ pm_status pm_debug_stage(pm_plan* plan, const uint32_t* a, const uint32_t* b, in
                     v[k * s.n + i] = tiles[(((i >> 8) * ksteps + k / 16) * 256 + (i & 255)) * 16 + k % 16] ^ 0x80808080u;
         } else {
             // device rows have stride n_pad; the tap returns rows of exactly N
-            const size_t elem = stage == PM_STAGE_WORDS ? 8 : 4;
-            if (stage == PM_STAGE_WORDS && pm::words_by_coefficient(s)) {
+            const size_t elem = 4;
+            if (stage == PM_STAGE_WORDS) {
                 // coefficient-major on the device: transpose into the tap's [crt_words][N]
                 const size_t ws = pm::word_stride(s);
                 std::vector<int64_t> sums(size_t(s.n) * ws);
@@ -389,10 +389,6 @@ pm_status pm_debug_stage(pm_plan* plan, const uint32_t* a, const uint32_t* b, in
                 int64_t* w = static_cast<int64_t*>(out);
                 for (size_t j = 0; j < s.crt_words; ++j)
                     for (size_t i = 0; i < s.n; ++i) w[j * s.n + i] = sums[i * ws + j];
-            } else if (stage == PM_STAGE_WORDS) {
-                hip_check(hipMemcpy2DAsync(out, s.n * elem, plan->work.words, size_t(s.n_pad) * elem, s.n * elem,
-                                           s.crt_words, hipMemcpyDeviceToHost, st),
-                          "copy stage");
             } else {  // residues of a then b; the b plane starts r_pad rows in
                 for (size_t op = 0; op < 2; ++op)
                     hip_check(hipMemcpy2DAsync(static_cast<uint8_t*>(out) + op * s.r * s.n * elem, s.n * elem,

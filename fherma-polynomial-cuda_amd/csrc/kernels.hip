@@ -371,12 +371,10 @@ __global__ __launch_bounds__(512) void conversion_gemm(const int8_t* __restrict_
 // ---------------------------------------------------------------------------
 // 5. CRT GEMM: G[c][i] = sum_{k,d} w[c][4k+d] * (byte_d(v_{k,i}) - 128),
 //    D_j(i) = sum_t 256^t G[4j+t][i]   (int64, exact)
-//    stored word-major words[j][i] (row stride n_pad), or, for the
-//    wave-per-coefficient reconstruction, coefficient-major words[i][j] (row
-//    stride ws): a wave's 4 x 16 words of 16 coefficients are then 128-byte
-//    runs per coefficient, written one after another.
+//    stored coefficient-major words[i][j] (row stride ws): a wave's 4 x 16
+//    words of 16 coefficients are 128-byte runs per coefficient, written one
+//    after another.
 // ---------------------------------------------------------------------------
-template <bool kByCoefficient>
 __device__ __forceinline__ void crt_body(const int8_t* __restrict__ wtiles, const int8_t* __restrict__ rtiles,
                                          int64_t* __restrict__ words, uint32_t n, uint32_t n_pad, uint32_t crt_rows,
                                          uint32_t ksteps, uint32_t crt_words, uint32_t ws, TileSet ts,
@@ -400,39 +398,24 @@ __device__ __forceinline__ void crt_body(const int8_t* __restrict__ wtiles, cons
 
     const DigitScales ds = digit_scales();
     const uint32_t m0 = tm * kTile + wm * kWaveRows, c0 = tn * kTile + wn * kWaveCols;
-    if constexpr (kByCoefficient) {
 #pragma unroll
-        for (uint32_t ni = 0; ni < kWaveN; ++ni) {
-            const uint32_t coef = c0 + ni * 16 + (lane & 15);
-            int64_t* out = words + size_t(coef) * ws;
-#pragma unroll
-            for (uint32_t mi = 0; mi < kWaveM; ++mi) {
-                const uint32_t word = (m0 + mi * 16) / 4 + (lane >> 4);
-                if (word < crt_words && coef < n) out[word] = combine4(acc[mi][ni], ds);
-            }
-        }
-    } else {
+    for (uint32_t ni = 0; ni < kWaveN; ++ni) {
+        const uint32_t coef = c0 + ni * 16 + (lane & 15);
+        int64_t* out = words + size_t(coef) * ws;
 #pragma unroll
         for (uint32_t mi = 0; mi < kWaveM; ++mi) {
             const uint32_t word = (m0 + mi * 16) / 4 + (lane >> 4);
-            if (word >= crt_words) continue;
-            int64_t* out = words + size_t(word) * n_pad;
-#pragma unroll
-            for (uint32_t ni = 0; ni < kWaveN; ++ni) {
-                const uint32_t coef = c0 + ni * 16 + (lane & 15);
-                if (coef < n) out[coef] = combine4(acc[mi][ni], ds);
-            }
+            if (word < crt_words && coef < n) out[word] = combine4(acc[mi][ni], ds);
         }
     }
 }
 
-template <bool kByCoefficient>
 __global__ __launch_bounds__(512) void crt_gemm(const int8_t* __restrict__ wtiles,
                                                 const int8_t* __restrict__ rtiles,
                                                 int64_t* __restrict__ words, uint32_t n, uint32_t n_pad,
                                                 uint32_t crt_rows, uint32_t ksteps, uint32_t crt_words,
                                                 uint32_t ws, TileSet ts) {
-    crt_body<kByCoefficient>(wtiles, rtiles, words, n, n_pad, crt_rows, ksteps, crt_words, ws, ts, blockIdx.x);
+    crt_body(wtiles, rtiles, words, n, n_pad, crt_rows, ksteps, crt_words, ws, ts, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -895,162 +878,6 @@ __global__ __launch_bounds__(256) void ntt_rows_2048(uint32_t* __restrict__ plan
 }
 
 // ---------------------------------------------------------------------------
-// 6. reconstruction: one lane per coefficient, for q of up to 62 limbs (T of at
-// most 64 words), words in [j][n_pad] layout.  Output row k*256 + u is
-// coefficient tile_at(ts, k)*256 + u.
-// ---------------------------------------------------------------------------
-struct ReconstructArgs {
-    uint32_t n, n_pad, limbs, t_words;
-    TileSet ts;
-    uint32_t s_shift, k_shift;
-    uint64_t mu;
-};
-
-__device__ __forceinline__ void reconstruct_body(const int64_t* __restrict__ words, uint32_t* __restrict__ tsc,
-                                                 uint32_t* __restrict__ c, const uint32_t* __restrict__ q,
-                                                 const uint32_t* __restrict__ neg_p,
-                                                 const uint32_t* __restrict__ corr_t,
-                                                 const uint32_t* __restrict__ corr_e, ReconstructArgs args,
-                                                 uint32_t bx) {
-    __shared__ uint32_t tile[64][65];
-    // Output rows k0 .. k0+63 lie in one tile of the set: coefficients i0 .. i0+63.
-    const uint32_t lane = threadIdx.x, k0 = bx * 64;
-    const uint32_t i0 = tile_at(args.ts, k0 / 256) * 256 + k0 % 256, i = i0 + lane;
-    const uint32_t ps = args.n_pad, L = args.limbs, tw = args.t_words;
-    const bool valid = i < args.n;
-    const uint32_t ic = valid ? i : 0;  // clamp reads of idle lanes
-
-    // K = floor((E + 2^63) / 2^64), E = sum_j 2^32j words[L+1+j] + corr_e
-    uint32_t ew[4];
-    {
-        int64_t carry = 0;
-        for (uint32_t j = 0; j < 4; ++j) {
-            int64_t x = (j < 3 ? words[size_t(L + 1 + j) * ps + ic] : 0) + int64_t(corr_e[j]) + carry;
-            ew[j] = uint32_t(uint64_t(x));
-            carry = x >> 32;
-        }
-    }
-    const uint64_t kq = uint64_t(ew[2]) + (uint64_t(ew[3]) << 32) + ((uint64_t(ew[1]) + 0x80000000ull) >> 32);
-
-    // Pass 1: T = sum_j 2^32j words[j] + corr_t + K*R, carried into 32-bit words.
-    // One lane owns a whole coefficient, so memory-level parallelism comes from
-    // running the loads ahead of the carry chain: two groups of kG1 words
-    // alternate, one in flight while the other is carried.
-    const uint32_t sw = args.s_shift / 32, sb = args.s_shift % 32;
-    uint32_t top[3] = {0, 0, 0};
-    {
-        constexpr uint32_t kG1 = 32;
-        int64_t da[kG1], db[kG1];
-        int64_t carry = 0;
-        auto fetch = [&](int64_t (&d)[kG1], uint32_t j0) {
-#pragma unroll
-            for (uint32_t u = 0; u < kG1; ++u) {
-                const uint32_t j = j0 + u;
-                d[u] = j <= L && j < tw ? words[size_t(j) * ps + ic] : 0;
-            }
-        };
-        auto carry_group = [&](const int64_t (&d)[kG1], uint32_t j0) {
-#pragma unroll
-            for (uint32_t u = 0; u < kG1; ++u) {
-                const uint32_t j = j0 + u;
-                if (j >= tw) break;
-                int64_t x = d[u] + int64_t(corr_t[j]) + carry;
-                if (j < L) x += int64_t(kq) * int64_t(neg_p[j]);
-                const uint32_t tj = uint32_t(uint64_t(x));
-                carry = x >> 32;
-                if (valid) tsc[size_t(j) * ps + ic] = tj;
-                // the three words Barrett reads; compares, not a runtime index (which would spill)
-                if (j == sw) top[0] = tj;
-                if (j == sw + 1) top[1] = tj;
-                if (j == sw + 2) top[2] = tj;
-            }
-        };
-        fetch(da, 0);
-        for (uint32_t j0 = 0; j0 < tw; j0 += 2 * kG1) {
-            if (j0 + kG1 < tw) fetch(db, j0 + kG1);
-            carry_group(da, j0);
-            if (j0 + kG1 >= tw) break;
-            if (j0 + 2 * kG1 < tw) fetch(da, j0 + 2 * kG1);
-            carry_group(db, j0 + kG1);
-        }
-    }
-    const unsigned __int128 topv = (unsigned __int128)top[0] | ((unsigned __int128)top[1] << 32) |
-                                   ((unsigned __int128)top[2] << 64);
-    const uint64_t t_scaled = uint64_t(topv >> sb);
-    const uint64_t qe = uint64_t(((unsigned __int128)t_scaled * args.mu) >> args.k_shift);
-
-    // Pass 2: rem = T - qe*q (in [0, 2q)) into an LDS row per lane, in two
-    // halves of 32 words (the second in flight while the first is reduced); a
-    // second borrow chain tracks rem - q, and when rem >= q the row is reduced
-    // once more in LDS.  The block's rows are then stored as one contiguous run
-    // of words: c is written once and never read back, so it may be pinned host
-    // memory.
-    {
-        uint64_t pc = 0;
-        uint32_t bo = 0, bo2 = 0;
-        constexpr uint32_t kH = 32;
-        uint32_t ta[kH], tb[kH];
-        auto fetch = [&](uint32_t (&t)[kH], uint32_t j0) {
-#pragma unroll
-            for (uint32_t u = 0; u < kH; ++u) t[u] = j0 + u < tw ? tsc[size_t(j0 + u) * ps + ic] : 0;
-        };
-        auto reduce_half = [&](const uint32_t (&t)[kH], uint32_t j0, uint32_t col0) {
-#pragma unroll
-            for (uint32_t u = 0; u < kH; ++u) {
-                const uint32_t j = j0 + u;
-                if (j >= tw) break;
-                const uint32_t qj = j < L ? q[j] : 0;
-                const unsigned __int128 pr = (unsigned __int128)qe * qj + pc;
-                const uint32_t x = uint32_t(pr);
-                pc = uint64_t(pr >> 32);
-                const uint64_t d = uint64_t(t[u]) - x - bo;
-                const uint32_t rj = uint32_t(d);
-                bo = uint32_t(d >> 63);
-                const uint64_t d2 = uint64_t(rj) - qj - bo2;
-                bo2 = uint32_t(d2 >> 63);
-                tile[lane][col0 + u] = rj;
-            }
-        };
-        fetch(ta, 0);
-        if (kH < tw) fetch(tb, kH);
-        reduce_half(ta, 0, 0);
-        if (kH < tw) reduce_half(tb, kH, kH);
-        if (bo2 == 0) {
-            uint32_t borrow = 0;
-            for (uint32_t j = 0; j < L; ++j) {
-                const uint64_t d = uint64_t(tile[lane][j]) - q[j] - borrow;
-                tile[lane][j] = uint32_t(d);
-                borrow = uint32_t(d >> 63);
-            }
-        }
-        __syncthreads();
-        const uint32_t rows = i0 < args.n ? (args.n - i0 < 64 ? args.n - i0 : 64) : 0;
-        uint32_t* out = c + size_t(k0) * L;
-        const uint32_t dq = 64 / L, dr = 64 % L;  // (row, col) of word k, stepped by 64 words
-        uint32_t row = lane / L, col = lane % L;
-        for (uint32_t k = lane; k < rows * L; k += 64) {
-            out[k] = tile[row][col];
-            row += dq;
-            col += dr;
-            if (col >= L) {
-                col -= L;
-                ++row;
-            }
-        }
-    }
-}
-
-__global__ __launch_bounds__(64) void reconstruct(const int64_t* __restrict__ words,
-                                                  uint32_t* __restrict__ tsc, uint32_t* __restrict__ c,
-                                                  const uint32_t* __restrict__ q,
-                                                  const uint32_t* __restrict__ neg_p,
-                                                  const uint32_t* __restrict__ corr_t,
-                                                  const uint32_t* __restrict__ corr_e,
-                                                  ReconstructArgs args) {
-    reconstruct_body(words, tsc, c, q, neg_p, corr_t, corr_e, args, blockIdx.x);
-}
-
-// ---------------------------------------------------------------------------
 // 6'. reconstruction, one wave per coefficient (q wider than 62 limbs): the
 // coefficient's CRT word sums are coefficient-major (words[i][0 .. L+3]) and
 // each lane takes one of 64 consecutive words per round, so every round is one
@@ -1228,6 +1055,285 @@ __global__ __launch_bounds__(256) void reconstruct_waves(const int64_t* __restri
 }
 
 // ---------------------------------------------------------------------------
+// 5+6. CRT GEMM and reconstruction in one kernel, for q of up to 60 limbs (at
+// most 64 word sums): a block of NW waves owns 16 NW coefficients and all
+// their word sums, so the sums never leave the CU.
+//
+//  * GEMM: every wave holds 64 weight rows (16 word sums) x 16 WM coefficients;
+//    WM waves cover the word sums (16 WM >= crt_words), the others split the
+//    coefficients.  The block's residue bytes (all K steps) come in by
+//    direct-to-LDS loads behind one barrier; the weights are read as MFMA
+//    fragments straight from global memory, two K steps ahead.  Only the K
+//    steps that hold primes run (the padded ones have zero weights).
+//  * The int64 word sums go to LDS, coefficient-major, over the operand bytes.
+//  * One lane per coefficient forms K and the Barrett estimate Qe, by the
+//    formulas of reconstruct_waves.
+//  * Then G = 4 WM lanes per coefficient, four consecutive words each: a lane
+//    carries through its own words and hands its carry to the next lane (a row
+//    shift within 16 lanes); a second hand-over happens only when four words in
+//    a row ripple.  A Qe that was off (by two at most) is mended by adding or
+//    subtracting q in place.
+//  * c is staged in LDS and stored as one contiguous run of words, each once,
+//    so c may be pinned host memory.
+// What bounds it at N = 65536 with 55 limbs (23.4 us, of which 17-19 us inside
+// a block): the weight fragments' way from L2 (7 us: 67 MB, every block reads
+// all of them) and the carry chains (4 us).  It replaces a CRT GEMM that wrote
+// 8 (L+4) bytes per coefficient and a kernel that walked them with one lane per
+// coefficient: 15.7 + 27.9 us there, 6.7 + 7.1 against 4.2 us at N = 1024 with
+// 8 limbs, 13.8 + 8.0 against 10.0 us at N = 131072 with 4.
+// ---------------------------------------------------------------------------
+struct CrtFusedArgs {
+    uint32_t n, limbs, t_words;
+    uint32_t ksteps, kstride;  // K steps that hold primes; K steps of a residue tile
+    TileSet ts;                // output row k*256 + u is coefficient tile_at(ts, k)*256 + u
+    uint32_t top_m, top_e, k_shift;
+    uint64_t mu;
+};
+
+constexpr uint32_t fused_row_words(uint32_t wm) { return 16 * wm + 2; }  // int64 per coefficient, 16-byte rows
+
+constexpr size_t fused_lds_bytes(uint32_t wm, uint32_t nw, uint32_t ksteps) {
+    const size_t operands = size_t(ksteps) * 16 * nw * kTK, sums = size_t(16) * nw * fused_row_words(wm) * 8;
+    return operands > sums ? operands : sums;
+}
+
+typedef uint32_t u32_alias __attribute__((may_alias));
+
+template <int WM, int NW>
+__device__ __forceinline__ void crt_reconstruct_body(const int8_t* __restrict__ wtiles,
+                                                     const int8_t* __restrict__ rtiles, uint32_t* __restrict__ c,
+                                                     const uint32_t* __restrict__ q,
+                                                     const uint32_t* __restrict__ neg_p,
+                                                     const uint32_t* __restrict__ corr_t,
+                                                     const uint32_t* __restrict__ corr_e, const CrtFusedArgs& args,
+                                                     uint32_t bx, int8_t* lds) {
+    constexpr uint32_t NT = WM, G = 4 * WM, S = fused_row_words(WM), T = 16 * NW, NTH = 64 * NW;
+    __shared__ uint64_t quotient[T];
+    __shared__ uint32_t multiple[T];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t wm = wave % WM, wn = wave / WM;
+    const uint32_t L = args.limbs, tw = args.t_words, ksteps = args.ksteps;
+    const uint32_t k0 = bx * T, tile = tile_at(args.ts, k0 / kTile), i0 = tile * kTile + k0 % kTile;
+
+    // operand bytes: slot tid of a K step holds row tid>>2, its chunk swizzled as in swz
+    {
+        const uint32_t row = tid >> 2, chunk = (tid & 3) ^ ((row >> 1) & 3);
+        const int8_t* src = rtiles + size_t(tile) * args.kstride * kTileBytes + (k0 % kTile + row) * kTK + chunk * 16;
+        for (uint32_t ks = 0; ks < ksteps; ++ks)
+            __builtin_amdgcn_global_load_lds(reinterpret_cast<const void*>(src + size_t(ks) * kTileBytes),
+                                             (__attribute__((address_space(3))) void*)(lds + ks * (T * kTK) + wave * 1024),
+                                             16, 0, 0);
+    }
+    const v4i* ap = reinterpret_cast<const v4i*>(wtiles + (wm * kWaveRows + (lane & 15)) * kTK + (lane >> 4) * 16);
+    v4i acc[kWaveM][NT], f0[kWaveM], f1[kWaveM], f2[kWaveM];
+    auto load_a = [&](uint32_t ks, v4i (&f)[kWaveM]) {
+#pragma unroll
+        for (uint32_t mi = 0; mi < kWaveM; ++mi) f[mi] = ap[size_t(ks) * (kTileBytes / 16) + mi * 64];
+    };
+    load_a(0, f0);
+    load_a(ksteps > 1 ? 1 : 0, f1);
+#pragma unroll
+    for (uint32_t mi = 0; mi < kWaveM; ++mi)
+#pragma unroll
+        for (uint32_t ni = 0; ni < NT; ++ni) acc[mi][ni] = v4i{0, 0, 0, 0};
+    __syncthreads();
+    auto step = [&](uint32_t ks, const v4i (&fa)[kWaveM], v4i (&refill)[kWaveM]) {
+        load_a(ks + 2 < ksteps ? ks + 2 : ksteps - 1, refill);  // past the end: the last step again
+        v4i fb[NT];
+#pragma unroll
+        for (uint32_t ni = 0; ni < NT; ++ni)
+            fb[ni] = *reinterpret_cast<const v4i*>(lds + ks * (T * kTK) +
+                                                   swz((wn * NT + ni) * 16 + (lane & 15), lane >> 4));
+#pragma unroll
+        for (uint32_t mi = 0; mi < kWaveM; ++mi)
+#pragma unroll
+            for (uint32_t ni = 0; ni < NT; ++ni)
+                acc[mi][ni] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[mi], fb[ni], acc[mi][ni], 0, 0, 0);
+    };
+    uint32_t ks = 0;  // three fragment sets in rotation
+    for (; ks + 3 <= ksteps; ks += 3) {
+        step(ks, f0, f2);
+        step(ks + 1, f1, f0);
+        step(ks + 2, f2, f1);
+    }
+    if (ks < ksteps) step(ks, f0, f2);
+    if (ks + 1 < ksteps) step(ks + 1, f1, f0);
+    // this lane's four words of the constants
+    const uint32_t g = tid % G, j0 = 4 * g;
+    // (every load unconditional, its index clamped, the value selected after)
+    uint32_t ct[4], np[4], qv[6];  // qv[u + 2] = q[j0 + u], two words below included
+#pragma unroll
+    for (uint32_t u = 0; u < 4; ++u) {
+        const uint32_t j = j0 + u;
+        const uint32_t cv = corr_t[j < tw ? j : tw - 1], nv = neg_p[j < L ? j : L - 1];
+        ct[u] = j < tw ? cv : 0;
+        np[u] = j < L ? nv : 0;
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < 6; ++u) {
+        const uint32_t j = j0 + u - 2;  // wraps above L below word 0
+        const uint32_t v = q[j < L ? j : L - 1];
+        qv[u] = j < L ? v : 0;
+    }
+    uint32_t top_c[4], top_n[4];  // the Barrett window's constants, the same for every lane
+#pragma unroll
+    for (uint32_t t = 0; t < 4; ++t) {
+        const uint32_t j = args.top_m + t;
+        const uint32_t cv = corr_t[j < tw ? j : tw - 1], nv = neg_p[j < L ? j : L - 1];
+        top_c[t] = j < tw ? cv : 0;
+        top_n[t] = j < L ? nv : 0;
+    }
+    uint32_t ce[4];
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) ce[j] = corr_e[j];
+    __syncthreads();  // every wave has read the operand bytes; the sums go over them
+    int64_t* sums = reinterpret_cast<int64_t*>(lds);
+    const DigitScales ds = digit_scales();
+#pragma unroll
+    for (uint32_t ni = 0; ni < NT; ++ni)
+#pragma unroll
+        for (uint32_t mi = 0; mi < kWaveM; ++mi)
+            sums[((wn * NT + ni) * 16 + (lane & 15)) * S + wm * 16 + mi * 4 + (lane >> 4)] = combine4(acc[mi][ni], ds);
+    __syncthreads();
+
+    const uint32_t shift = lane & ~(G - 1), last = lane | (G - 1);
+    const uint64_t group_mask = (uint64_t(1) << G) - 1;
+    // The lane's words plus carry-in `cin`; returns the carry out.
+    auto add_carry = [](uint32_t (&w)[4], int32_t cin) {
+        int64_t t = cin;
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+            t += int64_t(w[u]);
+            w[u] = uint32_t(uint64_t(t));
+            t >>= 32;
+        }
+        return int32_t(t);
+    };
+    // Passes each lane's carry to the next lane of its group until none is left;
+    // the last lane's carries add up in `top` (0 on the other lanes).
+    auto settle = [&](uint32_t (&w)[4], int32_t carry, int32_t& top) {
+        for (;;) {
+            if (g == G - 1) top += carry;
+            int32_t cin = __builtin_amdgcn_update_dpp(0, carry, 0x111, 0xF, 0xF, true);  // row_shr:1
+            if (g == 0) cin = 0;
+            if (!__ballot(cin != 0)) break;
+            carry = add_carry(w, cin);
+        }
+    };
+    // K and the Barrett quotient Qe: one lane per coefficient, for all of them
+    if (tid < T) {
+        const int64_t* d = sums + tid * S;
+        int64_t e[3], dt[4];
+#pragma unroll
+        for (uint32_t j = 0; j < 3; ++j) e[j] = d[L + 1 + j];
+#pragma unroll
+        for (uint32_t t = 0; t < 4; ++t) {
+            const uint32_t j = args.top_m + t;
+            dt[t] = d[j <= L ? j : L];
+            if (j > L) dt[t] = 0;
+        }
+        // K = floor((E + 2^63) / 2^64)
+        uint32_t ew[4];
+        int64_t carry = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+            const int64_t x = (j < 3 ? e[j] : 0) + int64_t(ce[j]) + carry;
+            ew[j] = uint32_t(uint64_t(x));
+            carry = x >> 32;
+        }
+        const uint32_t k32 = uint32_t(ew[2] + ((uint64_t(ew[1]) + 0x80000000ull) >> 32));
+        // the four words at top_m (words past the last are zero)
+        unsigned __int128 sum = 0;
+#pragma unroll
+        for (uint32_t t = 0; t < 4; ++t) {
+            const int64_t x = dt[t] + int64_t(top_c[t]) + int64_t(uint64_t(k32) * top_n[t]);
+            sum += (unsigned __int128)(__int128)x << (32 * t);
+        }
+        __int128 ts = __int128(sum) >> args.top_e;
+        if (ts < 0) ts = 0;
+        quotient[tid] = uint64_t(((unsigned __int128)uint64_t(ts) * args.mu) >> args.k_shift);
+        multiple[tid] = k32;
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (uint32_t cl = tid / G; cl < T; cl += 64 * NW / G) {  // whole waves: T G is a multiple of the threads
+        const int64_t* d = sums + cl * S;
+        const uint64_t qe = quotient[cl];
+        const uint32_t k32 = multiple[cl];
+        // R = T - Qe*q: this lane's four words and the carry out of them
+        const uint64_t q0 = uint32_t(qe), q1 = uint32_t(qe >> 32);
+        uint32_t w[4];
+        int32_t top = 0;
+        {
+            uint64_t pa = q0 * qv[1], pc = q1 * qv[1], pc2 = q1 * qv[0];
+            int64_t carry = 0;
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) {
+                const uint64_t a = q0 * qv[u + 2];
+                const int64_t sub = int64_t(uint32_t(a)) + int64_t(pa >> 32) + int64_t(uint32_t(pc)) + int64_t(pc2 >> 32);
+                const int64_t dj = d[j0 + u];  // words past L hold E or the row's pad
+                carry += (j0 + u <= L ? dj : 0) + int64_t(ct[u]) + int64_t(uint64_t(k32) * np[u]) - sub;
+                w[u] = uint32_t(uint64_t(carry));
+                carry >>= 32;
+                pa = a, pc2 = pc, pc = q1 * qv[u + 2];
+            }
+            settle(w, int32_t(carry), top);
+        }
+        const bool valid = i0 + cl < args.n;
+        for (int pass = 0; pass < 6; ++pass) {
+            bool gt = false, lt = false;
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) {  // the highest differing word decides
+                if (w[u] != qv[u + 2]) gt = w[u] > qv[u + 2], lt = !gt;
+            }
+            const uint64_t gm = (__ballot(gt) >> shift) & group_mask, lm = (__ballot(lt) >> shift) & group_mask;
+            const bool neg = (__ballot(top < 0) >> last) & 1, pos = (__ballot(top > 0) >> last) & 1;
+            const int32_t adj = !valid ? 0 : neg ? 1 : (pos || gm >= lm) ? -1 : 0;
+            if (!__ballot(adj != 0)) break;
+            int64_t carry = 0;
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) {
+                carry += int64_t(w[u]) + (adj > 0 ? int64_t(qv[u + 2]) : adj < 0 ? -int64_t(qv[u + 2]) : 0);
+                w[u] = uint32_t(uint64_t(carry));
+                carry >>= 32;
+            }
+            settle(w, int32_t(carry), top);
+        }
+        // c over the coefficient's own sums (its lanes have read them all)
+        u32_alias* cw = reinterpret_cast<u32_alias*>(lds + size_t(cl) * S * 8);
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u)
+            if (j0 + u < L) cw[j0 + u] = w[u];
+    }
+    __syncthreads();
+    const uint32_t rows = i0 < args.n ? (args.n - i0 < T ? args.n - i0 : T) : 0;
+    uint32_t* out = c + size_t(k0) * L;
+    const u32_alias* staged = reinterpret_cast<const u32_alias*>(lds);
+    const uint32_t dq = NTH / L, dr = NTH % L;  // (row, column) of word k, stepped by NTH words
+    uint32_t row = tid / L, col = tid % L;
+    for (uint32_t k = tid; k < rows * L; k += NTH) {
+        out[k] = staged[row * (2 * S) + col];
+        row += dq;
+        col += dr;
+        if (col >= L) {
+            col -= L;
+            ++row;
+        }
+    }
+}
+
+template <int WM, int NW>
+__global__ __launch_bounds__(64 * NW, 4) void crt_reconstruct(const int8_t* __restrict__ wtiles,
+                                                       const int8_t* __restrict__ rtiles, uint32_t* __restrict__ c,
+                                                       const uint32_t* __restrict__ q,
+                                                       const uint32_t* __restrict__ neg_p,
+                                                       const uint32_t* __restrict__ corr_t,
+                                                       const uint32_t* __restrict__ corr_e, CrtFusedArgs args) {
+    extern __shared__ __attribute__((aligned(16))) int8_t fused_lds[];
+    crt_reconstruct_body<WM, NW>(wtiles, rtiles, c, q, neg_p, corr_t, corr_e, args, blockIdx.x, fused_lds);
+}
+
+// ---------------------------------------------------------------------------
 // 6''. Grouped launches: one stage of many products in one launch.  Entry j of
 // a launch owns blocks [start[j], start[j+1]) and runs them as the blocks of
 // product item[j]'s own launch of that stage (kernels.hpp, GroupItem).
@@ -1308,19 +1414,21 @@ __global__ __launch_bounds__(256) void inverse_tiles_group(GroupLaunch g) {
                              it.r_pad / 16, it.rtiles, 0, local % nx, local / nx, nx);
 }
 
-template <bool kByCoefficient>
 __global__ __launch_bounds__(512) void crt_group(GroupLaunch g) {
     uint32_t local;
     const GroupItem& it = group_entry(g, local);
-    crt_body<kByCoefficient>(it.wcrt, it.rtiles, it.words, it.n, it.n_pad, it.crt_rows, it.crt_k / kTK, it.crt_words,
-                             it.ws, every_tile(it), local);
+    crt_body(it.wcrt, it.rtiles, it.words, it.n, it.n_pad, it.crt_rows, it.crt_k / kTK, it.crt_words, it.ws,
+             every_tile(it), local);
 }
 
-__global__ __launch_bounds__(64) void reconstruct_group(GroupLaunch g) {
+template <int WM, int NW>
+__global__ __launch_bounds__(64 * NW, 4) void crt_reconstruct_group(GroupLaunch g) {
+    extern __shared__ __attribute__((aligned(16))) int8_t fused_lds[];
     uint32_t local;
     const GroupItem& it = group_entry(g, local);
-    const ReconstructArgs args{it.n, it.n_pad, it.limbs, it.t_words, every_tile(it), it.s_shift, it.k_shift, it.mu};
-    reconstruct_body(it.words, it.t_scratch, it.c, it.q, it.neg_p, it.corr_t, it.corr_e, args, local);
+    const CrtFusedArgs args{it.n, it.limbs, it.t_words, (it.r + 15) / 16, it.r_pad / 16, every_tile(it),
+                            it.top_m, it.top_e, it.k_shift, it.mu};
+    crt_reconstruct_body<WM, NW>(it.wcrt, it.rtiles, it.c, it.q, it.neg_p, it.corr_t, it.corr_e, args, local, fused_lds);
 }
 
 __global__ __launch_bounds__(256) void reconstruct_waves_group(GroupLaunch g) {
@@ -1664,33 +1772,59 @@ void launch_crt(const Shape& s, const DeviceTables& t, const int8_t* rtiles, int
                 hipStream_t stream) {
     check_tiles(s, ts, "crt_gemm");
     const uint32_t blocks = (s.crt_rows / kTile) * ts.count;
-    if (words_by_coefficient(s))
-        hipLaunchKernelGGL(crt_gemm<true>, dim3(blocks), dim3(kGemmThreads), 0, stream, t.wcrt, rtiles, words,
-                           s.n, s.n_pad, s.crt_rows, s.crt_k / kTK, s.crt_words, word_stride(s), ts);
-    else
-        hipLaunchKernelGGL(crt_gemm<false>, dim3(blocks), dim3(kGemmThreads), 0, stream, t.wcrt, rtiles, words,
-                           s.n, s.n_pad, s.crt_rows, s.crt_k / kTK, s.crt_words, word_stride(s), ts);
+    hipLaunchKernelGGL(crt_gemm, dim3(blocks), dim3(kGemmThreads), 0, stream, t.wcrt, rtiles, words, s.n, s.n_pad,
+                       s.crt_rows, s.crt_k / kTK, s.crt_words, word_stride(s), ts);
     check_launch("crt_gemm");
 }
 
-void launch_reconstruct(const Shape& s, const DeviceTables& t, const int64_t* words, uint32_t* t_scratch,
-                        uint32_t* c, const TileSet& ts, hipStream_t stream) {
-    check_tiles(s, ts, "reconstruct");
-    if (words_by_coefficient(s)) {
-        // Barrett window: the four words of x from m up (m = floor(s/32) - 1, or 0 below s = 64)
-        const uint32_t top_m = s.s_shift >= 64 ? s.s_shift / 32 - 1 : 0;
-        WaveReconstructArgs args{s.n, word_stride(s), s.limbs, s.t_words, ts,
-                                 top_m, s.s_shift - 32 * top_m, s.k_shift, s.mu};
-        hipLaunchKernelGGL(reconstruct_waves, dim3(ts.count * 64), dim3(256), 0, stream, words, c, t.q, t.neg_p,
-                           t.corr_t, t.corr_e, args);
-        check_launch("reconstruct_waves");
-        return;
+namespace {
+
+// Barrett window: the four words of x from m up (m = floor(s/32) - 1, or 0 below s = 64)
+uint32_t barrett_top(const Shape& s) { return s.s_shift >= 64 ? s.s_shift / 32 - 1 : 0; }
+
+// Wave rows of the fused kernel: 16 word sums each.
+uint32_t fused_waves(uint32_t crt_words) { return crt_words <= 16 ? 1 : crt_words <= 32 ? 2 : 4; }
+
+}  // namespace
+
+void launch_crt_reconstruct(const Shape& s, const DeviceTables& t, const int8_t* rtiles, uint32_t* c,
+                            const TileSet& ts, hipStream_t stream) {
+    check_tiles(s, ts, "crt_reconstruct");
+    if (!reconstruct_fused(s)) throw std::logic_error("crt_reconstruct: more word sums than a block holds");
+    const uint32_t top_m = barrett_top(s), ksteps = (s.r + 15) / 16, wm = fused_waves(s.crt_words);
+    const CrtFusedArgs args{s.n, s.limbs, s.t_words, ksteps, s.r_pad / 16, ts, top_m, s.s_shift - 32 * top_m,
+                            s.k_shift, s.mu};
+#define PM_FUSED(W, NW)                                                                                          \
+    hipLaunchKernelGGL((crt_reconstruct<W, NW>), dim3(ts.count * (kTile / (16 * NW))), dim3(64 * NW),             \
+                       fused_lds_bytes(W, NW, ksteps), stream, t.wcrt, rtiles, c, t.q, t.neg_p, t.corr_t,         \
+                       t.corr_e, args)
+    // Blocks of eight waves read the weights half as often per coefficient (at
+    // N = 65536 with 55 limbs 23.4 us against 29.2 us with four waves); below
+    // 65536 coefficients there are too few of them, and smaller blocks start sooner.
+    const bool wide = ts.count >= 256;
+    if (wm == 1) {
+        if (wide) PM_FUSED(1, 8);
+        else PM_FUSED(1, 4);
+    } else if (wm == 2) {
+        if (wide) PM_FUSED(2, 8);
+        else PM_FUSED(2, 4);
+    } else {
+        if (wide) PM_FUSED(4, 8);
+        else PM_FUSED(4, 4);
     }
-    if (s.t_words > 64) throw std::logic_error("reconstruct: the lane-per-coefficient kernel takes T of 64 words at most");
-    ReconstructArgs args{s.n, s.n_pad, s.limbs, s.t_words, ts, s.s_shift, s.k_shift, s.mu};
-    hipLaunchKernelGGL(reconstruct, dim3(ts.count * 4), dim3(64), 0, stream, words, t_scratch, c, t.q, t.neg_p,
+#undef PM_FUSED
+    check_launch("crt_reconstruct");
+}
+
+void launch_reconstruct(const Shape& s, const DeviceTables& t, const int64_t* words, uint32_t* c, const TileSet& ts,
+                        hipStream_t stream) {
+    check_tiles(s, ts, "reconstruct");
+    const uint32_t top_m = barrett_top(s);
+    WaveReconstructArgs args{s.n, word_stride(s), s.limbs, s.t_words, ts,
+                             top_m, s.s_shift - 32 * top_m, s.k_shift, s.mu};
+    hipLaunchKernelGGL(reconstruct_waves, dim3(ts.count * 64), dim3(256), 0, stream, words, c, t.q, t.neg_p,
                        t.corr_t, t.corr_e, args);
-    check_launch("reconstruct");
+    check_launch("reconstruct_waves");
 }
 
 GroupItem group_item(const Shape& s, const DeviceTables& t, const DeviceWork& w, const uint32_t* a,
@@ -1701,13 +1835,13 @@ GroupItem group_item(const Shape& s, const DeviceTables& t, const DeviceWork& w,
     it.crt_words = s.crt_words, it.ws = word_stride(s), it.t_words = s.t_words;
     it.n1 = s.n1, it.n2 = s.n2, it.rows = s.rows, it.row_width = s.row_width;
     it.s_shift = s.s_shift, it.k_shift = s.k_shift;
-    it.top_m = s.s_shift >= 64 ? s.s_shift / 32 - 1 : 0;  // as launch_reconstruct
+    it.top_m = barrett_top(s);
     it.top_e = s.s_shift - 32 * it.top_m;
     it.mu = s.mu;
     it.consts = t.consts, it.wconv = t.wconv, it.tw_fwd = t.tw_fwd, it.tw_inv = t.tw_inv, it.wcrt = t.wcrt;
     it.q = t.q, it.neg_p = t.neg_p, it.corr_t = t.corr_t, it.corr_e = t.corr_e;
     it.a = a, it.b = b, it.c = c;
-    it.packed = w.packed, it.planes = w.planes, it.rtiles = w.rtiles, it.words = w.words, it.t_scratch = w.t_words;
+    it.packed = w.packed, it.planes = w.planes, it.rtiles = w.rtiles, it.words = w.words;
     return it;
 }
 
@@ -1722,10 +1856,11 @@ namespace {
 
 // Launches of one batch: pack, conversion, forward columns (one per row count),
 // rows (one per block size n1, and the LDS kernel), inverse columns (one per
-// row count), CRT GEMM (two word layouts), reconstruction (two kernels).
-constexpr size_t kGroupLaunches = 2 + 6 + 5 + 7 + 2 + 2;
+// row count), CRT GEMM with reconstruction (one per wave-row count), CRT GEMM,
+// reconstruction.
+constexpr size_t kGroupLaunches = 2 + 6 + 5 + 7 + 3 + 2;
 
-enum GroupKind { kPack, kConversion, kForward, kRows2048, kRowsProduct, kInverse, kCrt, kRecLane, kRecWave };
+enum GroupKind { kPack, kConversion, kForward, kRows2048, kRowsProduct, kInverse, kCrtRec, kCrt, kRecWave };
 
 size_t group_item_bytes(size_t count) { return (count * sizeof(GroupItem) + 255) / 256 * 256; }
 size_t group_table_words(size_t count) { return kGroupLaunches * (2 * count + 1); }
@@ -1765,7 +1900,9 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
             start[j] = uint32_t(total);
             item[j] = sel[j];
             total += blocks(items[sel[j]]);
-            lds = std::max<size_t>(lds, size_t(2) * items[sel[j]].row_width * 4);
+            const GroupItem& it = items[sel[j]];
+            lds = std::max<size_t>(lds, kind == kCrtRec ? fused_lds_bytes(variant, 4, (it.r + 15) / 16)
+                                                        : size_t(2) * it.row_width * 4);
         }
         if (total >= (uint64_t(1) << 31)) throw std::invalid_argument("launch_group: batch too large for one grid");
         start[sel.size()] = uint32_t(total);
@@ -1791,10 +1928,14 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
         add(kInverse, R, [&](const GroupItem& it) {
             return it.rows == R ? uint64_t(it.row_width / 16) * (it.r_pad / 16) : 0;
         });
-    add(kCrt, 0, [&](const GroupItem& it) { return it.t_words > 64 ? 0 : uint64_t(it.crt_rows / kTile) * ntiles(it); });
-    add(kCrt, 1, [&](const GroupItem& it) { return it.t_words > 64 ? uint64_t(it.crt_rows / kTile) * ntiles(it) : 0; });
-    add(kRecLane, 0, [&](const GroupItem& it) { return it.t_words > 64 ? 0 : 4 * ntiles(it); });
-    add(kRecWave, 0, [&](const GroupItem& it) { return it.t_words > 64 ? 64 * ntiles(it) : 0; });
+    for (uint32_t wm = 1; wm <= 4; wm *= 2)
+        add(kCrtRec, wm, [&](const GroupItem& it) {
+            return it.crt_words <= kFusedWords && fused_waves(it.crt_words) == wm ? 4 * ntiles(it) : 0;
+        });
+    add(kCrt, 0, [&](const GroupItem& it) {
+        return it.crt_words <= kFusedWords ? 0 : uint64_t(it.crt_rows / kTile) * ntiles(it);
+    });
+    add(kRecWave, 0, [&](const GroupItem& it) { return it.crt_words <= kFusedWords ? 0 : 64 * ntiles(it); });
     // the items and the work lists, one copy
     std::vector<char> upload(item_bytes + used * sizeof(uint32_t));
     std::memcpy(upload.data(), items.data(), count * sizeof(GroupItem));
@@ -1844,14 +1985,18 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
 #undef PM_GINV
                 }
                 break;
-            case kCrt:
-                if (L.variant)
-                    hipLaunchKernelGGL(crt_group<true>, grid, dim3(kGemmThreads), 0, stream, g);
-                else
-                    hipLaunchKernelGGL(crt_group<false>, grid, dim3(kGemmThreads), 0, stream, g);
+            case kCrtRec:
+                switch (L.variant) {
+#define PM_GFUSED(W)                                                                    \
+    case W:                                                                             \
+        hipLaunchKernelGGL((crt_reconstruct_group<W, 4>), grid, dim3(256), L.lds, stream, g); \
+        break;
+                    PM_GFUSED(1) PM_GFUSED(2) PM_GFUSED(4)
+#undef PM_GFUSED
+                }
                 break;
-            case kRecLane:
-                hipLaunchKernelGGL(reconstruct_group, grid, dim3(64), 0, stream, g);
+            case kCrt:
+                hipLaunchKernelGGL(crt_group, grid, dim3(kGemmThreads), 0, stream, g);
                 break;
             case kRecWave:
                 hipLaunchKernelGGL(reconstruct_waves_group, grid, dim3(256), 0, stream, g);
@@ -1939,7 +2084,7 @@ size_t work_bytes(const Shape& s) { return carve_work(s, nullptr, nullptr); }
 
 size_t carve_work(const Shape& s, uint8_t* base, DeviceWork* w) {
     const size_t packed = packed_operand_bytes(s);
-    const size_t half = size_t(s.r_pad > scratch_rows(s) ? s.r_pad : scratch_rows(s)) * s.n_pad;
+    const size_t half = size_t(s.r_pad) * s.n_pad;
     const size_t planes = 2 * half * sizeof(uint32_t);
     const size_t words = word_sum_elements(s) * sizeof(int64_t);
     auto round = [](size_t b) { return (b + 255) / 256 * 256; };
@@ -1947,7 +2092,6 @@ size_t carve_work(const Shape& s, uint8_t* base, DeviceWork* w) {
         w->packed = reinterpret_cast<int8_t*>(base);
         w->planes = reinterpret_cast<uint32_t*>(base + round(packed));
         w->rtiles = reinterpret_cast<int8_t*>(w->planes + half);
-        w->t_words = w->planes;
         w->words = reinterpret_cast<int64_t*>(base + round(packed) + round(planes));
     }
     return round(packed) + round(planes) + round(words);

@@ -32,22 +32,17 @@ struct DeviceWork {
     int8_t* packed = nullptr;    // [2][n_pad/256][conv_k/64][256][64] signed operand bytes
     uint32_t* planes = nullptr;  // [2][r_pad][n_pad] residues of a and b
     int8_t* rtiles = nullptr;    // CRT operand tiles of v_k (aliases the b plane, dead after the row stages)
-    int64_t* words = nullptr;    // CRT word sums: [crt_words][n_pad], or [n_pad][ws] (words_by_coefficient)
-    uint32_t* t_words = nullptr; // [t_words][n_pad] T scratch of the lane-per-coefficient reconstruction
-                                 // (aliases the a plane, dead after the CRT GEMM)
+    int64_t* words = nullptr;    // CRT word sums [n_pad][ws] (q wider than 60 limbs, and the debug tap)
 };
 
-// Layout of the CRT word sums.  Up to 62 limbs (t_words <= 64) one lane
-// reconstructs one coefficient and the sums are word-major [crt_words][n_pad];
-// wider q takes one wave per coefficient over coefficient-major sums
-// [n_pad][ws], ws = crt_words rounded up to 16 (128-byte rows).
-inline bool words_by_coefficient(const Shape& s) { return s.t_words > 64; }
-inline uint32_t word_stride(const Shape& s) { return words_by_coefficient(s) ? (s.crt_words + 15) / 16 * 16 : s.n_pad; }
-inline size_t word_sum_elements(const Shape& s) {
-    return words_by_coefficient(s) ? size_t(s.n_pad) * word_stride(s) : size_t(s.crt_words) * s.n_pad;
-}
-// Rows of the a plane the T scratch needs (the lane-per-coefficient reconstruction only).
-inline uint32_t scratch_rows(const Shape& s) { return words_by_coefficient(s) ? 0 : s.t_words; }
+// Up to 60 limbs (64 word sums) one kernel does the CRT GEMM and the
+// reconstruction, and the sums stay in LDS; wider q takes the GEMM, then one
+// wave per coefficient over coefficient-major sums [n_pad][ws] in memory, ws =
+// crt_words rounded up to 16 (128-byte rows) above 64 words.
+constexpr uint32_t kFusedWords = 64;
+inline bool reconstruct_fused(const Shape& s) { return s.crt_words <= kFusedWords; }
+inline uint32_t word_stride(const Shape& s) { return s.t_words > 64 ? (s.crt_words + 15) / 16 * 16 : s.crt_words; }
+inline size_t word_sum_elements(const Shape& s) { return size_t(s.n_pad) * word_stride(s); }
 
 // Static device workspace of pm_multiply_device_scratch: kScratchBytes per GPU,
 // held from the library's first plan on that GPU until the process ends.
@@ -90,17 +85,19 @@ void launch_ntt_rows_product(const Shape& s, const DeviceTables& t, uint32_t* pl
 // [n_pad/256][r_pad/16][256][64] (signed bytes) of those columns.
 void launch_ntt_inverse_columns(const Shape& s, const DeviceTables& t, uint32_t* planes, int8_t* rtiles,
                                 hipStream_t stream, uint32_t strip_begin = 0, uint32_t strip_end = ~0u);
+// CRT word sums of the coefficients of the tiles of `ts`, coefficient-major.
 void launch_crt(const Shape& s, const DeviceTables& t, const int8_t* rtiles, int64_t* words, const TileSet& ts,
                 hipStream_t stream);
 // Reconstructs the coefficients of the tiles of `ts`: output row k*256 + u of c
 // (L words each) is coefficient tile_at(ts, k)*256 + u; rows of coefficients at
-// or past N are not written.  When reconstruct_writes_once(s), each word of c
-// is written once, so c may well be pinned host memory; otherwise (q wider than
-// 62 limbs) a coefficient whose quotient estimate was off is written again by
-// a later pass.
-inline bool reconstruct_writes_once(const Shape& s) { return s.t_words <= 64; }
-void launch_reconstruct(const Shape& s, const DeviceTables& t, const int64_t* words, uint32_t* t_scratch,
-                        uint32_t* c, const TileSet& ts, hipStream_t stream);
+// or past N are not written.  launch_crt_reconstruct (reconstruct_fused(s))
+// takes the residue tiles and writes each word of c once, so c may well be
+// pinned host memory; launch_reconstruct takes the word sums, and a coefficient
+// whose quotient estimate was off is written again by a later pass.
+void launch_crt_reconstruct(const Shape& s, const DeviceTables& t, const int8_t* rtiles, uint32_t* c,
+                            const TileSet& ts, hipStream_t stream);
+void launch_reconstruct(const Shape& s, const DeviceTables& t, const int64_t* words, uint32_t* c, const TileSet& ts,
+                        hipStream_t stream);
 void launch_zero(uint32_t* c, size_t words, hipStream_t stream);
 
 // Grouped launches: every stage of a batch of device products (each its own
@@ -128,7 +125,6 @@ struct GroupItem {
     uint32_t* planes;
     int8_t* rtiles;
     int64_t* words;
-    uint32_t* t_scratch;
 };
 // The item of one plain product (a, b -> c on the working buffers w).
 GroupItem group_item(const Shape& s, const DeviceTables& t, const DeviceWork& w, const uint32_t* a,

@@ -338,19 +338,19 @@ struct pm_plan {
             // Output half, per chunk: the inverse column stages of the strips it
             // starts, its CRT GEMM, its reconstruction, then its D2H on the copy
             // stream, which overlaps the next chunk's GEMM.
-            const bool direct = pm::reconstruct_writes_once(s);
+            const bool direct = pm::reconstruct_fused(s);
             for (uint32_t ch = 0; ch < chunks.count; ++ch) {
                 const size_t rows = chunks.rows_of(ch), at = size_t(chunks.local[ch]) * L;
                 if (chunks.strips && chunks.inv_end[ch] > chunks.inv_begin[ch])
                     pm::launch_ntt_inverse_columns(s, tables, work.planes, work.rtiles, stream, chunks.inv_begin[ch],
                                                    chunks.inv_end[ch]);
-                pm::launch_crt(s, tables, work.rtiles, work.words, chunks.set[ch], stream);
-                pm::launch_reconstruct(s, tables, work.words, work.t_words, (direct ? lane->pin_out : io_c) + at,
-                                       chunks.set[ch], stream);
                 if (direct) {
+                    pm::launch_crt_reconstruct(s, tables, work.rtiles, lane->pin_out + at, chunks.set[ch], stream);
                     hip_check(hipEventRecord(lane->out_ready[ch], stream), "hipEventRecord");
                     continue;
                 }
+                pm::launch_crt(s, tables, work.rtiles, work.words, chunks.set[ch], stream);
+                pm::launch_reconstruct(s, tables, work.words, io_c + at, chunks.set[ch], stream);
                 // With two_streams the D2Hs alternate too (the input stream is idle
                 // by now), so that a chunk's D2H does not wait behind the previous
                 // one's completion event.  Where a chunk's conversion is long
@@ -449,12 +449,10 @@ struct pm_plan {
         tables.corr_e = upload(host.corr_e);
         work.packed = alloc<int8_t>(pm::packed_operand_bytes(s));
         // planes: [2][r_pad][n_pad].  After the row stages the b half is dead and
-        // receives the CRT operand tiles of v_k (exactly r_pad*n_pad words);
-        // after the CRT GEMM the a half is dead and holds T ([L+2][n_pad]).
-        const size_t half = size_t(std::max(s.r_pad, pm::scratch_rows(s))) * s.n_pad;
+        // receives the CRT operand tiles of v_k (exactly r_pad*n_pad words).
+        const size_t half = size_t(s.r_pad) * s.n_pad;
         work.planes = alloc<uint32_t>(2 * half);
         work.rtiles = reinterpret_cast<int8_t*>(work.planes + half);
-        work.t_words = work.planes;
         work.words = alloc<int64_t>(pm::word_sum_elements(s));
         // pinned staging of the host entry points is sized here, with the rest
         // of the plan, not inside the first product
@@ -551,10 +549,15 @@ struct pm_plan {
         pm::launch_ntt_inverse_columns(s, tables, w.planes, w.rtiles, st);
         mark(5);
         if (last == PM_STAGE_PRODUCT) return;
-        pm::launch_crt(s, tables, w.rtiles, w.words, all, st);
-        mark(6);
-        if (last == PM_STAGE_WORDS) return;
-        pm::launch_reconstruct(s, tables, w.words, w.t_words, c, all, st);
+        if (pm::reconstruct_fused(s) && last != PM_STAGE_WORDS) {  // reported as the CRT GEMM's time
+            pm::launch_crt_reconstruct(s, tables, w.rtiles, c, all, st);
+            mark(6);
+        } else {
+            pm::launch_crt(s, tables, w.rtiles, w.words, all, st);
+            mark(6);
+            if (last == PM_STAGE_WORDS) return;
+            pm::launch_reconstruct(s, tables, w.words, c, all, st);
+        }
         mark(7);
     }
 
@@ -595,7 +598,7 @@ inline size_t plan_footprint(const pm::HostPlan& h) {
     t += aligned_bytes(size_t(2) * s.conv_rows * s.conv_k) + 2 * aligned_bytes(r * s.n2 * 2 * 4) +
          aligned_bytes(size_t(s.crt_rows) * s.crt_k);
     t += 2 * aligned_bytes(size_t(s.limbs) * 4) + aligned_bytes(size_t(s.t_words) * 4) + aligned_bytes(4 * 4);
-    const size_t half = size_t(std::max(s.r_pad, pm::scratch_rows(s))) * s.n_pad;
+    const size_t half = size_t(s.r_pad) * s.n_pad;
     t += aligned_bytes(pm::packed_operand_bytes(s)) + aligned_bytes(2 * half * 4) +
          aligned_bytes(pm::word_sum_elements(s) * 8);
     return t;
