@@ -40,6 +40,7 @@ namespace {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+typedef uint32_t u32_alias __attribute__((may_alias));
 
 // GEMM block tile: 256 weight rows x 256 coefficients x 64 bytes of K, eight
 // waves in a 4x2 grid, each owning a 64x128 slab = 4x8 MFMA 16x16 tiles
@@ -79,32 +80,35 @@ __device__ __forceinline__ uint32_t mul_shoup(uint32_t a, uint32_t w, uint32_t w
 __device__ __forceinline__ uint32_t redc(uint64_t t, uint32_t p, uint32_t pinv) {
     uint32_t m = uint32_t(t) * pinv;
     uint32_t mh = __umulhi(m, p);
-    uint32_t hi = uint32_t(t >> 32);
-    uint32_t r = hi - mh;
-    return hi < mh ? r + p : r;
+    uint32_t r = uint32_t(t >> 32) - mh;  // in (-p, p) mod 2^32: r + p is the smaller exactly when r < 0
+    return min(r, r + p);
 }
 
 // REDC for t < 2p*2^32 (four products of residues: 4p^2 < 2p*2^32 as 2p < 2^32):
-// hi(t) - hi(m*p) lies in (-p, 2p); one more conditional subtraction than redc.
+// one more conditional subtraction than redc.
 __device__ __forceinline__ uint32_t redc_wide(uint64_t t, uint32_t p, uint32_t pinv) {
-    const uint32_t r = redc(t, p, pinv);  // in [0, 2p) for such t
-    return r >= p ? r - p : r;
+    const uint32_t mh = __umulhi(uint32_t(t) * pinv, p);
+    uint32_t hi = uint32_t(t >> 32);
+    hi = min(hi, hi - p);  // t - p*2^32, in redc's range, when that is not negative
+    const uint32_t r = hi - mh;
+    return min(r, r + p);
 }
 
 __device__ __forceinline__ uint32_t mont(uint32_t a, uint32_t b, uint32_t p, uint32_t pinv) {
     return redc(uint64_t(a) * b, p, pinv);
 }
 
-// 256, 65536 and 2^24 in scalar registers the compiler cannot see through.
+// 1, 256, 65536 and 2^24 in scalar registers the compiler cannot see through.
 // With literal scales each int64 term becomes a sign extension and a 64-bit
 // shift and add (about four instructions); with a register scale it is one
 // v_mad_i64_i32 (32x32 signed product plus 64-bit addend).
 struct DigitScales {
-    int32_t s8, s16, s24;
+    int32_t s0, s8, s16, s24;
 };
 
 __device__ __forceinline__ DigitScales digit_scales() {
     DigitScales s;
+    asm volatile("s_mov_b32 %0, 1" : "=s"(s.s0));
     asm volatile("s_mov_b32 %0, 0x100" : "=s"(s.s8));
     asm volatile("s_mov_b32 %0, 0x10000" : "=s"(s.s16));
     asm volatile("s_mov_b32 %0, 0x1000000" : "=s"(s.s24));
@@ -113,7 +117,7 @@ __device__ __forceinline__ DigitScales digit_scales() {
 
 // base + sum_d 256^d v[d], exact in int64.
 __device__ __forceinline__ int64_t combine4(const v4i& v, const DigitScales& s, int64_t base = 0) {
-    int64_t t = int64_t(v[0]) + base;
+    int64_t t = int64_t(v[0]) * int64_t(s.s0) + base;
     t += int64_t(v[1]) * int64_t(s.s8);
     t += int64_t(v[2]) * int64_t(s.s16);
     t += int64_t(v[3]) * int64_t(s.s24);
@@ -366,6 +370,149 @@ __global__ __launch_bounds__(512) void conversion_gemm(const int8_t* __restrict_
                                                        uint32_t r, uint32_t r_pad, uint32_t conv_rows,
                                                        uint32_t ksteps, TileSet ts, uint32_t op0, uint32_t nops) {
     conversion_body(wtiles, packed, consts, planes, n, n_pad, r, r_pad, conv_rows, ksteps, ts, op0, nops, blockIdx.x);
+}
+
+// ---------------------------------------------------------------------------
+// 1'. packing and conversion in one kernel, for q of up to kShortLimbs limbs:
+// the coefficients' limbs go straight from [N][L] into MFMA operand registers,
+// and the packed copy is never written.
+//
+//  * A wave owns 16 NT coefficients of one operand and holds all their bytes (at
+//    most KS K steps) in registers: lane l of a fragment loads the 16 bytes of
+//    coefficient l & 15, chunk l >> 4, which are only 4-byte aligned.  Bytes
+//    past a coefficient's limbs are 0 there; their weights are 0 too.
+//  * The block's four waves then walk the primes together, 64 weight rows (16
+//    primes) at a time.  The weights come in by direct-to-LDS loads, as many
+//    64-row chunks at once as kConvertStage holds, in the swizzled layout of
+//    gemm_mainloop; each chunk is multiplied, reduced and stored with no wait
+//    in between.
+//  * gridDim.y splits the primes over blocks when there are few coefficients.
+// What bounds it at N = 65536 with 55 limbs (30.7 us, packing and GEMM before:
+// 14.7 + 36.5): the 29 MB of limbs read and 60 MB of residues written, about
+// 18 us at a large copy's rate, with the MFMAs (7 us) and the reductions (5 us)
+// beside them.  At N = 131072 with 4 limbs 11.1 against 18.4 + 21.2 us, at
+// N = 128 with 128 limbs 4.8 against 2.9 + 12.0.  (Operand bytes in LDS and
+// weights straight from L2, one barrier per block: 37 us at N = 65536; the
+// weight fragments then come from L2 once per wave.)
+// ---------------------------------------------------------------------------
+constexpr uint32_t kConvertStage = 48 << 10;  // LDS bytes of weights: three blocks per CU
+
+struct ConvertArgs {
+    uint32_t n, n_pad, limbs, r, r_pad, conv_rows, ksteps;
+    TileSet ts;  // tile k's rows are rows k*256 .. of a and b (pack_body)
+    uint32_t op0;
+};
+
+constexpr uint32_t convert_stage_chunks(uint32_t ksteps) { return kConvertStage / (ksteps * kWaveRows * kTK); }
+
+// The staged weights, then the primes' constants.
+constexpr size_t convert_lds_bytes(uint32_t ksteps, uint32_t r) {
+    return size_t(convert_stage_chunks(ksteps)) * ksteps * kWaveRows * kTK + size_t(r) * sizeof(PrimeConst);
+}
+
+// Blocks (bx, by) of (., ny).
+template <int KS, int NT>
+__device__ __forceinline__ void convert_body(const uint32_t* __restrict__ a, const uint32_t* __restrict__ b,
+                                             const int8_t* __restrict__ wtiles,
+                                             const PrimeConst* __restrict__ consts, uint32_t* __restrict__ planes,
+                                             const ConvertArgs& args, uint32_t bx, uint32_t by, uint32_t ny,
+                                             int8_t* lds) {
+    typedef uint32_t v4u_word __attribute__((ext_vector_type(4), aligned(4)));  // 4-byte aligned
+    constexpr uint32_t T = 64 * NT, kChunkStep = kWaveRows * kTK;                 // 4 KB: 64 rows of one K step
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t L = args.limbs, ksteps = args.ksteps;
+    const uint32_t per_op = args.ts.count * (kTile / T);
+    const uint32_t op = args.op0 + bx / per_op, k0 = bx % per_op * T;
+    const uint32_t i0 = tile_at(args.ts, k0 / kTile) * kTile + k0 % kTile;
+    const uint32_t rows = i0 < args.n ? (args.n - i0 < T ? args.n - i0 : T) : 0;
+    const uint32_t chunks = (args.r + 15) / 16, share = (chunks + ny - 1) / ny;
+    const uint32_t c0 = by * share, c1 = c0 + share < chunks ? c0 + share : chunks;
+    if (!rows || c0 >= c1) return;  // whole block
+    const uint32_t cl = wave * 16 * NT + (lane & 15);  // the lane's first coefficient of the block's
+
+    v4i fb[KS][NT];
+    {
+        const uint32_t* src = (op ? b : a) + size_t(k0) * L;
+        const uint32_t w0 = (lane >> 4) * 4;
+#pragma unroll
+        for (uint32_t ks = 0; ks < KS; ++ks)
+#pragma unroll
+            for (uint32_t ni = 0; ni < NT; ++ni) {
+                const uint32_t row = cl + ni * 16 < rows ? cl + ni * 16 : rows - 1, w = ks * 16 + w0;
+                const uint32_t* p = src + size_t(row) * L + w;
+                v4u x = {0, 0, 0, 0};
+                if (w + 4 <= L) {
+                    x = *reinterpret_cast<const v4u_word*>(p);
+                } else {
+                    if (w < L) x[0] = p[0];
+                    if (w + 1 < L) x[1] = p[1];
+                    if (w + 2 < L) x[2] = p[2];
+                }
+                fb[ks][ni] = __builtin_bit_cast(v4i, x ^ 0x80808080u);
+            }
+    }
+    const uint32_t stage = convert_stage_chunks(ksteps), num_m = args.conv_rows / kTile;
+    PrimeConst* pcs = reinterpret_cast<PrimeConst*>(lds + stage * ksteps * kChunkStep);
+    for (uint32_t k = c0 * 16 + tid; k < args.r && k < c1 * 16; k += 256) pcs[k - c0 * 16] = consts[k];
+    // thread tid fills slot tid of a chunk's K step: row tid>>2, chunk swizzled as in swz
+    const uint32_t srow = tid >> 2, sbyte = srow * kTK + ((tid & 3) ^ ((srow >> 1) & 3)) * 16;
+    const DigitScales ds = digit_scales();
+    for (uint32_t s0 = c0; s0 < c1; s0 += stage) {
+        const uint32_t s1 = s0 + stage < c1 ? s0 + stage : c1;
+        if (s0 != c0) __syncthreads();  // every wave is done with the previous stage
+        for (uint32_t c = s0; c < s1; ++c) {
+            const int8_t* src = wtiles + (size_t(op) * num_m + c / 4) * ksteps * kTileBytes + (c % 4) * kChunkStep + sbyte;
+            for (uint32_t ks = 0; ks < ksteps; ++ks)
+                __builtin_amdgcn_global_load_lds(
+                    reinterpret_cast<const void*>(src + size_t(ks) * kTileBytes),
+                    (__attribute__((address_space(3))) void*)(lds + ((c - s0) * ksteps + ks) * kChunkStep + wave * 1024),
+                    16, 0, 0);
+        }
+        __syncthreads();
+        for (uint32_t c = s0; c < s1; ++c) {
+            const int8_t* wl = lds + (c - s0) * ksteps * kChunkStep + swz(lane & 15, lane >> 4);
+            v4i acc[kWaveM][NT];
+#pragma unroll
+            for (uint32_t mi = 0; mi < kWaveM; ++mi)
+#pragma unroll
+                for (uint32_t ni = 0; ni < NT; ++ni) acc[mi][ni] = v4i{0, 0, 0, 0};
+#pragma unroll
+            for (uint32_t ks = 0; ks < KS; ++ks)
+                if (KS <= 2 || ks < ksteps) {
+                    v4i fa[kWaveM];
+#pragma unroll
+                    for (uint32_t mi = 0; mi < kWaveM; ++mi)
+                        fa[mi] = *reinterpret_cast<const v4i*>(wl + ks * kChunkStep + mi * 16 * kTK);
+#pragma unroll
+                    for (uint32_t mi = 0; mi < kWaveM; ++mi)
+#pragma unroll
+                        for (uint32_t ni = 0; ni < NT; ++ni)
+                            acc[mi][ni] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[mi], fb[ks][ni], acc[mi][ni], 0, 0, 0);
+                }
+            // the epilogue of conversion_body
+#pragma unroll
+            for (uint32_t mi = 0; mi < kWaveM; ++mi) {
+                const uint32_t kp = c * 16 + mi * 4 + (lane >> 4);
+                if (kp >= args.r) continue;
+                const PrimeConst pc = pcs[kp - c0 * 16];
+                const int64_t off = int64_t(op ? pc.off_b : pc.off_a) + (int64_t(pc.p) << 31);
+                uint32_t* out = planes + (size_t(op) * args.r_pad + kp) * args.n_pad + i0 + cl;
+#pragma unroll
+                for (uint32_t ni = 0; ni < NT; ++ni)
+                    if (cl + ni * 16 < rows)
+                        out[ni * 16] = redc(uint64_t(combine4(acc[mi][ni], ds, off)), pc.p, pc.pinv);
+            }
+        }
+    }
+}
+
+template <int KS, int NT>
+__global__ __launch_bounds__(256, 3) void convert(const uint32_t* __restrict__ a, const uint32_t* __restrict__ b,
+                                                  const int8_t* __restrict__ wtiles,
+                                                  const PrimeConst* __restrict__ consts,
+                                                  uint32_t* __restrict__ planes, ConvertArgs args) {
+    extern __shared__ __attribute__((aligned(16))) int8_t dyn_lds[];
+    convert_body<KS, NT>(a, b, wtiles, consts, planes, args, blockIdx.x, blockIdx.y, gridDim.y, dyn_lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -1097,8 +1244,6 @@ constexpr size_t fused_lds_bytes(uint32_t wm, uint32_t nw, uint32_t ksteps) {
     return operands > sums ? operands : sums;
 }
 
-typedef uint32_t u32_alias __attribute__((may_alias));
-
 template <int WM, int NW>
 __device__ __forceinline__ void crt_reconstruct_body(const int8_t* __restrict__ wtiles,
                                                      const int8_t* __restrict__ rtiles, uint32_t* __restrict__ c,
@@ -1329,8 +1474,8 @@ __global__ __launch_bounds__(64 * NW, 4) void crt_reconstruct(const int8_t* __re
                                                        const uint32_t* __restrict__ neg_p,
                                                        const uint32_t* __restrict__ corr_t,
                                                        const uint32_t* __restrict__ corr_e, CrtFusedArgs args) {
-    extern __shared__ __attribute__((aligned(16))) int8_t fused_lds[];
-    crt_reconstruct_body<WM, NW>(wtiles, rtiles, c, q, neg_p, corr_t, corr_e, args, blockIdx.x, fused_lds);
+    extern __shared__ __attribute__((aligned(16))) int8_t dyn_lds[];
+    crt_reconstruct_body<WM, NW>(wtiles, rtiles, c, q, neg_p, corr_t, corr_e, args, blockIdx.x, dyn_lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -1338,8 +1483,45 @@ __global__ __launch_bounds__(64 * NW, 4) void crt_reconstruct(const int8_t* __re
 // a launch owns blocks [start[j], start[j+1]) and runs them as the blocks of
 // product item[j]'s own launch of that stage (kernels.hpp, GroupItem).
 // ---------------------------------------------------------------------------
+// GroupItem as the kernels read it.  A pointer read from memory could point
+// anywhere, which costs flat loads and stores (they wait for LDS and memory
+// together); these point to global memory, and their types say so.
+#ifdef __HIP_DEVICE_COMPILE__
+#define PM_GLOBAL __attribute__((address_space(1)))
+#else
+#define PM_GLOBAL
+#endif
+struct GroupView {
+    uint32_t n, n_pad, limbs, r, r_pad, conv_rows, conv_k, crt_rows, crt_k, crt_words, ws, t_words;
+    uint32_t n1, n2, rows, row_width, s_shift, k_shift, top_m, top_e;
+    uint32_t conv_variant, conv_split;  // short conversion (launch_convert)
+    uint64_t mu;
+    const PM_GLOBAL PrimeConst* consts;
+    const PM_GLOBAL int8_t* wconv;
+    const PM_GLOBAL uint2* tw_fwd;
+    const PM_GLOBAL uint2* tw_inv;
+    const PM_GLOBAL int8_t* wcrt;
+    const PM_GLOBAL uint32_t* q;
+    const PM_GLOBAL uint32_t* neg_p;
+    const PM_GLOBAL uint32_t* corr_t;
+    const PM_GLOBAL uint32_t* corr_e;
+    const PM_GLOBAL uint32_t* a;
+    const PM_GLOBAL uint32_t* b;
+    PM_GLOBAL uint32_t* c;
+    PM_GLOBAL int8_t* packed;
+    PM_GLOBAL uint32_t* planes;
+    PM_GLOBAL int8_t* rtiles;
+    PM_GLOBAL int64_t* words;
+};
+static_assert(sizeof(GroupView) == sizeof(GroupItem), "GroupView has GroupItem's layout");
+
+template <class T>
+__device__ __forceinline__ T* in_global(PM_GLOBAL T* p) {
+    return (T*)p;
+}
+
 struct GroupLaunch {
-    const GroupItem* items;
+    const GroupView* items;
     const uint32_t* start;  // count + 1 block offsets
     const uint32_t* item;   // the product of each entry
     uint32_t count;
@@ -1347,7 +1529,7 @@ struct GroupLaunch {
 
 // The product owning this block (a binary search over the offsets, the same
 // for every thread of the block) and the block's index in that product's grid.
-__device__ __forceinline__ const GroupItem& group_entry(const GroupLaunch& g, uint32_t& local) {
+__device__ __forceinline__ const GroupView& group_entry(const GroupLaunch& g, uint32_t& local) {
     const uint32_t b = blockIdx.x;
     uint32_t lo = 0, hi = g.count;
     while (hi - lo > 1) {
@@ -1361,29 +1543,42 @@ __device__ __forceinline__ const GroupItem& group_entry(const GroupLaunch& g, ui
     return g.items[g.item[lo]];
 }
 
-__device__ __forceinline__ TileSet every_tile(const GroupItem& it) { return tile_range(0, it.n_pad / kTile); }
+__device__ __forceinline__ TileSet every_tile(const GroupView& it) { return tile_range(0, it.n_pad / kTile); }
 
 __global__ __launch_bounds__(256) void pack_group(GroupLaunch g) {
     uint32_t local;
-    const GroupItem& it = group_entry(g, local);
-    pack_body(it.a, it.b, reinterpret_cast<uint32_t*>(it.packed), it.n, it.limbs, it.conv_k / kTK, it.n_pad / kTile,
+    const GroupView& it = group_entry(g, local);
+    pack_body(in_global(it.a), in_global(it.b), reinterpret_cast<uint32_t*>(in_global(it.packed)), it.n, it.limbs, it.conv_k / kTK, it.n_pad / kTile,
               every_tile(it), 0, 2, local);
 }
 
 __global__ __launch_bounds__(512) void conversion_group(GroupLaunch g) {
     uint32_t local;
-    const GroupItem& it = group_entry(g, local);
-    conversion_body(it.wconv, it.packed, it.consts, it.planes, it.n, it.n_pad, it.r, it.r_pad, it.conv_rows,
+    const GroupView& it = group_entry(g, local);
+    conversion_body(in_global(it.wconv), in_global(it.packed), in_global(it.consts), in_global(it.planes), it.n, it.n_pad, it.r, it.r_pad, it.conv_rows,
                     it.conv_k / kTK, every_tile(it), 0, 2, local);
+}
+
+// grid per product: (2 n_pad / 64 NT, prime splits)
+template <int KS, int NT>
+__global__ __launch_bounds__(256, 3) void convert_group(GroupLaunch g) {
+    extern __shared__ __attribute__((aligned(16))) int8_t dyn_lds[];
+    uint32_t local;
+    const GroupView& it = group_entry(g, local);
+    const uint32_t nx = 2 * it.n_pad / (64 * NT);
+    const ConvertArgs args{it.n, it.n_pad, it.limbs, it.r, it.r_pad, it.conv_rows, it.conv_k / kTK,
+                           every_tile(it), 0};
+    convert_body<KS, NT>(in_global(it.a), in_global(it.b), in_global(it.wconv), in_global(it.consts), in_global(it.planes), args, local % nx, local / nx, it.conv_split,
+                         dyn_lds);
 }
 
 // grid per product: (row_width / 256, r, 2)
 template <int ROWS>
 __global__ __launch_bounds__(256) void forward_reg_group(GroupLaunch g) {
     uint32_t local;
-    const GroupItem& it = group_entry(g, local);
+    const GroupView& it = group_entry(g, local);
     const uint32_t nx = it.row_width / 256, bx = local % nx, rest = local / nx;
-    forward_reg_body<ROWS>(it.planes, it.consts, it.tw_fwd, it.n_pad, it.n2, it.row_width, it.r_pad, 0, 0, bx,
+    forward_reg_body<ROWS>(in_global(it.planes), in_global(it.consts), in_global(it.tw_fwd), it.n_pad, it.n2, it.row_width, it.r_pad, 0, 0, bx,
                            rest % it.r, rest / it.r);
 }
 
@@ -1391,16 +1586,16 @@ __global__ __launch_bounds__(256) void forward_reg_group(GroupLaunch g) {
 template <uint32_t N1>
 __global__ __launch_bounds__(256) void rows_2048_group(GroupLaunch g) {
     uint32_t local;
-    const GroupItem& it = group_entry(g, local);
-    rows_2048_body<N1>(it.planes, it.planes + size_t(it.r_pad) * it.n_pad, it.consts, it.tw_fwd, it.tw_inv, it.n_pad,
+    const GroupView& it = group_entry(g, local);
+    rows_2048_body<N1>(in_global(it.planes), in_global(it.planes) + size_t(it.r_pad) * it.n_pad, in_global(it.consts), in_global(it.tw_fwd), in_global(it.tw_inv), it.n_pad,
                        it.n2, it.rows, local % it.rows, local / it.rows);
 }
 
 __global__ __launch_bounds__(256) void rows_product_group(GroupLaunch g) {
     extern __shared__ uint32_t lds32[];
     uint32_t local;
-    const GroupItem& it = group_entry(g, local);
-    rows_product_body(it.planes, it.planes + size_t(it.r_pad) * it.n_pad, it.consts, it.tw_fwd, it.tw_inv, it.n_pad,
+    const GroupView& it = group_entry(g, local);
+    rows_product_body(in_global(it.planes), in_global(it.planes) + size_t(it.r_pad) * it.n_pad, in_global(it.consts), in_global(it.tw_fwd), in_global(it.tw_inv), it.n_pad,
                       it.n1, it.n2, it.row_width, it.rows, lds32, local % it.rows, local / it.rows);
 }
 
@@ -1408,35 +1603,35 @@ __global__ __launch_bounds__(256) void rows_product_group(GroupLaunch g) {
 template <int ROWS>
 __global__ __launch_bounds__(256) void inverse_tiles_group(GroupLaunch g) {
     uint32_t local;
-    const GroupItem& it = group_entry(g, local);
+    const GroupView& it = group_entry(g, local);
     const uint32_t nx = it.row_width / 16;
-    inverse_tiles_body<ROWS>(it.planes, it.consts, it.tw_inv, it.n_pad, it.n, it.n2, it.row_width, it.r,
-                             it.r_pad / 16, it.rtiles, 0, local % nx, local / nx, nx);
+    inverse_tiles_body<ROWS>(in_global(it.planes), in_global(it.consts), in_global(it.tw_inv), it.n_pad, it.n, it.n2, it.row_width, it.r,
+                             it.r_pad / 16, in_global(it.rtiles), 0, local % nx, local / nx, nx);
 }
 
 __global__ __launch_bounds__(512) void crt_group(GroupLaunch g) {
     uint32_t local;
-    const GroupItem& it = group_entry(g, local);
-    crt_body(it.wcrt, it.rtiles, it.words, it.n, it.n_pad, it.crt_rows, it.crt_k / kTK, it.crt_words, it.ws,
+    const GroupView& it = group_entry(g, local);
+    crt_body(in_global(it.wcrt), in_global(it.rtiles), in_global(it.words), it.n, it.n_pad, it.crt_rows, it.crt_k / kTK, it.crt_words, it.ws,
              every_tile(it), local);
 }
 
 template <int WM, int NW>
 __global__ __launch_bounds__(64 * NW, 4) void crt_reconstruct_group(GroupLaunch g) {
-    extern __shared__ __attribute__((aligned(16))) int8_t fused_lds[];
+    extern __shared__ __attribute__((aligned(16))) int8_t dyn_lds[];
     uint32_t local;
-    const GroupItem& it = group_entry(g, local);
+    const GroupView& it = group_entry(g, local);
     const CrtFusedArgs args{it.n, it.limbs, it.t_words, (it.r + 15) / 16, it.r_pad / 16, every_tile(it),
                             it.top_m, it.top_e, it.k_shift, it.mu};
-    crt_reconstruct_body<WM, NW>(it.wcrt, it.rtiles, it.c, it.q, it.neg_p, it.corr_t, it.corr_e, args, local, fused_lds);
+    crt_reconstruct_body<WM, NW>(in_global(it.wcrt), in_global(it.rtiles), in_global(it.c), in_global(it.q), in_global(it.neg_p), in_global(it.corr_t), in_global(it.corr_e), args, local, dyn_lds);
 }
 
 __global__ __launch_bounds__(256) void reconstruct_waves_group(GroupLaunch g) {
     uint32_t local;
-    const GroupItem& it = group_entry(g, local);
+    const GroupView& it = group_entry(g, local);
     const WaveReconstructArgs args{it.n, it.ws, it.limbs, it.t_words, every_tile(it),
                                    it.top_m, it.top_e, it.k_shift, it.mu};
-    reconstruct_waves_body(it.words, it.c, it.q, it.neg_p, it.corr_t, it.corr_e, args, local);
+    reconstruct_waves_body(in_global(it.words), in_global(it.c), in_global(it.q), in_global(it.neg_p), in_global(it.corr_t), in_global(it.corr_e), args, local);
 }
 
 __global__ void fill_zero(uint32_t* __restrict__ c, size_t words) {
@@ -1689,6 +1884,53 @@ void launch_conversion(const Shape& s, const DeviceTables& t, const int8_t* pack
     check_launch("conversion_gemm");
 }
 
+namespace {
+
+// Variant of the short conversion: K steps held in registers (KS), 16-coefficient
+// fragments per wave (NT), splits of the primes over blocks.
+struct ConvertPlan {
+    uint32_t ks, nt, split;
+};
+constexpr uint32_t kConvertBlocks = 512, kConvertGroupBlocks = 64;  // two per CU; a batch's share
+
+// `tiles` 256-coefficient tiles in all (of both operands).  Wide waves (NT 2 or
+// 4) read each weight from LDS for 32 or 64 coefficients; where they would
+// leave most of the GPU idle (fewer than want_blocks / 2 blocks even with every
+// 16 primes in a block of their own) waves of 16 coefficients take over: N =
+// 1024 with 8 limbs 3.5 us against 4.3 with 64-coefficient blocks.  Then the
+// primes are split until there are want_blocks blocks.  In a batch the other
+// products fill the GPU, so there want_blocks is small and the waves wide: the
+// batch of 64 small products' conversions take 152 us in all, and 210 with each
+// product spread as if it were alone.
+ConvertPlan convert_plan(uint32_t r, uint32_t ksteps, uint32_t tiles, uint32_t want_blocks) {
+    const uint32_t chunks = (r + 15) / 16, ks = ksteps <= 1 ? 1 : ksteps <= 2 ? 2 : ksteps <= 4 ? 4 : 8;
+    uint32_t nt = ks == 8 ? 2 : 4;
+    if (want_blocks == kConvertBlocks && tiles * (4 / nt) * chunks < want_blocks / 2) nt = 1;
+    const uint32_t blocks = tiles * (4 / nt), want = (want_blocks + blocks - 1) / blocks;
+    return ConvertPlan{ks, nt, chunks < want ? chunks : want};
+}
+
+}  // namespace
+
+#define PM_CONVERT_VARIANTS(X) X(1, 1) X(2, 1) X(4, 1) X(8, 1) X(1, 4) X(2, 4) X(4, 4) X(8, 2)
+
+void launch_convert(const Shape& s, const DeviceTables& t, const uint32_t* a, const uint32_t* b, uint32_t* planes,
+                    const TileSet& ts, uint32_t op0, uint32_t nops, hipStream_t stream) {
+    check_tiles(s, ts, "convert");
+    if (!conversion_short(s)) throw std::logic_error("convert: operands wider than a wave holds");
+    const uint32_t ksteps = s.conv_k / kTK;
+    const ConvertArgs args{s.n, s.n_pad, s.limbs, s.r, s.r_pad, s.conv_rows, ksteps, ts, op0};
+    const ConvertPlan cp = convert_plan(s.r, ksteps, nops * ts.count, kConvertBlocks);
+    const dim3 grid(nops * ts.count * (4 / cp.nt), cp.split);
+#define PM_CONVERT(K, N)                                                                                  \
+    if (cp.ks == K && cp.nt == N)                                                                         \
+        hipLaunchKernelGGL((convert<K, N>), grid, dim3(256), convert_lds_bytes(ksteps, s.r), stream, a, b, \
+                           t.wconv, t.consts, planes, args);
+    PM_CONVERT_VARIANTS(PM_CONVERT)
+#undef PM_CONVERT
+    check_launch("convert");
+}
+
 void launch_ntt_forward_columns(const Shape& s, const DeviceTables& t, uint32_t* planes, uint32_t op0,
                                 uint32_t nops, hipStream_t stream, uint32_t strip_begin, uint32_t strip_end) {
     const bool whole = whole_columns(s, strip_begin, strip_end, "ntt_columns_forward");
@@ -1835,6 +2077,8 @@ GroupItem group_item(const Shape& s, const DeviceTables& t, const DeviceWork& w,
     it.crt_words = s.crt_words, it.ws = word_stride(s), it.t_words = s.t_words;
     it.n1 = s.n1, it.n2 = s.n2, it.rows = s.rows, it.row_width = s.row_width;
     it.s_shift = s.s_shift, it.k_shift = s.k_shift;
+    const ConvertPlan cp = convert_plan(s.r, s.conv_k / kTK, 2 * s.n_pad / kTile, kConvertGroupBlocks);
+    it.conv_variant = cp.ks * 8 + cp.nt, it.conv_split = cp.split;
     it.top_m = barrett_top(s);
     it.top_e = s.s_shift - 32 * it.top_m;
     it.mu = s.mu;
@@ -1854,13 +2098,14 @@ bool groupable(const Shape& s) {
 
 namespace {
 
-// Launches of one batch: pack, conversion, forward columns (one per row count),
+// Launches of one batch: conversion from the limbs (one per variant),
+// pack and conversion, forward columns (one per row count),
 // rows (one per block size n1, and the LDS kernel), inverse columns (one per
 // row count), CRT GEMM with reconstruction (one per wave-row count), CRT GEMM,
 // reconstruction.
-constexpr size_t kGroupLaunches = 2 + 6 + 5 + 7 + 3 + 2;
+constexpr size_t kGroupLaunches = 8 + 2 + 6 + 5 + 7 + 3 + 2;
 
-enum GroupKind { kPack, kConversion, kForward, kRows2048, kRowsProduct, kInverse, kCrtRec, kCrt, kRecWave };
+enum GroupKind { kConvert, kPack, kConversion, kForward, kRows2048, kRowsProduct, kInverse, kCrtRec, kCrt, kRecWave };
 
 size_t group_item_bytes(size_t count) { return (count * sizeof(GroupItem) + 255) / 256 * 256; }
 size_t group_table_words(size_t count) { return kGroupLaunches * (2 * count + 1); }
@@ -1873,7 +2118,7 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
     const uint32_t count = uint32_t(items.size());
     if (!count) return;
     const size_t item_bytes = group_item_bytes(count);
-    const GroupItem* dev_items = static_cast<const GroupItem*>(dev_buffer);
+    const GroupView* dev_items = static_cast<const GroupView*>(dev_buffer);  // GroupItems, uploaded below
     uint32_t* dev_tables = reinterpret_cast<uint32_t*>(static_cast<char*>(dev_buffer) + item_bytes);
     struct Launch {
         GroupKind kind;
@@ -1901,8 +2146,9 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
             item[j] = sel[j];
             total += blocks(items[sel[j]]);
             const GroupItem& it = items[sel[j]];
-            lds = std::max<size_t>(lds, kind == kCrtRec ? fused_lds_bytes(variant, 4, (it.r + 15) / 16)
-                                                        : size_t(2) * it.row_width * 4);
+            lds = std::max<size_t>(lds, kind == kCrtRec    ? fused_lds_bytes(variant, 4, (it.r + 15) / 16)
+                                        : kind == kConvert ? convert_lds_bytes(it.conv_k / kTK, it.r)
+                                                           : size_t(2) * it.row_width * 4);
         }
         if (total >= (uint64_t(1) << 31)) throw std::invalid_argument("launch_group: batch too large for one grid");
         start[sel.size()] = uint32_t(total);
@@ -1911,10 +2157,19 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
     };
     auto ntiles = [](const GroupItem& it) { return uint64_t(it.n_pad / kTile); };
     auto rows_2048 = [](const GroupItem& it) { return it.row_width == kRowC && it.n1 <= 8; };
-    add(kPack, 0, [&](const GroupItem& it) {  // as launch_pack: 2 * ntiles * 256 rows
-        return 128 * ntiles(it) / pack_rows_per_wave(it.conv_k / kTK);
+#define PM_GCONV(K, N)                                                                                            \
+    add(kConvert, K * 8 + N, [&](const GroupItem& it) {                                                           \
+        return it.limbs <= kShortLimbs && it.conv_variant == K * 8 + N ? uint64_t(it.conv_split) * (8 / N) * ntiles(it) \
+                                                                       : 0;                                       \
     });
-    add(kConversion, 0, [&](const GroupItem& it) { return uint64_t(it.conv_rows / kTile) * 2 * ntiles(it); });
+    PM_CONVERT_VARIANTS(PM_GCONV)
+#undef PM_GCONV
+    add(kPack, 0, [&](const GroupItem& it) {  // as launch_pack: 2 * ntiles * 256 rows
+        return it.limbs <= kShortLimbs ? 0 : 128 * ntiles(it) / pack_rows_per_wave(it.conv_k / kTK);
+    });
+    add(kConversion, 0, [&](const GroupItem& it) {
+        return it.limbs <= kShortLimbs ? 0 : uint64_t(it.conv_rows / kTile) * 2 * ntiles(it);
+    });
     for (uint32_t R = 2; R <= 64; R *= 2)
         add(kForward, R, [&](const GroupItem& it) {
             return it.rows == R ? uint64_t(it.row_width / 256) * it.r * 2 : 0;
@@ -1946,6 +2201,13 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
         const GroupLaunch g{dev_items, dev_tables + L.offset, dev_tables + L.offset + L.entries + 1, L.entries};
         const dim3 grid(uint32_t(L.blocks));
         switch (L.kind) {
+            case kConvert:
+#define PM_GCONV(K, N)                                                                       \
+    if (L.variant == K * 8 + N)                                                              \
+        hipLaunchKernelGGL((convert_group<K, N>), grid, dim3(256), L.lds, stream, g);
+                PM_CONVERT_VARIANTS(PM_GCONV)
+#undef PM_GCONV
+                break;
             case kPack:
                 hipLaunchKernelGGL(pack_group, grid, dim3(256), 0, stream, g);
                 break;

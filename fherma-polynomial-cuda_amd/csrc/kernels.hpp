@@ -69,6 +69,12 @@ void launch_pack(const Shape& s, const uint32_t* a, const uint32_t* b, int8_t* p
                  uint32_t op0, uint32_t nops, hipStream_t stream);
 void launch_conversion(const Shape& s, const DeviceTables& t, const int8_t* packed, uint32_t* planes,
                        const TileSet& ts, uint32_t op0, uint32_t nops, hipStream_t stream);
+// Both of the above in one kernel that reads a and b itself (rows as launch_pack),
+// for q of up to kShortLimbs limbs.
+constexpr uint32_t kShortLimbs = 128;
+inline bool conversion_short(const Shape& s) { return s.limbs <= kShortLimbs; }
+void launch_convert(const Shape& s, const DeviceTables& t, const uint32_t* a, const uint32_t* b, uint32_t* planes,
+                    const TileSet& ts, uint32_t op0, uint32_t nops, hipStream_t stream);
 // Forward row-spanning (column) stages of column strips [strip_begin,
 // strip_end) of 256 columns each, or of every column with the defaults; a strip
 // range needs the register-resident kernel (row_width a multiple of 256, 2 to
@@ -108,6 +114,7 @@ void launch_zero(uint32_t* c, size_t words, hipStream_t stream);
 struct GroupItem {
     uint32_t n, n_pad, limbs, r, r_pad, conv_rows, conv_k, crt_rows, crt_k, crt_words, ws, t_words;
     uint32_t n1, n2, rows, row_width, s_shift, k_shift, top_m, top_e;
+    uint32_t conv_variant, conv_split;  // short conversion (launch_convert)
     uint64_t mu;
     const PrimeConst* consts;
     const int8_t* wconv;

@@ -326,8 +326,12 @@ struct pm_plan {
                 hip_check(hipStreamWaitEvent(stream, lane->in_ready[ch], 0), "hipStreamWaitEvent");
                 const uint32_t* xa = io_a + base;  // pack reads the chunk's k-th tile at rows k*256..
                 const uint32_t* xb = xa + rows * L;
-                pm::launch_pack(s, xa, xb, work.packed, chunks.set[ch], 0, nops, stream);
-                pm::launch_conversion(s, tables, work.packed, work.planes, chunks.set[ch], 0, nops, stream);
+                if (pm::conversion_short(s)) {
+                    pm::launch_convert(s, tables, xa, xb, work.planes, chunks.set[ch], 0, nops, stream);
+                } else {
+                    pm::launch_pack(s, xa, xb, work.packed, chunks.set[ch], 0, nops, stream);
+                    pm::launch_conversion(s, tables, work.packed, work.planes, chunks.set[ch], 0, nops, stream);
+                }
                 if (chunks.strips && chunks.fwd_end[ch] > chunks.fwd_begin[ch])
                     pm::launch_ntt_forward_columns(s, tables, work.planes, 0, nops, stream, chunks.fwd_begin[ch],
                                                    chunks.fwd_end[ch]);
@@ -537,9 +541,11 @@ struct pm_plan {
         const uint32_t nops = b ? 2 : 1;
         const uint32_t* bplanes = b ? b_planes(w) : bplanes_in;
         mark(0);
-        pm::launch_pack(s, a, b, w.packed, all, 0, nops, st);
+        const bool packed = !pm::conversion_short(s);  // else packing is part of the conversion's time
+        if (packed) pm::launch_pack(s, a, b, w.packed, all, 0, nops, st);
         mark(1);
-        pm::launch_conversion(s, tables, w.packed, w.planes, all, 0, nops, st);
+        if (packed) pm::launch_conversion(s, tables, w.packed, w.planes, all, 0, nops, st);
+        else pm::launch_convert(s, tables, a, b, w.planes, all, 0, nops, st);
         mark(2);
         if (last == PM_STAGE_RESIDUES) return;
         pm::launch_ntt_forward_columns(s, tables, w.planes, 0, nops, st);
