@@ -61,19 +61,28 @@ void check_launch(const char* what) {
 }
 
 __device__ __forceinline__ uint32_t add_mod(uint32_t a, uint32_t b, uint32_t p) {
-    uint32_t t = a + b;
-    return t >= p ? t - p : t;
+    const uint32_t t = a + b;
+    return min(t, t - p);
 }
 
 __device__ __forceinline__ uint32_t sub_mod(uint32_t a, uint32_t b, uint32_t p) {
-    return a >= b ? a - b : a + p - b;
+    const uint32_t t = a - b;
+    return min(t, t + p);
 }
 
-// Shoup: wq = floor(w*2^32/p); for a < 2^32, a*w - hi(a*wq)*p lies in [0, 2p).
+// Shoup: wq = floor(w*2^32/p); for any a < 2^32, a*w - hi(a*wq)*p lies in [0, 2p).
+// Both low products are taken as v_mad_u64_u32 in 64 bits, the second with the
+// first as its addend, which saves the subtraction (on gfx950 all of these issue
+// at the same rate, one per 4 cycles and SIMD); only the low word counts.
+__device__ __forceinline__ uint32_t mul_shoup_lazy(uint32_t a, uint32_t w, uint32_t wq, uint32_t p) {
+    uint64_t r = uint64_t(__umulhi(a, wq)) * (0u - p) + uint64_t(a) * w;
+    asm("" : "+v"(r));  // keeps the 64-bit form, which the compiler would narrow to three instructions
+    return uint32_t(r);
+}
+
 __device__ __forceinline__ uint32_t mul_shoup(uint32_t a, uint32_t w, uint32_t wq, uint32_t p) {
-    uint32_t q = __umulhi(a, wq);
-    uint32_t r = a * w - q * p;
-    return r >= p ? r - p : r;
+    const uint32_t r = mul_shoup_lazy(a, w, wq, p);
+    return min(r, r - p);  // r - p wraps above r exactly when r < p
 }
 
 // Subtractive Montgomery REDC of t < p*2^32: (t - m p)/2^32, m = t p^-1 mod 2^32.
@@ -722,16 +731,29 @@ __global__ __launch_bounds__(256) void ntt_columns_inverse(uint32_t* __restrict_
 // ---------------------------------------------------------------------------
 // Register-resident NTT kernels for the usual shapes (rows <= 64, C = 2048).
 // ---------------------------------------------------------------------------
+// Cooley-Tukey: (a, b) -> (a + wb, a - wb).  a < p; b may be any 32-bit value
+// congruent to its residue.  With kReduce the outputs are below p; without,
+// below 2p, which is all the next level asks of the values it multiplies (b),
+// and half of every level's outputs are that: 8 instead of 11 instructions.
+// (Primes just below 2^31 leave no room for Harvey's form, lazy in all of them.)
+template <bool kReduce>
 __device__ __forceinline__ void ct_butterfly(uint32_t& a, uint32_t& b, uint2 w, uint32_t p) {
     const uint32_t v = mul_shoup(b, w.x, w.y, p);
-    b = sub_mod(a, v, p);
-    a = add_mod(a, v, p);
+    if constexpr (kReduce) {
+        b = sub_mod(a, v, p);
+        a = add_mod(a, v, p);
+    } else {
+        b = a - v + p;
+        a = a + v;
+    }
 }
 
+// Gentleman-Sande: (a, b) -> (a + b, w (a - b)), all below p; the difference
+// goes into the product as it is, below 2p.
 __device__ __forceinline__ void gs_butterfly(uint32_t& a, uint32_t& b, uint2 w, uint32_t p) {
     const uint32_t u = a, v = b;
     a = add_mod(u, v, p);
-    b = mul_shoup(sub_mod(u, v, p), w.x, w.y, p);
+    b = mul_shoup(u - v + p, w.x, w.y, p);
 }
 
 // Forward row-spanning stages: one thread per (operand, prime, column) holding
@@ -755,7 +777,12 @@ __device__ __forceinline__ void forward_reg_body(uint32_t* __restrict__ planes, 
         for (int g = 0; g < m; ++g) {
             const uint2 t = w[m + g];
 #pragma unroll
-            for (int jr = 0; jr < half; ++jr) ct_butterfly(x[2 * half * g + jr], x[2 * half * g + jr + half], t, p);
+            for (int jr = 0; jr < half; ++jr) {
+                // the next level multiplies the rows with its distance's bit set
+                uint32_t &lo = x[2 * half * g + jr], &hi = x[2 * half * g + jr + half];
+                if (half == 1 || !(jr & (half / 2))) ct_butterfly<true>(lo, hi, t, p);
+                else ct_butterfly<false>(lo, hi, t, p);
+            }
         }
 #pragma unroll
     for (int j = 0; j < ROWS; ++j) data[size_t(j) * C] = x[j];
@@ -840,7 +867,13 @@ __global__ __launch_bounds__(256) void ntt_columns_inverse_tiles(const uint32_t*
 }
 
 // Row stages for C = 2048: one block per (row, prime), 256 threads x 8 values
-// per operand.  The 11 butterfly levels inside a row are done three at a time
+// per operand.  Bound by VALU issue where there are many blocks (N = 65536 with
+// 1747 limbs: 1.12 ms, 95 % of the issue rate; 1.34 ms with every butterfly
+// fully reduced, 1599 instead of 1282 VALU instructions per thread), and partly
+// by the first loads' latency where there are two rounds of them (N = 65536
+// with 55 limbs: 48 us, before 59).  Reading the inverse twiddles out of the
+// forward table (mirrored, half the twiddle bytes) and half the barriers both
+// measured the same.  The 11 butterfly levels inside a row are done three at a time
 // in registers, with an LDS exchange between groups:
 //   layout A: jj = t + 256e      distances 1024, 512, 256
 //   layout B: jj = 256(t/32) + (t%32) + 32e   distances 128, 64, 32
@@ -859,21 +892,40 @@ __device__ __forceinline__ uint32_t layout_index(int layout, uint32_t t, int e) 
     }
 }
 
-// forward levels of one layout: distances stride*2^(levels-1) .. stride (those >= n1)
+// Twiddle index of the butterfly of value e at level b (distance 2^b times the
+// layout's stride): (base + jj) >> log2(2 distance), which is the same for the
+// whole block in layout A and 1, 2 or 4 consecutive entries per thread in the
+// others.
+__device__ __forceinline__ uint32_t twiddle_index(int layout, uint32_t t, int e, int b, uint32_t base, uint32_t d) {
+    const uint32_t first = layout == 0 ? 0 : (layout == 1 ? t >> 5 : layout == 2 ? t >> 2 : t) << (2 - b);
+    return (base >> (31 - __clz(2 * d))) + first + (uint32_t(e) >> (b + 1));
+}
+
+// Forward levels of one layout: distances stride*2^(levels-1) .. stride (those
+// >= n1).  `lazy_in`: the values are below 2p (left so by the group before);
+// the ones the first level does not multiply are reduced first.  The last
+// level of a group leaves its outputs below 2p, unless it is the transform's
+// last (distance n1): then they are below p, or stay below 2p with `lazy_out`.
 __device__ __forceinline__ void row_forward_group(uint32_t (&x)[8], int layout, int levels, uint32_t t,
-                                                  uint32_t stride, uint32_t n1, uint32_t base_index,
-                                                  const uint2* w, uint32_t p) {
+                                                  uint32_t stride, uint32_t n1, uint32_t base_index, bool lazy_in,
+                                                  bool lazy_out, const uint2* w, uint32_t p) {
+    if (lazy_in && (stride << (levels - 1)) >= n1) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            if (!(e & (1 << (levels - 1)))) x[e] = min(x[e], x[e] - p);
+    }
 #pragma unroll
     for (int b = levels - 1; b >= 0; --b) {
         const uint32_t d = stride << b;
         if (d < n1) continue;
-        const uint32_t shift = 31 - __clz(2 * d);  // log2(2d)
+        const bool last = d == n1;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             if (e & (1 << b)) continue;
-            const uint32_t jj = layout_index(layout, t, e);
-            const uint2 tw = w[(base_index >> shift) + (jj >> shift)];
-            ct_butterfly(x[e], x[e + (1 << b)], tw, p);
+            const uint2 tw = w[twiddle_index(layout, t, e, b, base_index, d)];
+            const bool reduce = last ? !lazy_out : b > 0 && !(e & (1 << (b - 1)));
+            if (reduce) ct_butterfly<true>(x[e], x[e + (1 << b)], tw, p);
+            else ct_butterfly<false>(x[e], x[e + (1 << b)], tw, p);
         }
     }
 }
@@ -885,13 +937,10 @@ __device__ __forceinline__ void row_inverse_group(uint32_t (&x)[8], int layout, 
     for (int b = 0; b < levels; ++b) {
         const uint32_t d = stride << b;
         if (d < n1) continue;
-        const uint32_t shift = 31 - __clz(2 * d);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             if (e & (1 << b)) continue;
-            const uint32_t jj = layout_index(layout, t, e);
-            const uint2 tw = w[(base_index >> shift) + (jj >> shift)];
-            gs_butterfly(x[e], x[e + (1 << b)], tw, p);
+            gs_butterfly(x[e], x[e + (1 << b)], w[twiddle_index(layout, t, e, b, base_index, d)], p);
         }
     }
 }
@@ -943,27 +992,28 @@ __device__ __forceinline__ void rows_2048_body(uint32_t* __restrict__ planes, co
         xa[e] = pa[t + 256 * e];
         xb[e] = pb[t + 256 * e];
     }
-    row_forward_group(xa, 0, 3, t, 256, n1, base_index, wf, p);
-    row_forward_group(xb, 0, 3, t, 256, n1, base_index, wf, p);
+    row_forward_group(xa, 0, 3, t, 256, n1, base_index, false, N1 == 1, wf, p);
+    row_forward_group(xb, 0, 3, t, 256, n1, base_index, false, false, wf, p);
     row_exchange(buf[0], xa, 0, 1, t);
     row_exchange(buf[1], xb, 0, 1, t);
-    row_forward_group(xa, 1, 3, t, 32, n1, base_index, wf, p);
-    row_forward_group(xb, 1, 3, t, 32, n1, base_index, wf, p);
+    row_forward_group(xa, 1, 3, t, 32, n1, base_index, true, N1 == 1, wf, p);
+    row_forward_group(xb, 1, 3, t, 32, n1, base_index, true, false, wf, p);
     row_exchange(buf[0], xa, 1, 2, t);
     row_exchange(buf[1], xb, 1, 2, t);
-    row_forward_group(xa, 2, 3, t, 4, n1, base_index, wf, p);
-    row_forward_group(xb, 2, 3, t, 4, n1, base_index, wf, p);
+    row_forward_group(xa, 2, 3, t, 4, n1, base_index, true, N1 == 1, wf, p);
+    row_forward_group(xb, 2, 3, t, 4, n1, base_index, true, false, wf, p);
     row_exchange(buf[0], xa, 2, 3, t);
     row_exchange(buf[1], xb, 2, 3, t);
-    row_forward_group(xa, 3, 2, t, 1, n1, base_index, wf, p);
-    row_forward_group(xb, 3, 2, t, 1, n1, base_index, wf, p);
+    row_forward_group(xa, 3, 2, t, 1, n1, base_index, true, N1 == 1, wf, p);
+    row_forward_group(xb, 3, 2, t, 1, n1, base_index, true, false, wf, p);
 
     // base case: thread t holds jj = 8t .. 8t+7, i.e. 8/n1 whole blocks.  Block g
     // is reduced mod (X^n1 - zeta_g): c_s = sum_{u<=s} a_u b_{s-u} + sum_{u>s}
     // a_u (zeta_g b_{s+n1-u}).  The wrapped factors zeta_g*b_v are formed once per
-    // block (Shoup), so each output is one sum of n1 products, reduced four at a
-    // time (a sum of four products of residues is below 4p^2 < 2p*2^32, in
-    // redc_wide's range; 32-bit multiplies are the scarce resource here).
+    // block (Shoup), so each output is one sum of n1 products and one REDC: four
+    // products of residues stay below 4p^2 < 2p*2^32, and from there on p*2^32
+    // is taken off (a minimum on the high word) before every second product.
+    // With n1 = 1 the a values come unreduced: 2p*p < p*2^32.
     uint32_t xc[8];
     constexpr int n1i = int(N1);
 #pragma unroll
@@ -990,16 +1040,17 @@ __device__ __forceinline__ void rows_2048_body(uint32_t* __restrict__ planes, co
 #pragma unroll
         for (int s1 = 0; s1 < n1i; ++s1) {
             uint64_t acc = 0;
-            uint32_t value = 0;
 #pragma unroll
             for (int u = 0; u < n1i; ++u) {
                 const uint32_t f = u <= s1 ? xb[blk0 + s1 - u] : bw[s1 + n1i - u];
-                acc += uint64_t(xa[blk0 + u]) * f;
-                if ((u & 3) == 3 || u == n1i - 1) {
-                    value = add_mod(value, redc_wide(acc, p, pinv), p);
-                    acc = 0;
+                // at most two products on top of p*2^32, or four alone: below 2p*2^32
+                if (u >= 4 && u % 2 == 0) {
+                    const uint32_t hi = uint32_t(acc >> 32);
+                    acc = (uint64_t(min(hi, hi - p)) << 32) | uint32_t(acc);
                 }
+                acc += uint64_t(xa[blk0 + u]) * f;
             }
+            const uint32_t value = n1i == 1 ? redc(acc, p, pinv) : redc_wide(acc, p, pinv);
             xc[blk0 + s1] = value;
         }
     }
