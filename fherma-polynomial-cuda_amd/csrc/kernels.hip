@@ -866,21 +866,28 @@ __global__ __launch_bounds__(256) void ntt_columns_inverse_tiles(const uint32_t*
     inverse_tiles_body<ROWS>(plane, consts, tw, ps, n, n2, C, r, ksteps, tiles, g0, blockIdx.x, blockIdx.y, gridDim.x);
 }
 
-// Row stages for C = 2048: one block per (row, prime), 256 threads x 8 values
-// per operand.  Bound by VALU issue where there are many blocks (N = 65536 with
-// 1747 limbs: 1.12 ms, 95 % of the issue rate; 1.34 ms with every butterfly
-// fully reduced, 1599 instead of 1282 VALU instructions per thread), and partly
-// by the first loads' latency where there are two rounds of them (N = 65536
-// with 55 limbs: 48 us, before 59).  Reading the inverse twiddles out of the
-// forward table (mirrored, half the twiddle bytes) and half the barriers both
-// measured the same.  The 11 butterfly levels inside a row are done three at a time
-// in registers, with an LDS exchange between groups:
+// Row stages held in registers: 256 threads x 8 values per operand, i.e. 2048
+// values jj of one row of one prime (C = 2048), or, for N = C < 2048, the whole
+// transforms of 2048 / C consecutive primes side by side (prime jj / C).  The
+// butterfly levels are done three at a time, with an LDS exchange between
+// groups:
 //   layout A: jj = t + 256e      distances 1024, 512, 256
 //   layout B: jj = 256(t/32) + (t%32) + 32e   distances 128, 64, 32
 //   layout C: jj = 32(t/4) + (t%4) + 4e       distances 16, 8, 4
 //   layout D: jj = 8t + e        distances 2, 1, and the base case (n1 <= 8)
-// Forward stops at distance n1, the base case multiplies each n1-block mod
-// (X^n1 - zeta), and the inverse climbs back from n1 to 1024.
+// Forward runs the distances C/2 .. n1, the base case multiplies each n1-block
+// mod (X^n1 - zeta), and the inverse climbs back from n1 to C/2.  (C <= 256
+// starts and ends in layout B.)
+//
+// Bound by VALU issue where there are many blocks (N = 65536 with 1747 limbs:
+// 1.12 ms, 95 % of the issue rate; 1.34 ms with every butterfly fully reduced),
+// by latency where there are few, so each group's twiddles are fetched a group
+// ahead (N = 65536 with 55 limbs 48 -> 45.5 us, N = 16384 with 28 limbs 12.8 ->
+// 11.2 us).  Below C = 2048 it takes the place of the LDS kernel's one level per
+// barrier: N = 1024 with 8 limbs 16.8 -> 6.3 us, a batch's N = 1024 products
+// 40 -> 14 us.
+// Reading the inverse twiddles out of the forward table (mirrored, half the
+// twiddle bytes) and half the barriers both measured the same.
 constexpr uint32_t kRowC = 2048;
 
 __device__ __forceinline__ uint32_t layout_index(int layout, uint32_t t, int e) {
@@ -892,55 +899,95 @@ __device__ __forceinline__ uint32_t layout_index(int layout, uint32_t t, int e) 
     }
 }
 
-// Twiddle index of the butterfly of value e at level b (distance 2^b times the
-// layout's stride): (base + jj) >> log2(2 distance), which is the same for the
-// whole block in layout A and 1, 2 or 4 consecutive entries per thread in the
-// others.
-__device__ __forceinline__ uint32_t twiddle_index(int layout, uint32_t t, int e, int b, uint32_t base, uint32_t d) {
-    const uint32_t first = layout == 0 ? 0 : (layout == 1 ? t >> 5 : layout == 2 ? t >> 2 : t) << (2 - b);
-    return (base >> (31 - __clz(2 * d))) + first + (uint32_t(e) >> (b + 1));
+// The prime (of the block's) that value e belongs to, written so that the
+// compiler sees where it is the same for a block, a wave or a thread.
+template <int LOGC>
+__device__ __forceinline__ uint32_t layout_prime(int layout, uint32_t t, int e) {
+    if constexpr (LOGC == 11) return 0;
+    if (layout == 0 && LOGC >= 8) return uint32_t(e) >> (LOGC - 8);
+    if (layout == 1 && LOGC < 8) return ((t >> 5) << (8 - LOGC)) + (uint32_t(e) >> (LOGC - 5));
+    const uint32_t k = t >> (LOGC - 3);
+    return LOGC >= 9 ? uint32_t(__builtin_amdgcn_readfirstlane(int(k))) : k;
 }
 
-// Forward levels of one layout: distances stride*2^(levels-1) .. stride (those
-// >= n1).  `lazy_in`: the values are below 2p (left so by the group before);
-// the ones the first level does not multiply are reduced first.  The last
-// level of a group leaves its outputs below 2p, unless it is the transform's
-// last (distance n1): then they are below p, or stay below 2p with `lazy_out`.
-__device__ __forceinline__ void row_forward_group(uint32_t (&x)[8], int layout, int levels, uint32_t t,
-                                                  uint32_t stride, uint32_t n1, uint32_t base_index, bool lazy_in,
-                                                  bool lazy_out, const uint2* w, uint32_t p) {
-    if (lazy_in && (stride << (levels - 1)) >= n1) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-            if (!(e & (1 << (levels - 1)))) x[e] = min(x[e], x[e] - p);
+// The twiddles of one group of levels: level b (distance d = stride << b) has
+// 4 >> b of them per thread, at tw[(4 >> b) - 1 ..].  In layout A they are the
+// same for the whole block, in the others consecutive entries per thread.
+struct RowTables {
+    const uint2* tw;      // [r][n2]
+    const PrimeConst* consts;
+    uint32_t n2, k0, r;
+    uint32_t base;        // (rows + row) * C: level d starts at base / 2d
+    // primes past the last one are computed on its tables (and not stored)
+    template <int LOGC>
+    __device__ __forceinline__ uint32_t prime(uint32_t k) const {
+        return LOGC == 11 || k0 + k < r ? k0 + k : r - 1;
     }
+};
+
+template <int LOGC>
+__device__ __forceinline__ bool row_level(uint32_t d, uint32_t n1) {
+    return d >= n1 && 2 * d <= (1u << LOGC);
+}
+
+template <int LOGC>
+__device__ __forceinline__ void row_twiddles(uint2 (&tw)[7], const RowTables& tb, int layout, int levels, uint32_t t,
+                                             uint32_t stride, uint32_t n1) {
 #pragma unroll
-    for (int b = levels - 1; b >= 0; --b) {
+    for (int b = 0; b < levels; ++b) {
         const uint32_t d = stride << b;
-        if (d < n1) continue;
-        const bool last = d == n1;
+        if (!row_level<LOGC>(d, n1)) continue;
+        const uint32_t shift = 31 - __clz(2 * d);
+        const uint32_t first = layout == 0 ? 0 : (layout == 1 ? t >> 5 : layout == 2 ? t >> 2 : t) << (2 - b);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            if (e & (1 << b)) continue;
-            const uint2 tw = w[twiddle_index(layout, t, e, b, base_index, d)];
-            const bool reduce = last ? !lazy_out : b > 0 && !(e & (1 << (b - 1)));
-            if (reduce) ct_butterfly<true>(x[e], x[e + (1 << b)], tw, p);
-            else ct_butterfly<false>(x[e], x[e + (1 << b)], tw, p);
+        for (uint32_t s = 0; s < (4u >> b); ++s) {
+            const uint32_t k = layout_prime<LOGC>(layout, t, int(s << (b + 1)));
+            const uint32_t g = LOGC == 11 ? first + s : (first + s) & ((1u << (LOGC - shift)) - 1);
+            tw[(4u >> b) - 1 + s] = (tb.tw + size_t(tb.prime<LOGC>(k)) * tb.n2)[(tb.base >> shift) + g];
         }
     }
 }
 
-__device__ __forceinline__ void row_inverse_group(uint32_t (&x)[8], int layout, int levels, uint32_t t,
-                                                  uint32_t stride, uint32_t n1, uint32_t base_index,
-                                                  const uint2* w, uint32_t p) {
+// Forward levels of one group.  `lazy_in`: the values are below 2p (left so by
+// the group before); the ones the first level does not multiply are reduced
+// first.  The last level of a group leaves its outputs below 2p, unless it is
+// the transform's last (distance n1): then they are below p, or stay below 2p
+// with `lazy_out`.
+template <int LOGC>
+__device__ __forceinline__ void row_forward_group(uint32_t (&x)[8], const uint2 (&tw)[7], const uint32_t (&p)[8],
+                                                  int levels, uint32_t stride, uint32_t n1, bool lazy_in,
+                                                  bool lazy_out) {
+    if (lazy_in && row_level<LOGC>(stride << (levels - 1), n1)) {
 #pragma unroll
-    for (int b = 0; b < levels; ++b) {
+        for (int e = 0; e < 8; ++e)
+            if (!(e & (1 << (levels - 1)))) x[e] = min(x[e], x[e] - p[e]);
+    }
+#pragma unroll
+    for (int b = levels - 1; b >= 0; --b) {
         const uint32_t d = stride << b;
-        if (d < n1) continue;
+        if (!row_level<LOGC>(d, n1)) continue;
+        const bool last = d == n1;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             if (e & (1 << b)) continue;
-            gs_butterfly(x[e], x[e + (1 << b)], w[twiddle_index(layout, t, e, b, base_index, d)], p);
+            const uint2 w = tw[(4 >> b) - 1 + (e >> (b + 1))];
+            const bool reduce = last ? !lazy_out : b > 0 && !(e & (1 << (b - 1)));
+            if (reduce) ct_butterfly<true>(x[e], x[e + (1 << b)], w, p[e]);
+            else ct_butterfly<false>(x[e], x[e + (1 << b)], w, p[e]);
+        }
+    }
+}
+
+template <int LOGC>
+__device__ __forceinline__ void row_inverse_group(uint32_t (&x)[8], const uint2 (&tw)[7], const uint32_t (&p)[8],
+                                                  int levels, uint32_t stride, uint32_t n1) {
+#pragma unroll
+    for (int b = 0; b < levels; ++b) {
+        if (!row_level<LOGC>(stride << b, n1)) continue;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            if (e & (1 << b)) continue;
+            gs_butterfly(x[e], x[e + (1 << b)], tw[(4 >> b) - 1 + (e >> (b + 1))], p[e]);
         }
     }
 }
@@ -970,42 +1017,62 @@ __device__ __forceinline__ void row_exchange(uint32_t* buf, uint32_t (&x)[8], in
     __syncthreads();
 }
 
-template <uint32_t N1>
-__device__ __forceinline__ void rows_2048_body(uint32_t* __restrict__ planes, const uint32_t* __restrict__ bplanes,
-                                               const PrimeConst* __restrict__ consts, const uint2* __restrict__ twf,
-                                               const uint2* __restrict__ twi, uint32_t ps, uint32_t n2, uint32_t rows,
-                                               uint32_t row, uint32_t k) {
-    constexpr uint32_t n1 = N1;
+template <int LOGC, uint32_t N1>
+__device__ __forceinline__ void rows_reg_body(uint32_t* __restrict__ planes, const uint32_t* __restrict__ bplanes,
+                                              const PrimeConst* __restrict__ consts, const uint2* __restrict__ twf,
+                                              const uint2* __restrict__ twi, uint32_t ps, uint32_t n2, uint32_t rows,
+                                              uint32_t r, uint32_t row, uint32_t k0) {
+    constexpr uint32_t n1 = N1, C = 1u << LOGC;
+    constexpr int kFirst = LOGC >= 9 ? 0 : 1;  // layout of the loads and stores
     __shared__ uint32_t buf[2][kRowPadded];
     const uint32_t t = threadIdx.x;
-    const uint32_t p = consts[k].p, pinv = consts[k].pinv;
-    uint32_t* pa = planes + size_t(k) * ps + size_t(row) * kRowC;
-    const uint32_t* pb = bplanes + size_t(k) * ps + size_t(row) * kRowC;
-    const uint2* wf = twf + size_t(k) * n2;
-    const uint2* wi = twi + size_t(k) * n2;
-    // Table index of the group holding row-local jj at distance d:
-    // (rows + row) * (C / 2d) + jj / 2d  ==  ((rows + row) * C + jj) >> log2(2d).
-    const uint32_t base_index = (rows + row) * kRowC;
+    const RowTables fwd{twf, consts, n2, k0, r, (rows + row) * C}, inv{twi, consts, n2, k0, r, (rows + row) * C};
+    uint2 wa[7], wb[7];
     uint32_t xa[8], xb[8];
+    // the primes' values in each layout (D has C's)
+    uint32_t pa[8], pb[8], pc[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-        xa[e] = pa[t + 256 * e];
-        xb[e] = pb[t + 256 * e];
+        if constexpr (kFirst == 0) pa[e] = consts[fwd.prime<LOGC>(layout_prime<LOGC>(0, t, e))].p;
+        pb[e] = consts[fwd.prime<LOGC>(layout_prime<LOGC>(1, t, e))].p;
+        pc[e] = consts[fwd.prime<LOGC>(layout_prime<LOGC>(2, t, e))].p;
     }
-    row_forward_group(xa, 0, 3, t, 256, n1, base_index, false, N1 == 1, wf, p);
-    row_forward_group(xb, 0, 3, t, 256, n1, base_index, false, false, wf, p);
-    row_exchange(buf[0], xa, 0, 1, t);
-    row_exchange(buf[1], xb, 0, 1, t);
-    row_forward_group(xa, 1, 3, t, 32, n1, base_index, true, N1 == 1, wf, p);
-    row_forward_group(xb, 1, 3, t, 32, n1, base_index, true, false, wf, p);
+    auto place = [&](int e) {  // where value e lies in the planes, in the first layout
+        const size_t k = fwd.prime<LOGC>(layout_prime<LOGC>(kFirst, t, e));
+        return LOGC == 11 ? layout_index(kFirst, t, e) : k * ps + (layout_index(kFirst, t, e) & (C - 1));
+    };
+    if constexpr (LOGC == 11) {
+        planes += size_t(k0) * ps + size_t(row) * C;
+        bplanes += size_t(k0) * ps + size_t(row) * C;
+    }
+    if constexpr (kFirst == 0) row_twiddles<LOGC>(wa, fwd, 0, 3, t, 256, n1);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        xa[e] = planes[place(e)];
+        xb[e] = bplanes[place(e)];
+    }
+    row_twiddles<LOGC>(wb, fwd, 1, 3, t, 32, n1);
+    if constexpr (kFirst == 0) {
+        row_forward_group<LOGC>(xa, wa, pa, 3, 256, n1, false, false);
+        row_forward_group<LOGC>(xb, wa, pa, 3, 256, n1, false, false);
+        row_exchange(buf[0], xa, 0, 1, t);
+        row_exchange(buf[1], xb, 0, 1, t);
+    }
+    row_twiddles<LOGC>(wa, fwd, 2, 3, t, 4, n1);
+    row_forward_group<LOGC>(xa, wb, pb, 3, 32, n1, kFirst == 0, false);
+    row_forward_group<LOGC>(xb, wb, pb, 3, 32, n1, kFirst == 0, false);
     row_exchange(buf[0], xa, 1, 2, t);
     row_exchange(buf[1], xb, 1, 2, t);
-    row_forward_group(xa, 2, 3, t, 4, n1, base_index, true, N1 == 1, wf, p);
-    row_forward_group(xb, 2, 3, t, 4, n1, base_index, true, false, wf, p);
+    row_twiddles<LOGC>(wb, fwd, 3, 2, t, 1, n1);
+    row_forward_group<LOGC>(xa, wa, pc, 3, 4, n1, true, false);
+    row_forward_group<LOGC>(xb, wa, pc, 3, 4, n1, true, false);
     row_exchange(buf[0], xa, 2, 3, t);
     row_exchange(buf[1], xb, 2, 3, t);
-    row_forward_group(xa, 3, 2, t, 1, n1, base_index, true, N1 == 1, wf, p);
-    row_forward_group(xb, 3, 2, t, 1, n1, base_index, true, false, wf, p);
+    const uint32_t kd = fwd.prime<LOGC>(layout_prime<LOGC>(3, t, 0)), p = pc[0], pinv = consts[kd].pinv;
+    const uint2* wf = twf + size_t(kd) * n2;
+    row_twiddles<LOGC>(wa, inv, 3, 2, t, 1, n1);
+    row_forward_group<LOGC>(xa, wb, pc, 2, 1, n1, true, N1 == 1);
+    row_forward_group<LOGC>(xb, wb, pc, 2, 1, n1, true, false);
 
     // base case: thread t holds jj = 8t .. 8t+7, i.e. 8/n1 whole blocks.  Block g
     // is reduced mod (X^n1 - zeta_g): c_s = sum_{u<=s} a_u b_{s-u} + sum_{u>s}
@@ -1021,7 +1088,7 @@ __device__ __forceinline__ void rows_2048_body(uint32_t* __restrict__ planes, co
         uint32_t bw[n1i];  // bw[v] = zeta_g * b_v for v >= 1
         bw[0] = 0;
         if constexpr (n1i > 1) {
-            const uint32_t gb = (row * kRowC + 8 * t + blk0) / n1;  // global block index
+            const uint32_t gb = (row * C + ((8 * t + blk0) & (C - 1))) / n1;  // global block index
             uint2 w{0, 0};
             if (n2 != 1) w = wf[n2 / 2 + gb / 2];  // zeta_{2g} = w, zeta_{2g+1} = -w
 #pragma unroll
@@ -1055,24 +1122,32 @@ __device__ __forceinline__ void rows_2048_body(uint32_t* __restrict__ planes, co
         }
     }
 
-    row_inverse_group(xc, 3, 2, t, 1, n1, base_index, wi, p);
+    row_twiddles<LOGC>(wb, inv, 2, 3, t, 4, n1);
+    row_inverse_group<LOGC>(xc, wa, pc, 2, 1, n1);
     row_exchange(buf[0], xc, 3, 2, t);
-    row_inverse_group(xc, 2, 3, t, 4, n1, base_index, wi, p);
+    row_twiddles<LOGC>(wa, inv, 1, 3, t, 32, n1);
+    row_inverse_group<LOGC>(xc, wb, pc, 3, 4, n1);
     row_exchange(buf[0], xc, 2, 1, t);
-    row_inverse_group(xc, 1, 3, t, 32, n1, base_index, wi, p);
-    row_exchange(buf[0], xc, 1, 0, t);
-    row_inverse_group(xc, 0, 3, t, 256, n1, base_index, wi, p);
+    if constexpr (kFirst == 0) row_twiddles<LOGC>(wb, inv, 0, 3, t, 256, n1);
+    row_inverse_group<LOGC>(xc, wa, pb, 3, 32, n1);
+    if constexpr (kFirst == 0) {
+        row_exchange(buf[0], xc, 1, 0, t);
+        row_inverse_group<LOGC>(xc, wb, pa, 3, 256, n1);
+    }
 #pragma unroll
-    for (int e = 0; e < 8; ++e) pa[t + 256 * e] = xc[e];
+    for (int e = 0; e < 8; ++e)
+        if (LOGC == 11 || k0 + layout_prime<LOGC>(kFirst, t, e) < r) planes[place(e)] = xc[e];
 }
 
-template <uint32_t N1>
-__global__ __launch_bounds__(256) void ntt_rows_2048(uint32_t* __restrict__ planes,
-                                                     const uint32_t* __restrict__ bplanes,
-                                                     const PrimeConst* __restrict__ consts,
-                                                     const uint2* __restrict__ twf, const uint2* __restrict__ twi,
-                                                     uint32_t ps, uint32_t n2, uint32_t rows, uint32_t r) {
-    rows_2048_body<N1>(planes, bplanes, consts, twf, twi, ps, n2, rows, blockIdx.x, blockIdx.y);
+// Blocks (row, k0): one prime per block with C = 2048, else 2048 / C from k0 on.
+template <int LOGC, uint32_t N1>
+__global__ __launch_bounds__(256, LOGC < 8 ? 4 : 8) void ntt_rows_reg(uint32_t* __restrict__ planes,
+                                                       const uint32_t* __restrict__ bplanes,
+                                                       const PrimeConst* __restrict__ consts,
+                                                       const uint2* __restrict__ twf, const uint2* __restrict__ twi,
+                                                       uint32_t ps, uint32_t n2, uint32_t rows, uint32_t r) {
+    rows_reg_body<LOGC, N1>(planes, bplanes, consts, twf, twi, ps, n2, rows, r, blockIdx.x,
+                            blockIdx.y * (kRowC >> LOGC));
 }
 
 // ---------------------------------------------------------------------------
@@ -1633,13 +1708,14 @@ __global__ __launch_bounds__(256) void forward_reg_group(GroupLaunch g) {
                            rest % it.r, rest / it.r);
 }
 
-// grid per product: (rows, r)
-template <uint32_t N1>
-__global__ __launch_bounds__(256) void rows_2048_group(GroupLaunch g) {
+// grid per product: (rows, r / primes per block)
+template <int LOGC, uint32_t N1>
+__global__ __launch_bounds__(256, LOGC < 8 ? 4 : 8) void rows_reg_group(GroupLaunch g) {
     uint32_t local;
     const GroupView& it = group_entry(g, local);
-    rows_2048_body<N1>(in_global(it.planes), in_global(it.planes) + size_t(it.r_pad) * it.n_pad, in_global(it.consts), in_global(it.tw_fwd), in_global(it.tw_inv), it.n_pad,
-                       it.n2, it.rows, local % it.rows, local / it.rows);
+    rows_reg_body<LOGC, N1>(in_global(it.planes), in_global(it.planes) + size_t(it.r_pad) * it.n_pad,
+                            in_global(it.consts), in_global(it.tw_fwd), in_global(it.tw_inv), it.n_pad, it.n2, it.rows,
+                            it.r, local % it.rows, local / it.rows * (kRowC >> LOGC));
 }
 
 __global__ __launch_bounds__(256) void rows_product_group(GroupLaunch g) {
@@ -2008,21 +2084,36 @@ void launch_ntt_forward_columns(const Shape& s, const DeviceTables& t, uint32_t*
     check_launch("ntt_columns_forward");
 }
 
+namespace {
+
+// log2 of the row width the register kernel takes, or 0 where the LDS kernel
+// runs: rows narrower than 128 values, and blocks wider than 8.
+uint32_t row_variant(uint32_t row_width, uint32_t n1) {
+    uint32_t logc = 0;
+    while ((1u << logc) < row_width) ++logc;
+    return logc >= 7 && n1 <= 8 ? logc : 0;
+}
+
+}  // namespace
+
+#define PM_ROWS_VARIANTS(X)                                                                                 \
+    X(7, 1) X(7, 2) X(7, 4) X(7, 8) X(8, 1) X(8, 2) X(8, 4) X(8, 8) X(9, 1) X(9, 2) X(9, 4) X(9, 8) X(10, 1) \
+        X(10, 2) X(10, 4) X(10, 8) X(11, 1) X(11, 2) X(11, 4) X(11, 8)
+
 void launch_ntt_rows_product(const Shape& s, const DeviceTables& t, uint32_t* planes, const uint32_t* bplanes,
                              hipStream_t stream) {
-    const uint32_t ps = s.n_pad, r = s.r_pad;
-    dim3 grid(s.rows, s.r);
-    if (s.row_width == kRowC && s.n1 <= 8) {
-        switch (s.n1) {
-#define PM_ROWS(B)                                                                                              \
-    case B:                                                                                                     \
-        hipLaunchKernelGGL(ntt_rows_2048<B>, grid, dim3(256), 0, stream, planes, bplanes, t.consts, t.tw_fwd,     \
-                           t.tw_inv, ps, s.n2, s.rows, r);                                                      \
-        break;
-            PM_ROWS(1) PM_ROWS(2) PM_ROWS(4) PM_ROWS(8)
+    const uint32_t ps = s.n_pad, r = s.r_pad, logc = row_variant(s.row_width, s.n1);
+    if (logc) {
+        const uint32_t per = kRowC >> logc;  // primes per block
+        const dim3 grid(s.rows, (s.r + per - 1) / per);
+#define PM_ROWS(LC, B)                                                                                      \
+    if (logc == LC && s.n1 == B)                                                                            \
+        hipLaunchKernelGGL((ntt_rows_reg<LC, B>), grid, dim3(256), 0, stream, planes, bplanes, t.consts,     \
+                           t.tw_fwd, t.tw_inv, ps, s.n2, s.rows, s.r);
+        PM_ROWS_VARIANTS(PM_ROWS)
 #undef PM_ROWS
-        }
     } else {
+        const dim3 grid(s.rows, s.r);
         hipLaunchKernelGGL(ntt_rows_product, grid, dim3(256), size_t(2) * s.row_width * 4, stream, planes, bplanes,
                            t.consts, t.tw_fwd, t.tw_inv, ps, s.n1, s.n2, s.row_width, s.rows, r);
     }
@@ -2151,12 +2242,12 @@ namespace {
 
 // Launches of one batch: conversion from the limbs (one per variant),
 // pack and conversion, forward columns (one per row count),
-// rows (one per block size n1, and the LDS kernel), inverse columns (one per
+// rows (one per row width and block size n1, and the LDS kernel), inverse columns (one per
 // row count), CRT GEMM with reconstruction (one per wave-row count), CRT GEMM,
 // reconstruction.
-constexpr size_t kGroupLaunches = 8 + 2 + 6 + 5 + 7 + 3 + 2;
+constexpr size_t kGroupLaunches = 8 + 2 + 6 + 21 + 7 + 3 + 2;
 
-enum GroupKind { kConvert, kPack, kConversion, kForward, kRows2048, kRowsProduct, kInverse, kCrtRec, kCrt, kRecWave };
+enum GroupKind { kConvert, kPack, kConversion, kForward, kRowsReg, kRowsProduct, kInverse, kCrtRec, kCrt, kRecWave };
 
 size_t group_item_bytes(size_t count) { return (count * sizeof(GroupItem) + 255) / 256 * 256; }
 size_t group_table_words(size_t count) { return kGroupLaunches * (2 * count + 1); }
@@ -2207,7 +2298,6 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
         used += 2 * sel.size() + 1;
     };
     auto ntiles = [](const GroupItem& it) { return uint64_t(it.n_pad / kTile); };
-    auto rows_2048 = [](const GroupItem& it) { return it.row_width == kRowC && it.n1 <= 8; };
 #define PM_GCONV(K, N)                                                                                            \
     add(kConvert, K * 8 + N, [&](const GroupItem& it) {                                                           \
         return it.limbs <= kShortLimbs && it.conv_variant == K * 8 + N ? uint64_t(it.conv_split) * (8 / N) * ntiles(it) \
@@ -2225,11 +2315,17 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
         add(kForward, R, [&](const GroupItem& it) {
             return it.rows == R ? uint64_t(it.row_width / 256) * it.r * 2 : 0;
         });
-    for (uint32_t b = 1; b <= 8; b *= 2)
-        add(kRows2048, b, [&](const GroupItem& it) {
-            return rows_2048(it) && it.n1 == b ? uint64_t(it.rows) * it.r : 0;
-        });
-    add(kRowsProduct, 0, [&](const GroupItem& it) { return rows_2048(it) ? 0 : uint64_t(it.rows) * it.r; });
+#define PM_GROWS(LC, B)                                                                                        \
+    add(kRowsReg, LC * 16 + B, [&](const GroupItem& it) {                                                      \
+        return row_variant(it.row_width, it.n1) == LC && it.n1 == B                                            \
+                   ? uint64_t(it.rows) * ((it.r + (kRowC >> LC) - 1) / (kRowC >> LC))                          \
+                   : 0;                                                                                        \
+    });
+    PM_ROWS_VARIANTS(PM_GROWS)
+#undef PM_GROWS
+    add(kRowsProduct, 0, [&](const GroupItem& it) {
+        return row_variant(it.row_width, it.n1) ? 0 : uint64_t(it.rows) * it.r;
+    });
     for (uint32_t R = 1; R <= 64; R *= 2)
         add(kInverse, R, [&](const GroupItem& it) {
             return it.rows == R ? uint64_t(it.row_width / 16) * (it.r_pad / 16) : 0;
@@ -2275,15 +2371,12 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
 #undef PM_GFWD
                 }
                 break;
-            case kRows2048:
-                switch (L.variant) {
-#define PM_GROWS(B)                                                                     \
-    case B:                                                                             \
-        hipLaunchKernelGGL(rows_2048_group<B>, grid, dim3(256), 0, stream, g);           \
-        break;
-                    PM_GROWS(1) PM_GROWS(2) PM_GROWS(4) PM_GROWS(8)
+            case kRowsReg:
+#define PM_GROWS(LC, B)                                                                       \
+    if (L.variant == LC * 16 + B)                                                             \
+        hipLaunchKernelGGL((rows_reg_group<LC, B>), grid, dim3(256), 0, stream, g);
+                PM_ROWS_VARIANTS(PM_GROWS)
 #undef PM_GROWS
-                }
                 break;
             case kRowsProduct:
                 hipLaunchKernelGGL(rows_product_group, grid, dim3(256), L.lds, stream, g);

@@ -1,5 +1,6 @@
 """The transforms' lazy forms against the oracle where their ranges are tight:
-every row count of the register column kernels (2 to 64), each base case (n1 =
+every row width of the register row kernel (128 to 2048; 64 takes the LDS one)
+and row count of the register column kernels (2 to 64), each base case (n1 =
 1, 2, 4, 8, whose last level hands different ranges on) and primes just below
 2^31, with operands that are all q-1, alternate 0 and q-1, and random.
 Bit-exact, so there is no tolerance."""
@@ -9,7 +10,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [2048, 4096, 8192, 16384, 32768, 65536, 131072])
+@pytest.mark.parametrize("n", [64, 128, 256, 512, 1024, 2048, 4096, 8192, 16384, 32768, 65536, 131072])
 @pytest.mark.parametrize("block", [1, 2, 4, 8])
 def test_forms(polymul, workloads, oracle, n, block):
     print("[gpu-case] transform forms", n, block, flush=True)
