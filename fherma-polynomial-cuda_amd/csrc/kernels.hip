@@ -33,6 +33,7 @@
 #include <mutex>
 #include <stdexcept>
 #include <string>
+#include <type_traits>
 
 namespace pm {
 namespace {
@@ -1358,10 +1359,14 @@ __global__ __launch_bounds__(256) void reconstruct_waves(const int64_t* __restri
 struct CrtFusedArgs {
     uint32_t n, limbs, t_words;
     uint32_t ksteps, kstride;  // K steps that hold primes; K steps of a residue tile
+    uint32_t r, ps;            // primes; plane row stride (residues read from the planes)
     TileSet ts;                // output row k*256 + u is coefficient tile_at(ts, k)*256 + u
     uint32_t top_m, top_e, k_shift;
     uint64_t mu;
 };
+
+// Wave rows of the fused kernel: 16 word sums each.
+constexpr uint32_t fused_waves(uint32_t crt_words) { return crt_words <= 16 ? 1 : crt_words <= 32 ? 2 : 4; }
 
 constexpr uint32_t fused_row_words(uint32_t wm) { return 16 * wm + 2; }  // int64 per coefficient, 16-byte rows
 
@@ -1370,9 +1375,10 @@ constexpr size_t fused_lds_bytes(uint32_t wm, uint32_t nw, uint32_t ksteps) {
     return operands > sums ? operands : sums;
 }
 
-template <int WM, int NW>
+template <int WM, int NW, bool kPlanes>
 __device__ __forceinline__ void crt_reconstruct_body(const int8_t* __restrict__ wtiles,
-                                                     const int8_t* __restrict__ rtiles, uint32_t* __restrict__ c,
+                                                     const int8_t* __restrict__ rtiles,
+                                                     const uint32_t* __restrict__ planes, uint32_t* __restrict__ c,
                                                      const uint32_t* __restrict__ q,
                                                      const uint32_t* __restrict__ neg_p,
                                                      const uint32_t* __restrict__ corr_t,
@@ -1386,8 +1392,20 @@ __device__ __forceinline__ void crt_reconstruct_body(const int8_t* __restrict__ 
     const uint32_t L = args.limbs, tw = args.t_words, ksteps = args.ksteps;
     const uint32_t k0 = bx * T, tile = tile_at(args.ts, k0 / kTile), i0 = tile * kTile + k0 % kTile;
 
-    // operand bytes: slot tid of a K step holds row tid>>2, its chunk swizzled as in swz
-    {
+    // operand bytes, a row's chunk (16 bytes: four primes) swizzled as in swz
+    if constexpr (kPlanes) {  // thread -> coefficient tid % T, primes 4 (tid / T) .. + 3 of each K step
+        const uint32_t cf = tid % T, chunk = tid / T;
+        const uint32_t* src = planes + i0 + cf;
+        for (uint32_t ks = 0; ks < ksteps; ++ks) {
+            v4u x;
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) {  // primes past the last have zero weights: read the last one's again
+                const uint32_t k = ks * 16 + chunk * 4 + u;
+                x[u] = src[size_t(k < args.r ? k : args.r - 1) * args.ps];
+            }
+            *reinterpret_cast<v4u*>(lds + ks * (T * kTK) + swz(cf, chunk)) = x ^ 0x80808080u;
+        }
+    } else {  // slot tid of a K step holds row tid>>2
         const uint32_t row = tid >> 2, chunk = (tid & 3) ^ ((row >> 1) & 3);
         const int8_t* src = rtiles + size_t(tile) * args.kstride * kTileBytes + (k0 % kTile + row) * kTK + chunk * 16;
         for (uint32_t ks = 0; ks < ksteps; ++ks)
@@ -1593,15 +1611,16 @@ __device__ __forceinline__ void crt_reconstruct_body(const int8_t* __restrict__ 
     }
 }
 
-template <int WM, int NW>
+template <int WM, int NW, bool kPlanes>
 __global__ __launch_bounds__(64 * NW, 4) void crt_reconstruct(const int8_t* __restrict__ wtiles,
-                                                       const int8_t* __restrict__ rtiles, uint32_t* __restrict__ c,
+                                                       const int8_t* __restrict__ rtiles,
+                                                       const uint32_t* __restrict__ planes, uint32_t* __restrict__ c,
                                                        const uint32_t* __restrict__ q,
                                                        const uint32_t* __restrict__ neg_p,
                                                        const uint32_t* __restrict__ corr_t,
                                                        const uint32_t* __restrict__ corr_e, CrtFusedArgs args) {
     extern __shared__ __attribute__((aligned(16))) int8_t dyn_lds[];
-    crt_reconstruct_body<WM, NW>(wtiles, rtiles, c, q, neg_p, corr_t, corr_e, args, blockIdx.x, dyn_lds);
+    crt_reconstruct_body<WM, NW, kPlanes>(wtiles, rtiles, planes, c, q, neg_p, corr_t, corr_e, args, blockIdx.x, dyn_lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -1620,7 +1639,7 @@ __global__ __launch_bounds__(64 * NW, 4) void crt_reconstruct(const int8_t* __re
 struct GroupView {
     uint32_t n, n_pad, limbs, r, r_pad, conv_rows, conv_k, crt_rows, crt_k, crt_words, ws, t_words;
     uint32_t n1, n2, rows, row_width, s_shift, k_shift, top_m, top_e;
-    uint32_t conv_variant, conv_split;  // short conversion (launch_convert)
+    uint32_t conv_ks, conv_nt, conv_split;  // short conversion (launch_convert)
     uint64_t mu;
     const PM_GLOBAL PrimeConst* consts;
     const PM_GLOBAL int8_t* wconv;
@@ -1685,27 +1704,45 @@ __global__ __launch_bounds__(512) void conversion_group(GroupLaunch g) {
                     it.conv_k / kTK, every_tile(it), 0, 2, local);
 }
 
+// The grouped kernels of a stage hold several of its variants, chosen per
+// product, so that products of every size share one launch and its tail (the
+// batch of 64 small products: six launches of the CRT stage took 81 us, one
+// takes 43).
+
 // grid per product: (2 n_pad / 64 NT, prime splits)
-template <int KS, int NT>
 __global__ __launch_bounds__(256, 3) void convert_group(GroupLaunch g) {
     extern __shared__ __attribute__((aligned(16))) int8_t dyn_lds[];
     uint32_t local;
     const GroupView& it = group_entry(g, local);
-    const uint32_t nx = 2 * it.n_pad / (64 * NT);
+    const uint32_t nx = 2 * it.n_pad / (64 * it.conv_nt);
     const ConvertArgs args{it.n, it.n_pad, it.limbs, it.r, it.r_pad, it.conv_rows, it.conv_k / kTK,
                            every_tile(it), 0};
-    convert_body<KS, NT>(in_global(it.a), in_global(it.b), in_global(it.wconv), in_global(it.consts), in_global(it.planes), args, local % nx, local / nx, it.conv_split,
-                         dyn_lds);
+    auto run = [&](auto ks, auto nt) {
+        convert_body<ks(), nt()>(in_global(it.a), in_global(it.b), in_global(it.wconv), in_global(it.consts),
+                                 in_global(it.planes), args, local % nx, local / nx, it.conv_split, dyn_lds);
+    };
+    switch (it.conv_ks) {  // convert_plan's wide waves
+        case 1: run(std::integral_constant<int, 1>(), std::integral_constant<int, 4>()); break;
+        case 2: run(std::integral_constant<int, 2>(), std::integral_constant<int, 4>()); break;
+        case 4: run(std::integral_constant<int, 4>(), std::integral_constant<int, 4>()); break;
+        default: run(std::integral_constant<int, 8>(), std::integral_constant<int, 2>()); break;
+    }
 }
 
-// grid per product: (row_width / 256, r, 2)
+// grid per product: (row_width / 256, r, 2).  ROWS = 8 holds 2, 4 and 8 rows.
 template <int ROWS>
 __global__ __launch_bounds__(256) void forward_reg_group(GroupLaunch g) {
     uint32_t local;
     const GroupView& it = group_entry(g, local);
     const uint32_t nx = it.row_width / 256, bx = local % nx, rest = local / nx;
-    forward_reg_body<ROWS>(in_global(it.planes), in_global(it.consts), in_global(it.tw_fwd), it.n_pad, it.n2, it.row_width, it.r_pad, 0, 0, bx,
-                           rest % it.r, rest / it.r);
+    auto run = [&](auto rows) {
+        forward_reg_body<rows()>(in_global(it.planes), in_global(it.consts), in_global(it.tw_fwd), it.n_pad, it.n2,
+                                 it.row_width, it.r_pad, 0, 0, bx, rest % it.r, rest / it.r);
+    };
+    if (ROWS > 8) run(std::integral_constant<int, ROWS>());
+    else if (it.rows == 2) run(std::integral_constant<int, 2>());
+    else if (it.rows == 4) run(std::integral_constant<int, 4>());
+    else run(std::integral_constant<int, 8>());
 }
 
 // grid per product: (rows, r / primes per block)
@@ -1727,13 +1764,22 @@ __global__ __launch_bounds__(256) void rows_product_group(GroupLaunch g) {
 }
 
 // grid per product: (row_width / 16, r_pad / 16)
+// ROWS = 8 holds 1, 2, 4 and 8 rows.
 template <int ROWS>
 __global__ __launch_bounds__(256) void inverse_tiles_group(GroupLaunch g) {
     uint32_t local;
     const GroupView& it = group_entry(g, local);
     const uint32_t nx = it.row_width / 16;
-    inverse_tiles_body<ROWS>(in_global(it.planes), in_global(it.consts), in_global(it.tw_inv), it.n_pad, it.n, it.n2, it.row_width, it.r,
-                             it.r_pad / 16, in_global(it.rtiles), 0, local % nx, local / nx, nx);
+    auto run = [&](auto rows) {
+        inverse_tiles_body<rows()>(in_global(it.planes), in_global(it.consts), in_global(it.tw_inv), it.n_pad, it.n,
+                                   it.n2, it.row_width, it.r, it.r_pad / 16, in_global(it.rtiles), 0, local % nx,
+                                   local / nx, nx);
+    };
+    if (ROWS > 8) run(std::integral_constant<int, ROWS>());
+    else if (it.rows == 1) run(std::integral_constant<int, 1>());
+    else if (it.rows == 2) run(std::integral_constant<int, 2>());
+    else if (it.rows == 4) run(std::integral_constant<int, 4>());
+    else run(std::integral_constant<int, 8>());
 }
 
 __global__ __launch_bounds__(512) void crt_group(GroupLaunch g) {
@@ -1743,14 +1789,26 @@ __global__ __launch_bounds__(512) void crt_group(GroupLaunch g) {
              every_tile(it), local);
 }
 
-template <int WM, int NW>
-__global__ __launch_bounds__(64 * NW, 4) void crt_reconstruct_group(GroupLaunch g) {
+__global__ __launch_bounds__(256, 4) void crt_reconstruct_group(GroupLaunch g) {
     extern __shared__ __attribute__((aligned(16))) int8_t dyn_lds[];
     uint32_t local;
     const GroupView& it = group_entry(g, local);
-    const CrtFusedArgs args{it.n, it.limbs, it.t_words, (it.r + 15) / 16, it.r_pad / 16, every_tile(it),
-                            it.top_m, it.top_e, it.k_shift, it.mu};
-    crt_reconstruct_body<WM, NW>(in_global(it.wcrt), in_global(it.rtiles), in_global(it.c), in_global(it.q), in_global(it.neg_p), in_global(it.corr_t), in_global(it.corr_e), args, local, dyn_lds);
+    const CrtFusedArgs args{it.n, it.limbs, it.t_words, (it.r + 15) / 16, it.r_pad / 16, it.r, it.n_pad,
+                            every_tile(it), it.top_m, it.top_e, it.k_shift, it.mu};
+    auto run = [&](auto wm, auto from_planes) {
+        crt_reconstruct_body<wm(), 4, from_planes()>(in_global(it.wcrt), in_global(it.rtiles), in_global(it.planes),
+                                                     in_global(it.c), in_global(it.q), in_global(it.neg_p),
+                                                     in_global(it.corr_t), in_global(it.corr_e), args, local, dyn_lds);
+    };
+    auto residues = [&](auto wm) {
+        if (it.rows == 1) run(wm, std::true_type());  // residues_from_planes
+        else run(wm, std::false_type());
+    };
+    switch (fused_waves(it.crt_words)) {
+        case 1: residues(std::integral_constant<int, 1>()); break;
+        case 2: residues(std::integral_constant<int, 2>()); break;
+        default: residues(std::integral_constant<int, 4>()); break;
+    }
 }
 
 __global__ __launch_bounds__(256) void reconstruct_waves_group(GroupLaunch g) {
@@ -2166,35 +2224,35 @@ namespace {
 // Barrett window: the four words of x from m up (m = floor(s/32) - 1, or 0 below s = 64)
 uint32_t barrett_top(const Shape& s) { return s.s_shift >= 64 ? s.s_shift / 32 - 1 : 0; }
 
-// Wave rows of the fused kernel: 16 word sums each.
-uint32_t fused_waves(uint32_t crt_words) { return crt_words <= 16 ? 1 : crt_words <= 32 ? 2 : 4; }
-
 }  // namespace
 
-void launch_crt_reconstruct(const Shape& s, const DeviceTables& t, const int8_t* rtiles, uint32_t* c,
-                            const TileSet& ts, hipStream_t stream) {
+void launch_crt_reconstruct(const Shape& s, const DeviceTables& t, const int8_t* rtiles, const uint32_t* planes,
+                            uint32_t* c, const TileSet& ts, hipStream_t stream) {
     check_tiles(s, ts, "crt_reconstruct");
     if (!reconstruct_fused(s)) throw std::logic_error("crt_reconstruct: more word sums than a block holds");
     const uint32_t top_m = barrett_top(s), ksteps = (s.r + 15) / 16, wm = fused_waves(s.crt_words);
-    const CrtFusedArgs args{s.n, s.limbs, s.t_words, ksteps, s.r_pad / 16, ts, top_m, s.s_shift - 32 * top_m,
+    const CrtFusedArgs args{s.n, s.limbs, s.t_words, ksteps, s.r_pad / 16, s.r, s.n_pad, ts, top_m, s.s_shift - 32 * top_m,
                             s.k_shift, s.mu};
-#define PM_FUSED(W, NW)                                                                                          \
-    hipLaunchKernelGGL((crt_reconstruct<W, NW>), dim3(ts.count * (kTile / (16 * NW))), dim3(64 * NW),             \
-                       fused_lds_bytes(W, NW, ksteps), stream, t.wcrt, rtiles, c, t.q, t.neg_p, t.corr_t,         \
+#define PM_FUSED(W, NW, P)                                                                                       \
+    hipLaunchKernelGGL((crt_reconstruct<W, NW, P>), dim3(ts.count * (kTile / (16 * NW))), dim3(64 * NW),             \
+                       fused_lds_bytes(W, NW, ksteps), stream, t.wcrt, rtiles, planes, c, t.q, t.neg_p, t.corr_t,         \
                        t.corr_e, args)
     // Blocks of eight waves read the weights half as often per coefficient (at
     // N = 65536 with 55 limbs 23.4 us against 29.2 us with four waves); below
     // 65536 coefficients there are too few of them, and smaller blocks start sooner.
     const bool wide = ts.count >= 256;
-    if (wm == 1) {
-        if (wide) PM_FUSED(1, 8);
-        else PM_FUSED(1, 4);
-    } else if (wm == 2) {
-        if (wide) PM_FUSED(2, 8);
-        else PM_FUSED(2, 4);
+    if (residues_from_planes(s)) {
+        if (wm == 1) PM_FUSED(1, 4, true);
+        else if (wm == 2) PM_FUSED(2, 4, true);
+        else PM_FUSED(4, 4, true);
+    } else if (wide) {
+        if (wm == 1) PM_FUSED(1, 8, false);
+        else if (wm == 2) PM_FUSED(2, 8, false);
+        else PM_FUSED(4, 8, false);
     } else {
-        if (wide) PM_FUSED(4, 8);
-        else PM_FUSED(4, 4);
+        if (wm == 1) PM_FUSED(1, 4, false);
+        else if (wm == 2) PM_FUSED(2, 4, false);
+        else PM_FUSED(4, 4, false);
     }
 #undef PM_FUSED
     check_launch("crt_reconstruct");
@@ -2220,7 +2278,7 @@ GroupItem group_item(const Shape& s, const DeviceTables& t, const DeviceWork& w,
     it.n1 = s.n1, it.n2 = s.n2, it.rows = s.rows, it.row_width = s.row_width;
     it.s_shift = s.s_shift, it.k_shift = s.k_shift;
     const ConvertPlan cp = convert_plan(s.r, s.conv_k / kTK, 2 * s.n_pad / kTile, kConvertGroupBlocks);
-    it.conv_variant = cp.ks * 8 + cp.nt, it.conv_split = cp.split;
+    it.conv_ks = cp.ks, it.conv_nt = cp.nt, it.conv_split = cp.split;
     it.top_m = barrett_top(s);
     it.top_e = s.s_shift - 32 * it.top_m;
     it.mu = s.mu;
@@ -2240,12 +2298,11 @@ bool groupable(const Shape& s) {
 
 namespace {
 
-// Launches of one batch: conversion from the limbs (one per variant),
-// pack and conversion, forward columns (one per row count),
-// rows (one per row width and block size n1, and the LDS kernel), inverse columns (one per
-// row count), CRT GEMM with reconstruction (one per wave-row count), CRT GEMM,
-// reconstruction.
-constexpr size_t kGroupLaunches = 8 + 2 + 6 + 21 + 7 + 3 + 2;
+// Launches of one batch: conversion from the limbs, pack, conversion GEMM,
+// forward columns (four row-count classes), rows (one per row width and block
+// size n1, and the LDS kernel), inverse columns (four classes), CRT GEMM with
+// reconstruction, CRT GEMM, reconstruction.
+constexpr size_t kGroupLaunches = 1 + 2 + 4 + 21 + 4 + 1 + 2;
 
 enum GroupKind { kConvert, kPack, kConversion, kForward, kRowsReg, kRowsProduct, kInverse, kCrtRec, kCrt, kRecWave };
 
@@ -2278,6 +2335,8 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
         for (uint32_t i = 0; i < count; ++i)
             if (blocks(items[i]) > 0) sel.push_back(i);
         if (sel.empty()) return;
+        // the longest blocks (most primes) start first, the short ones fill the tail
+        std::stable_sort(sel.begin(), sel.end(), [&](uint32_t x, uint32_t y) { return items[x].r > items[y].r; });
         if (launches.size() == kGroupLaunches) throw std::logic_error("launch_group: more launches than planned");
         uint32_t* start = tables.data() + used;
         uint32_t* item = start + sel.size() + 1;
@@ -2288,7 +2347,7 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
             item[j] = sel[j];
             total += blocks(items[sel[j]]);
             const GroupItem& it = items[sel[j]];
-            lds = std::max<size_t>(lds, kind == kCrtRec    ? fused_lds_bytes(variant, 4, (it.r + 15) / 16)
+            lds = std::max<size_t>(lds, kind == kCrtRec    ? fused_lds_bytes(fused_waves(it.crt_words), 4, (it.r + 15) / 16)
                                         : kind == kConvert ? convert_lds_bytes(it.conv_k / kTK, it.r)
                                                            : size_t(2) * it.row_width * 4);
         }
@@ -2298,22 +2357,19 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
         used += 2 * sel.size() + 1;
     };
     auto ntiles = [](const GroupItem& it) { return uint64_t(it.n_pad / kTile); };
-#define PM_GCONV(K, N)                                                                                            \
-    add(kConvert, K * 8 + N, [&](const GroupItem& it) {                                                           \
-        return it.limbs <= kShortLimbs && it.conv_variant == K * 8 + N ? uint64_t(it.conv_split) * (8 / N) * ntiles(it) \
-                                                                       : 0;                                       \
+    add(kConvert, 0, [&](const GroupItem& it) {
+        return it.limbs <= kShortLimbs ? uint64_t(it.conv_split) * (8 / it.conv_nt) * ntiles(it) : 0;
     });
-    PM_CONVERT_VARIANTS(PM_GCONV)
-#undef PM_GCONV
     add(kPack, 0, [&](const GroupItem& it) {  // as launch_pack: 2 * ntiles * 256 rows
         return it.limbs <= kShortLimbs ? 0 : 128 * ntiles(it) / pack_rows_per_wave(it.conv_k / kTK);
     });
     add(kConversion, 0, [&](const GroupItem& it) {
         return it.limbs <= kShortLimbs ? 0 : uint64_t(it.conv_rows / kTile) * 2 * ntiles(it);
     });
-    for (uint32_t R = 2; R <= 64; R *= 2)
+    auto row_kernel = [](const GroupItem& it) { return it.rows < 8 ? 8 : it.rows; };
+    for (uint32_t R = 8; R <= 64; R *= 2)
         add(kForward, R, [&](const GroupItem& it) {
-            return it.rows == R ? uint64_t(it.row_width / 256) * it.r * 2 : 0;
+            return it.rows > 1 && row_kernel(it) == R ? uint64_t(it.row_width / 256) * it.r * 2 : 0;
         });
 #define PM_GROWS(LC, B)                                                                                        \
     add(kRowsReg, LC * 16 + B, [&](const GroupItem& it) {                                                      \
@@ -2326,14 +2382,12 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
     add(kRowsProduct, 0, [&](const GroupItem& it) {
         return row_variant(it.row_width, it.n1) ? 0 : uint64_t(it.rows) * it.r;
     });
-    for (uint32_t R = 1; R <= 64; R *= 2)
+    for (uint32_t R = 8; R <= 64; R *= 2)
         add(kInverse, R, [&](const GroupItem& it) {
-            return it.rows == R ? uint64_t(it.row_width / 16) * (it.r_pad / 16) : 0;
+            const bool skip = it.rows == 1 && it.crt_words <= kFusedWords;  // residues_from_planes
+            return row_kernel(it) == R && !skip ? uint64_t(it.row_width / 16) * (it.r_pad / 16) : 0;
         });
-    for (uint32_t wm = 1; wm <= 4; wm *= 2)
-        add(kCrtRec, wm, [&](const GroupItem& it) {
-            return it.crt_words <= kFusedWords && fused_waves(it.crt_words) == wm ? 4 * ntiles(it) : 0;
-        });
+    add(kCrtRec, 0, [&](const GroupItem& it) { return it.crt_words <= kFusedWords ? 4 * ntiles(it) : 0; });
     add(kCrt, 0, [&](const GroupItem& it) {
         return it.crt_words <= kFusedWords ? 0 : uint64_t(it.crt_rows / kTile) * ntiles(it);
     });
@@ -2349,11 +2403,7 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
         const dim3 grid(uint32_t(L.blocks));
         switch (L.kind) {
             case kConvert:
-#define PM_GCONV(K, N)                                                                       \
-    if (L.variant == K * 8 + N)                                                              \
-        hipLaunchKernelGGL((convert_group<K, N>), grid, dim3(256), L.lds, stream, g);
-                PM_CONVERT_VARIANTS(PM_GCONV)
-#undef PM_GCONV
+                hipLaunchKernelGGL(convert_group, grid, dim3(256), L.lds, stream, g);
                 break;
             case kPack:
                 hipLaunchKernelGGL(pack_group, grid, dim3(256), 0, stream, g);
@@ -2367,7 +2417,7 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
     case R:                                                                             \
         hipLaunchKernelGGL(forward_reg_group<R>, grid, dim3(256), 0, stream, g);         \
         break;
-                    PM_GFWD(2) PM_GFWD(4) PM_GFWD(8) PM_GFWD(16) PM_GFWD(32) PM_GFWD(64)
+                    PM_GFWD(8) PM_GFWD(16) PM_GFWD(32) PM_GFWD(64)
 #undef PM_GFWD
                 }
                 break;
@@ -2387,19 +2437,12 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
     case R:                                                                             \
         hipLaunchKernelGGL(inverse_tiles_group<R>, grid, dim3(256), 0, stream, g);       \
         break;
-                    PM_GINV(1) PM_GINV(2) PM_GINV(4) PM_GINV(8) PM_GINV(16) PM_GINV(32) PM_GINV(64)
+                    PM_GINV(8) PM_GINV(16) PM_GINV(32) PM_GINV(64)
 #undef PM_GINV
                 }
                 break;
             case kCrtRec:
-                switch (L.variant) {
-#define PM_GFUSED(W)                                                                    \
-    case W:                                                                             \
-        hipLaunchKernelGGL((crt_reconstruct_group<W, 4>), grid, dim3(256), L.lds, stream, g); \
-        break;
-                    PM_GFUSED(1) PM_GFUSED(2) PM_GFUSED(4)
-#undef PM_GFUSED
-                }
+                hipLaunchKernelGGL(crt_reconstruct_group, grid, dim3(256), L.lds, stream, g);
                 break;
             case kCrt:
                 hipLaunchKernelGGL(crt_group, grid, dim3(kGemmThreads), 0, stream, g);

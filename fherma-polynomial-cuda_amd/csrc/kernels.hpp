@@ -41,6 +41,9 @@ struct DeviceWork {
 // crt_words rounded up to 16 (128-byte rows) above 64 words.
 constexpr uint32_t kFusedWords = 64;
 inline bool reconstruct_fused(const Shape& s) { return s.crt_words <= kFusedWords; }
+// One transform row: the inverse column stage would be a mere transpose into
+// the CRT operand tiles, which the fused kernel does on its way into LDS.
+inline bool residues_from_planes(const Shape& s) { return s.rows == 1 && reconstruct_fused(s); }
 inline uint32_t word_stride(const Shape& s) { return s.t_words > 64 ? (s.crt_words + 15) / 16 * 16 : s.crt_words; }
 inline size_t word_sum_elements(const Shape& s) { return size_t(s.n_pad) * word_stride(s); }
 
@@ -100,8 +103,10 @@ void launch_crt(const Shape& s, const DeviceTables& t, const int8_t* rtiles, int
 // takes the residue tiles and writes each word of c once, so c may well be
 // pinned host memory; launch_reconstruct takes the word sums, and a coefficient
 // whose quotient estimate was off is written again by a later pass.
-void launch_crt_reconstruct(const Shape& s, const DeviceTables& t, const int8_t* rtiles, uint32_t* c,
-                            const TileSet& ts, hipStream_t stream);
+// With residues_from_planes(s) it reads the row stage's results in `planes`
+// itself, and no inverse column launch is needed.
+void launch_crt_reconstruct(const Shape& s, const DeviceTables& t, const int8_t* rtiles, const uint32_t* planes,
+                            uint32_t* c, const TileSet& ts, hipStream_t stream);
 void launch_reconstruct(const Shape& s, const DeviceTables& t, const int64_t* words, uint32_t* c, const TileSet& ts,
                         hipStream_t stream);
 void launch_zero(uint32_t* c, size_t words, hipStream_t stream);
@@ -114,7 +119,7 @@ void launch_zero(uint32_t* c, size_t words, hipStream_t stream);
 struct GroupItem {
     uint32_t n, n_pad, limbs, r, r_pad, conv_rows, conv_k, crt_rows, crt_k, crt_words, ws, t_words;
     uint32_t n1, n2, rows, row_width, s_shift, k_shift, top_m, top_e;
-    uint32_t conv_variant, conv_split;  // short conversion (launch_convert)
+    uint32_t conv_ks, conv_nt, conv_split;  // short conversion (launch_convert)
     uint64_t mu;
     const PrimeConst* consts;
     const int8_t* wconv;

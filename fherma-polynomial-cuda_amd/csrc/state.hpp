@@ -338,7 +338,8 @@ struct pm_plan {
             }
             if (!chunks.strips) pm::launch_ntt_forward_columns(s, tables, work.planes, 0, nops, stream);
             pm::launch_ntt_rows_product(s, tables, work.planes, bplanes, stream);
-            if (!chunks.strips) pm::launch_ntt_inverse_columns(s, tables, work.planes, work.rtiles, stream);
+            if (!chunks.strips && !pm::residues_from_planes(s))
+                pm::launch_ntt_inverse_columns(s, tables, work.planes, work.rtiles, stream);
             // Output half, per chunk: the inverse column stages of the strips it
             // starts, its CRT GEMM, its reconstruction, then its D2H on the copy
             // stream, which overlaps the next chunk's GEMM.
@@ -349,7 +350,8 @@ struct pm_plan {
                     pm::launch_ntt_inverse_columns(s, tables, work.planes, work.rtiles, stream, chunks.inv_begin[ch],
                                                    chunks.inv_end[ch]);
                 if (direct) {
-                    pm::launch_crt_reconstruct(s, tables, work.rtiles, lane->pin_out + at, chunks.set[ch], stream);
+                    pm::launch_crt_reconstruct(s, tables, work.rtiles, work.planes, lane->pin_out + at, chunks.set[ch],
+                                               stream);
                     hip_check(hipEventRecord(lane->out_ready[ch], stream), "hipEventRecord");
                     continue;
                 }
@@ -552,11 +554,12 @@ struct pm_plan {
         mark(3);
         pm::launch_ntt_rows_product(s, tables, w.planes, bplanes, st);
         mark(4);
-        pm::launch_ntt_inverse_columns(s, tables, w.planes, w.rtiles, st);
+        if (!pm::residues_from_planes(s) || last != PM_STAGE_OUTPUT)
+            pm::launch_ntt_inverse_columns(s, tables, w.planes, w.rtiles, st);
         mark(5);
         if (last == PM_STAGE_PRODUCT) return;
         if (pm::reconstruct_fused(s) && last != PM_STAGE_WORDS) {  // reported as the CRT GEMM's time
-            pm::launch_crt_reconstruct(s, tables, w.rtiles, c, all, st);
+            pm::launch_crt_reconstruct(s, tables, w.rtiles, w.planes, c, all, st);
             mark(6);
         } else {
             pm::launch_crt(s, tables, w.rtiles, w.words, all, st);
