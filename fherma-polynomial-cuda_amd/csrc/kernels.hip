@@ -1329,6 +1329,233 @@ __global__ __launch_bounds__(256) void reconstruct_waves(const int64_t* __restri
 }
 
 // ---------------------------------------------------------------------------
+// Reconstruction of one coefficient by G lanes, four consecutive words each (the
+// formulas are those of reconstruct_waves): shared by the fused kernel and the
+// one for wider q.
+// ---------------------------------------------------------------------------
+
+// What one lane needs to form K and the Barrett estimate Qe of a coefficient:
+// the same constants for every lane.
+struct QuotientWords {
+    uint32_t ce[4], top_c[4], top_n[4];
+    __device__ __forceinline__ void load(const uint32_t* __restrict__ neg_p, const uint32_t* __restrict__ corr_t,
+                                         const uint32_t* __restrict__ corr_e, uint32_t L, uint32_t tw,
+                                         uint32_t top_m) {
+#pragma unroll
+        for (uint32_t t = 0; t < 4; ++t) {
+            const uint32_t j = top_m + t;
+            const uint32_t cv = corr_t[j < tw ? j : tw - 1], nv = neg_p[j < L ? j : L - 1];
+            top_c[t] = j < tw ? cv : 0;
+            top_n[t] = j < L ? nv : 0;
+            ce[t] = corr_e[t];
+        }
+    }
+    // d: the coefficient's word sums.  Leaves K in k32.
+    __device__ __forceinline__ uint64_t quotient(const int64_t* d, uint32_t L, uint32_t top_m, uint32_t top_e,
+                                                 uint32_t k_shift, uint64_t mu, uint32_t& k32) const {
+        int64_t e[3], dt[4];
+#pragma unroll
+        for (uint32_t j = 0; j < 3; ++j) e[j] = d[L + 1 + j];
+#pragma unroll
+        for (uint32_t t = 0; t < 4; ++t) {
+            const uint32_t j = top_m + t;
+            dt[t] = d[j <= L ? j : L];
+            if (j > L) dt[t] = 0;
+        }
+        // K = floor((E + 2^63) / 2^64)
+        uint32_t ew[4];
+        int64_t carry = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+            const int64_t x = (j < 3 ? e[j] : 0) + int64_t(ce[j]) + carry;
+            ew[j] = uint32_t(uint64_t(x));
+            carry = x >> 32;
+        }
+        const uint32_t k = uint32_t(ew[2] + ((uint64_t(ew[1]) + 0x80000000ull) >> 32));
+        k32 = k;
+        // the four words at top_m (words past the last are zero)
+        unsigned __int128 sum = 0;
+#pragma unroll
+        for (uint32_t t = 0; t < 4; ++t) {
+            const int64_t x = dt[t] + int64_t(top_c[t]) + int64_t(uint64_t(k) * top_n[t]);
+            sum += (unsigned __int128)(__int128)x << (32 * t);
+        }
+        __int128 ts = __int128(sum) >> top_e;
+        if (ts < 0) ts = 0;
+        return uint64_t(((unsigned __int128)uint64_t(ts) * mu) >> k_shift);
+    }
+};
+
+// Lane g of a group of G: its four words of the constants, and the group's part
+// of a reconstruction.  Whole waves call reconstruct together.
+template <int G>
+struct LaneWords {
+    uint32_t g;
+    uint32_t ct[4], np[4], qv[6];  // qv[u + 2] = q[4g + u], two words below included
+    __device__ __forceinline__ void load(const uint32_t* __restrict__ q, const uint32_t* __restrict__ neg_p,
+                                         const uint32_t* __restrict__ corr_t, uint32_t L, uint32_t tw, uint32_t lane) {
+        g = lane;
+        // (every load unconditional, its index clamped, the value selected after)
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+            const uint32_t j = 4 * g + u;
+            const uint32_t cv = corr_t[j < tw ? j : tw - 1], nv = neg_p[j < L ? j : L - 1];
+            ct[u] = j < tw ? cv : 0;
+            np[u] = j < L ? nv : 0;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 6; ++u) {
+            const uint32_t j = 4 * g + u - 2;  // wraps above L below word 0
+            const uint32_t v = q[j < L ? j : L - 1];
+            qv[u] = j < L ? v : 0;
+        }
+    }
+    // Adds cin to the lane's words; returns the carry out.
+    static __device__ __forceinline__ int32_t add_carry(uint32_t (&w)[4], int32_t cin) {
+        int64_t t = cin;
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+            t += int64_t(w[u]);
+            w[u] = uint32_t(uint64_t(t));
+            t >>= 32;
+        }
+        return int32_t(t);
+    }
+    // Passes each lane's carry to the next lane of its group until none is left;
+    // the last lane's carries add up in `top` (0 on the other lanes).
+    __device__ __forceinline__ void settle(uint32_t (&w)[4], int32_t carry, int32_t& top) const {
+        for (;;) {
+            if (g == G - 1) top += carry;
+            int32_t cin;
+            if constexpr (G <= 16) cin = __builtin_amdgcn_update_dpp(0, carry, 0x111, 0xF, 0xF, true);  // row_shr:1
+            else cin = __shfl_up(carry, 1, 64);
+            if (g == 0) cin = 0;
+            if (!__ballot(cin != 0)) break;
+            carry = add_carry(w, cin);
+        }
+    }
+    // The lane's word sums out of the coefficient's, d (those past word L hold E
+    // or nothing of the row's, and are 0 here).
+    __device__ __forceinline__ void sums(const int64_t* d, uint32_t L, int64_t (&x)[4]) const {
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+            const uint32_t j = 4 * g + u;
+            const int64_t v = d[j <= L ? j : L];
+            x[u] = j <= L ? v : 0;
+        }
+    }
+    // The lane's words of (T - Qe*q) mod q, from its word sums; `valid` false:
+    // they are garbage, and so are the words.
+    __device__ __forceinline__ void reconstruct(const int64_t (&d)[4], uint64_t qe, uint32_t k32, bool valid,
+                                                uint32_t (&w)[4]) const {
+        const uint32_t lane = threadIdx.x & 63, shift = lane & ~uint32_t(G - 1), last = lane | (G - 1);
+        constexpr uint64_t mask = G == 64 ? ~uint64_t(0) : (uint64_t(1) << (G & 63)) - 1;
+        // R = T - Qe*q: this lane's four words and the carry out of them
+        const uint64_t q0 = uint32_t(qe), q1 = uint32_t(qe >> 32);
+        int32_t top = 0;
+        {
+            uint64_t pa = q0 * qv[1], pc = q1 * qv[1], pc2 = q1 * qv[0];
+            int64_t carry = 0;
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) {
+                const uint64_t a = q0 * qv[u + 2];
+                const int64_t sub = int64_t(uint32_t(a)) + int64_t(pa >> 32) + int64_t(uint32_t(pc)) + int64_t(pc2 >> 32);
+                carry += d[u] + int64_t(ct[u]) + int64_t(uint64_t(k32) * np[u]) - sub;
+                w[u] = uint32_t(uint64_t(carry));
+                carry >>= 32;
+                pa = a, pc2 = pc, pc = q1 * qv[u + 2];
+            }
+            settle(w, int32_t(carry), top);
+        }
+        for (int pass = 0; pass < 6; ++pass) {
+            bool gt = false, lt = false;
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) {  // the highest differing word decides
+                if (w[u] != qv[u + 2]) gt = w[u] > qv[u + 2], lt = !gt;
+            }
+            const uint64_t gm = (__ballot(gt) >> shift) & mask, lm = (__ballot(lt) >> shift) & mask;
+            const bool neg = (__ballot(top < 0) >> last) & 1, pos = (__ballot(top > 0) >> last) & 1;
+            const int32_t adj = !valid ? 0 : neg ? 1 : (pos || gm >= lm) ? -1 : 0;
+            if (!__ballot(adj != 0)) break;
+            int64_t carry = 0;
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) {
+                carry += int64_t(w[u]) + (adj > 0 ? int64_t(qv[u + 2]) : adj < 0 ? -int64_t(qv[u + 2]) : 0);
+                w[u] = uint32_t(uint64_t(carry));
+                carry >>= 32;
+            }
+            settle(w, int32_t(carry), top);
+        }
+    }
+};
+
+// ---------------------------------------------------------------------------
+// 6''. reconstruction for q of 61 to 252 limbs, from the CRT GEMM's sums in
+// memory: G = 32 or 64 lanes per coefficient (up to 128 or 256 words), blocks of
+// NP passes of 256 / G coefficients, whose sums are all loaded ahead; K and Qe
+// by one lane per coefficient as in the fused kernel.
+// reconstruct_waves spends a whole wave on every 64 words and forms K and Qe in
+// all 64 lanes: N = 8192 with 226 limbs 18.1 us, here 8.1; a
+// batch of 64 small products 70 us, here 25.
+// ---------------------------------------------------------------------------
+constexpr uint32_t kWideWords = 256;
+
+template <int G, int NP>
+__device__ __forceinline__ void reconstruct_wide_body(const int64_t* __restrict__ words, uint32_t* __restrict__ c,
+                                                      const uint32_t* __restrict__ q,
+                                                      const uint32_t* __restrict__ neg_p,
+                                                      const uint32_t* __restrict__ corr_t,
+                                                      const uint32_t* __restrict__ corr_e,
+                                                      const WaveReconstructArgs& args, uint32_t bx) {
+    typedef uint32_t v4u_word __attribute__((ext_vector_type(4), aligned(4)));  // 4-byte aligned
+    constexpr uint32_t T = 256 / G * NP;
+    __shared__ uint64_t quotient[T];
+    __shared__ uint32_t multiple[T];
+    const uint32_t tid = threadIdx.x, g = tid % G, L = args.limbs;
+    const uint32_t k0 = bx * T, i0 = tile_at(args.ts, k0 / kTile) * kTile + k0 % kTile;
+    if (i0 >= args.n) return;  // whole block
+    const int64_t* rows = words + size_t(i0) * args.ws;
+    LaneWords<G> lw;
+    int64_t d[NP][4];
+    lw.load(q, neg_p, corr_t, L, args.t_words, g);
+#pragma unroll
+    for (uint32_t ps = 0; ps < NP; ++ps) lw.sums(rows + size_t(tid / G + ps * (256 / G)) * args.ws, L, d[ps]);
+    if (tid < T) {
+        QuotientWords qw;
+        qw.load(neg_p, corr_t, corr_e, L, args.t_words, args.top_m);
+        quotient[tid] = qw.quotient(rows + size_t(tid) * args.ws, L, args.top_m, args.top_e, args.k_shift, args.mu,
+                                    multiple[tid]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t ps = 0; ps < NP; ++ps) {
+        const uint32_t cl = tid / G + ps * (256 / G);
+        uint32_t w[4];
+        const bool valid = i0 + cl < args.n;
+        lw.reconstruct(d[ps], quotient[cl], multiple[cl], valid, w);
+        uint32_t* out = c + size_t(k0 + cl) * L + 4 * g;
+        if (!valid) continue;
+        if (4 * g + 4 <= L) {
+            *reinterpret_cast<v4u_word*>(out) = v4u{w[0], w[1], w[2], w[3]};
+        } else {
+#pragma unroll
+            for (uint32_t u = 0; u < 3; ++u)
+                if (4 * g + u < L) out[u] = w[u];
+        }
+    }
+}
+
+template <int G, int NP>
+__global__ __launch_bounds__(256) void reconstruct_wide(const int64_t* __restrict__ words, uint32_t* __restrict__ c,
+                                                        const uint32_t* __restrict__ q,
+                                                        const uint32_t* __restrict__ neg_p,
+                                                        const uint32_t* __restrict__ corr_t,
+                                                        const uint32_t* __restrict__ corr_e,
+                                                        WaveReconstructArgs args) {
+    reconstruct_wide_body<G, NP>(words, c, q, neg_p, corr_t, corr_e, args, blockIdx.x);
+}
+
+// ---------------------------------------------------------------------------
 // 5+6. CRT GEMM and reconstruction in one kernel, for q of up to 60 limbs (at
 // most 64 word sums): a block of NW waves owns 16 NW coefficients and all
 // their word sums, so the sums never leave the CU.
@@ -1447,34 +1674,11 @@ __device__ __forceinline__ void crt_reconstruct_body(const int8_t* __restrict__ 
     }
     if (ks < ksteps) step(ks, f0, f2);
     if (ks + 1 < ksteps) step(ks + 1, f1, f0);
-    // this lane's four words of the constants
-    const uint32_t g = tid % G, j0 = 4 * g;
-    // (every load unconditional, its index clamped, the value selected after)
-    uint32_t ct[4], np[4], qv[6];  // qv[u + 2] = q[j0 + u], two words below included
-#pragma unroll
-    for (uint32_t u = 0; u < 4; ++u) {
-        const uint32_t j = j0 + u;
-        const uint32_t cv = corr_t[j < tw ? j : tw - 1], nv = neg_p[j < L ? j : L - 1];
-        ct[u] = j < tw ? cv : 0;
-        np[u] = j < L ? nv : 0;
-    }
-#pragma unroll
-    for (uint32_t u = 0; u < 6; ++u) {
-        const uint32_t j = j0 + u - 2;  // wraps above L below word 0
-        const uint32_t v = q[j < L ? j : L - 1];
-        qv[u] = j < L ? v : 0;
-    }
-    uint32_t top_c[4], top_n[4];  // the Barrett window's constants, the same for every lane
-#pragma unroll
-    for (uint32_t t = 0; t < 4; ++t) {
-        const uint32_t j = args.top_m + t;
-        const uint32_t cv = corr_t[j < tw ? j : tw - 1], nv = neg_p[j < L ? j : L - 1];
-        top_c[t] = j < tw ? cv : 0;
-        top_n[t] = j < L ? nv : 0;
-    }
-    uint32_t ce[4];
-#pragma unroll
-    for (uint32_t j = 0; j < 4; ++j) ce[j] = corr_e[j];
+    const uint32_t g = tid % G;
+    LaneWords<G> lw;
+    lw.load(q, neg_p, corr_t, L, tw, g);
+    QuotientWords qw;
+    qw.load(neg_p, corr_t, corr_e, L, tw, args.top_m);
     __syncthreads();  // every wave has read the operand bytes; the sums go over them
     int64_t* sums = reinterpret_cast<int64_t*>(lds);
     const DigitScales ds = digit_scales();
@@ -1485,114 +1689,20 @@ __device__ __forceinline__ void crt_reconstruct_body(const int8_t* __restrict__ 
             sums[((wn * NT + ni) * 16 + (lane & 15)) * S + wm * 16 + mi * 4 + (lane >> 4)] = combine4(acc[mi][ni], ds);
     __syncthreads();
 
-    const uint32_t shift = lane & ~(G - 1), last = lane | (G - 1);
-    const uint64_t group_mask = (uint64_t(1) << G) - 1;
-    // The lane's words plus carry-in `cin`; returns the carry out.
-    auto add_carry = [](uint32_t (&w)[4], int32_t cin) {
-        int64_t t = cin;
-#pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) {
-            t += int64_t(w[u]);
-            w[u] = uint32_t(uint64_t(t));
-            t >>= 32;
-        }
-        return int32_t(t);
-    };
-    // Passes each lane's carry to the next lane of its group until none is left;
-    // the last lane's carries add up in `top` (0 on the other lanes).
-    auto settle = [&](uint32_t (&w)[4], int32_t carry, int32_t& top) {
-        for (;;) {
-            if (g == G - 1) top += carry;
-            int32_t cin = __builtin_amdgcn_update_dpp(0, carry, 0x111, 0xF, 0xF, true);  // row_shr:1
-            if (g == 0) cin = 0;
-            if (!__ballot(cin != 0)) break;
-            carry = add_carry(w, cin);
-        }
-    };
     // K and the Barrett quotient Qe: one lane per coefficient, for all of them
-    if (tid < T) {
-        const int64_t* d = sums + tid * S;
-        int64_t e[3], dt[4];
-#pragma unroll
-        for (uint32_t j = 0; j < 3; ++j) e[j] = d[L + 1 + j];
-#pragma unroll
-        for (uint32_t t = 0; t < 4; ++t) {
-            const uint32_t j = args.top_m + t;
-            dt[t] = d[j <= L ? j : L];
-            if (j > L) dt[t] = 0;
-        }
-        // K = floor((E + 2^63) / 2^64)
-        uint32_t ew[4];
-        int64_t carry = 0;
-#pragma unroll
-        for (uint32_t j = 0; j < 4; ++j) {
-            const int64_t x = (j < 3 ? e[j] : 0) + int64_t(ce[j]) + carry;
-            ew[j] = uint32_t(uint64_t(x));
-            carry = x >> 32;
-        }
-        const uint32_t k32 = uint32_t(ew[2] + ((uint64_t(ew[1]) + 0x80000000ull) >> 32));
-        // the four words at top_m (words past the last are zero)
-        unsigned __int128 sum = 0;
-#pragma unroll
-        for (uint32_t t = 0; t < 4; ++t) {
-            const int64_t x = dt[t] + int64_t(top_c[t]) + int64_t(uint64_t(k32) * top_n[t]);
-            sum += (unsigned __int128)(__int128)x << (32 * t);
-        }
-        __int128 ts = __int128(sum) >> args.top_e;
-        if (ts < 0) ts = 0;
-        quotient[tid] = uint64_t(((unsigned __int128)uint64_t(ts) * args.mu) >> args.k_shift);
-        multiple[tid] = k32;
-    }
+    if (tid < T) quotient[tid] = qw.quotient(sums + tid * S, L, args.top_m, args.top_e, args.k_shift, args.mu, multiple[tid]);
     __syncthreads();
 #pragma unroll 1
     for (uint32_t cl = tid / G; cl < T; cl += 64 * NW / G) {  // whole waves: T G is a multiple of the threads
-        const int64_t* d = sums + cl * S;
-        const uint64_t qe = quotient[cl];
-        const uint32_t k32 = multiple[cl];
-        // R = T - Qe*q: this lane's four words and the carry out of them
-        const uint64_t q0 = uint32_t(qe), q1 = uint32_t(qe >> 32);
         uint32_t w[4];
-        int32_t top = 0;
-        {
-            uint64_t pa = q0 * qv[1], pc = q1 * qv[1], pc2 = q1 * qv[0];
-            int64_t carry = 0;
-#pragma unroll
-            for (uint32_t u = 0; u < 4; ++u) {
-                const uint64_t a = q0 * qv[u + 2];
-                const int64_t sub = int64_t(uint32_t(a)) + int64_t(pa >> 32) + int64_t(uint32_t(pc)) + int64_t(pc2 >> 32);
-                const int64_t dj = d[j0 + u];  // words past L hold E or the row's pad
-                carry += (j0 + u <= L ? dj : 0) + int64_t(ct[u]) + int64_t(uint64_t(k32) * np[u]) - sub;
-                w[u] = uint32_t(uint64_t(carry));
-                carry >>= 32;
-                pa = a, pc2 = pc, pc = q1 * qv[u + 2];
-            }
-            settle(w, int32_t(carry), top);
-        }
-        const bool valid = i0 + cl < args.n;
-        for (int pass = 0; pass < 6; ++pass) {
-            bool gt = false, lt = false;
-#pragma unroll
-            for (uint32_t u = 0; u < 4; ++u) {  // the highest differing word decides
-                if (w[u] != qv[u + 2]) gt = w[u] > qv[u + 2], lt = !gt;
-            }
-            const uint64_t gm = (__ballot(gt) >> shift) & group_mask, lm = (__ballot(lt) >> shift) & group_mask;
-            const bool neg = (__ballot(top < 0) >> last) & 1, pos = (__ballot(top > 0) >> last) & 1;
-            const int32_t adj = !valid ? 0 : neg ? 1 : (pos || gm >= lm) ? -1 : 0;
-            if (!__ballot(adj != 0)) break;
-            int64_t carry = 0;
-#pragma unroll
-            for (uint32_t u = 0; u < 4; ++u) {
-                carry += int64_t(w[u]) + (adj > 0 ? int64_t(qv[u + 2]) : adj < 0 ? -int64_t(qv[u + 2]) : 0);
-                w[u] = uint32_t(uint64_t(carry));
-                carry >>= 32;
-            }
-            settle(w, int32_t(carry), top);
-        }
+        int64_t d[4];
+        lw.sums(sums + cl * S, L, d);
+        lw.reconstruct(d, quotient[cl], multiple[cl], i0 + cl < args.n, w);
         // c over the coefficient's own sums (its lanes have read them all)
         u32_alias* cw = reinterpret_cast<u32_alias*>(lds + size_t(cl) * S * 8);
 #pragma unroll
         for (uint32_t u = 0; u < 4; ++u)
-            if (j0 + u < L) cw[j0 + u] = w[u];
+            if (4 * g + u < L) cw[4 * g + u] = w[u];
     }
     __syncthreads();
     const uint32_t rows = i0 < args.n ? (args.n - i0 < T ? args.n - i0 : T) : 0;
@@ -1809,6 +1919,20 @@ __global__ __launch_bounds__(256, 4) void crt_reconstruct_group(GroupLaunch g) {
         case 2: residues(std::integral_constant<int, 2>()); break;
         default: residues(std::integral_constant<int, 4>()); break;
     }
+}
+
+__global__ __launch_bounds__(256) void reconstruct_wide_group(GroupLaunch g) {
+    uint32_t local;
+    const GroupView& it = group_entry(g, local);
+    const WaveReconstructArgs args{it.n, it.ws, it.limbs, it.t_words, every_tile(it),
+                                   it.top_m, it.top_e, it.k_shift, it.mu};
+    auto run = [&](auto lanes, auto passes) {
+        reconstruct_wide_body<lanes(), passes()>(in_global(it.words), in_global(it.c), in_global(it.q),
+                                                 in_global(it.neg_p), in_global(it.corr_t), in_global(it.corr_e), args,
+                                                 local);
+    };
+    if (it.crt_words <= 128) run(std::integral_constant<int, 32>(), std::integral_constant<int, 2>());
+    else run(std::integral_constant<int, 64>(), std::integral_constant<int, 4>());
 }
 
 __global__ __launch_bounds__(256) void reconstruct_waves_group(GroupLaunch g) {
@@ -2264,9 +2388,19 @@ void launch_reconstruct(const Shape& s, const DeviceTables& t, const int64_t* wo
     const uint32_t top_m = barrett_top(s);
     WaveReconstructArgs args{s.n, word_stride(s), s.limbs, s.t_words, ts,
                              top_m, s.s_shift - 32 * top_m, s.k_shift, s.mu};
-    hipLaunchKernelGGL(reconstruct_waves, dim3(ts.count * 64), dim3(256), 0, stream, words, c, t.q, t.neg_p,
-                       t.corr_t, t.corr_e, args);
-    check_launch("reconstruct_waves");
+#define PM_WIDE(G, NP)                                                                                              \
+    hipLaunchKernelGGL((reconstruct_wide<G, NP>), dim3(ts.count * (kTile / (256 / G * NP))), dim3(256), 0, stream,   \
+                       words, c, t.q, t.neg_p, t.corr_t, t.corr_e, args)
+    // Few coefficients leave the GPU idle either way, and a wave each is the
+    // shorter path: N = 128 with 128 limbs 4.1 us against 6.4.
+    const bool few = ts.count <= 8;
+    if (s.crt_words <= 128 && !few) PM_WIDE(32, 2);
+    else if (s.crt_words <= kWideWords && !few) PM_WIDE(64, 4);
+#undef PM_WIDE
+    else
+        hipLaunchKernelGGL(reconstruct_waves, dim3(ts.count * 64), dim3(256), 0, stream, words, c, t.q, t.neg_p,
+                           t.corr_t, t.corr_e, args);
+    check_launch("reconstruct");
 }
 
 GroupItem group_item(const Shape& s, const DeviceTables& t, const DeviceWork& w, const uint32_t* a,
@@ -2301,10 +2435,10 @@ namespace {
 // Launches of one batch: conversion from the limbs, pack, conversion GEMM,
 // forward columns (four row-count classes), rows (one per row width and block
 // size n1, and the LDS kernel), inverse columns (four classes), CRT GEMM with
-// reconstruction, CRT GEMM, reconstruction.
-constexpr size_t kGroupLaunches = 1 + 2 + 4 + 21 + 4 + 1 + 2;
+// reconstruction, CRT GEMM, reconstruction (two kernels).
+constexpr size_t kGroupLaunches = 1 + 2 + 4 + 21 + 4 + 1 + 3;
 
-enum GroupKind { kConvert, kPack, kConversion, kForward, kRowsReg, kRowsProduct, kInverse, kCrtRec, kCrt, kRecWave };
+enum GroupKind { kConvert, kPack, kConversion, kForward, kRowsReg, kRowsProduct, kInverse, kCrtRec, kCrt, kRecWide, kRecWave };
 
 size_t group_item_bytes(size_t count) { return (count * sizeof(GroupItem) + 255) / 256 * 256; }
 size_t group_table_words(size_t count) { return kGroupLaunches * (2 * count + 1); }
@@ -2391,7 +2525,10 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
     add(kCrt, 0, [&](const GroupItem& it) {
         return it.crt_words <= kFusedWords ? 0 : uint64_t(it.crt_rows / kTile) * ntiles(it);
     });
-    add(kRecWave, 0, [&](const GroupItem& it) { return it.crt_words <= kFusedWords ? 0 : 64 * ntiles(it); });
+    add(kRecWide, 0, [&](const GroupItem& it) {
+        return it.crt_words > kFusedWords && it.crt_words <= kWideWords ? 16 * ntiles(it) : 0;
+    });
+    add(kRecWave, 0, [&](const GroupItem& it) { return it.crt_words > kWideWords ? 64 * ntiles(it) : 0; });
     // the items and the work lists, one copy
     std::vector<char> upload(item_bytes + used * sizeof(uint32_t));
     std::memcpy(upload.data(), items.data(), count * sizeof(GroupItem));
@@ -2446,6 +2583,9 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
                 break;
             case kCrt:
                 hipLaunchKernelGGL(crt_group, grid, dim3(kGemmThreads), 0, stream, g);
+                break;
+            case kRecWide:
+                hipLaunchKernelGGL(reconstruct_wide_group, grid, dim3(256), 0, stream, g);
                 break;
             case kRecWave:
                 hipLaunchKernelGGL(reconstruct_waves_group, grid, dim3(256), 0, stream, g);
