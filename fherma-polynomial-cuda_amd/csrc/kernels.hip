@@ -43,16 +43,15 @@ typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 typedef uint32_t v2u __attribute__((ext_vector_type(2)));
 typedef uint32_t u32_alias __attribute__((may_alias));
 
-// GEMM block tile: 256 weight rows x 256 coefficients x 64 bytes of K, eight
-// waves in a 4x2 grid, each owning a 64x128 slab = 4x8 MFMA 16x16 tiles
-// (128 int32 accumulators per lane; two waves per SIMD).
+// GEMM block tile: 256 weight rows x 128 WN coefficients x 64 bytes of K, 4 x WN
+// waves, each owning a 64x128 slab = 4x8 MFMA 16x16 tiles (128 int32
+// accumulators per lane; two waves per SIMD).  WN is 2, or 1 where whole tiles
+// would leave CUs without a block (gemm_halves).
 constexpr uint32_t kTile = 256;
 constexpr uint32_t kTK = 64;
 constexpr uint32_t kTileBytes = kTile * kTK;  // one operand K step, 16 KB
-constexpr uint32_t kGemmThreads = 512;
-constexpr uint32_t kLoads = kTileBytes / 16 / kGemmThreads;  // 16-byte loads per thread per operand
+constexpr uint32_t kLoads = 2;                // 16-byte loads of B per thread and K step
 constexpr uint32_t kWaveM = 4, kWaveN = 8;    // 16x16 tiles per wave
-constexpr uint32_t kWavesN = 2;               // waves across the coefficient dimension
 constexpr uint32_t kWaveRows = kWaveM * 16, kWaveCols = kWaveN * 16;
 constexpr uint32_t kGroupM = 8;               // raster group height (tiles)
 
@@ -188,17 +187,18 @@ struct GemmStages {
     int8_t* s[4];
 };
 
+template <uint32_t WN>
 __device__ __forceinline__ void gemm_mainloop(const int8_t* __restrict__ a_panel, const int8_t* __restrict__ b_panel,
                                               uint32_t ksteps, const GemmStages& st, v4i (&acc)[kWaveM][kWaveN]) {
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t wm = wave / kWavesN, wn = wave % kWavesN;
+    const uint32_t wm = wave / WN, wn = wave % WN;
     const v4i* ap = reinterpret_cast<const v4i*>(a_panel + (wm * kWaveRows + (lane & 15)) * kTK + (lane >> 4) * 16);
-    // B: slot s = tid + 512 j of a stage holds row s>>2, swizzled chunk s&3,
+    // B: slot s = tid + 256 WN j of a stage holds row s>>2, swizzled chunk s&3,
     // i.e. the row's chunk (s&3) ^ ((row>>1)&3) in the global tile.
     uint32_t boff[kLoads];
 #pragma unroll
     for (uint32_t j = 0; j < kLoads; ++j) {
-        const uint32_t slot = tid + kGemmThreads * j, row = slot >> 2, chunk = (slot & 3) ^ ((row >> 1) & 3);
+        const uint32_t slot = tid + 256 * WN * j, row = slot >> 2, chunk = (slot & 3) ^ ((row >> 1) & 3);
         boff[j] = row * kTK + chunk * 16;
     }
     auto clamp = [&](uint32_t k) { return k < ksteps ? k : ksteps - 1; };  // past the end: repeat the last step
@@ -207,7 +207,7 @@ __device__ __forceinline__ void gemm_mainloop(const int8_t* __restrict__ a_panel
 #pragma unroll
         for (uint32_t j = 0; j < kLoads; ++j)
             __builtin_amdgcn_global_load_lds(reinterpret_cast<const void*>(src + boff[j]),
-                                             (__attribute__((address_space(3))) void*)(stage + (wave * 64 + kGemmThreads * j) * 16),
+                                             (__attribute__((address_space(3))) void*)(stage + (wave * 64 + 256 * WN * j) * 16),
                                              16, 0, 0);
     };
     auto load_a = [&](uint32_t ks, v4i (&fa)[kWaveM]) {
@@ -253,11 +253,11 @@ __device__ __forceinline__ void gemm_mainloop(const int8_t* __restrict__ a_panel
     __builtin_amdgcn_s_waitcnt((0x7 << 4) | (0xF << 8));  // vmcnt 0
 }
 
-// The four 16 KB LDS stages of gemm_mainloop, as separate arrays of the kernel
+// The four LDS stages of gemm_mainloop (8 KB times WN), as separate arrays of the kernel
 // (so the compiler can tell a stage being filled from the one being read).
 #define PM_GEMM_STAGES(name)                                                                               \
-    __shared__ __attribute__((aligned(16))) int8_t name##0[kTileBytes], name##1[kTileBytes],                \
-        name##2[kTileBytes], name##3[kTileBytes];                                                          \
+    __shared__ __attribute__((aligned(16))) int8_t name##0[kTileBytes / 2 * WN], name##1[kTileBytes / 2 * WN], \
+        name##2[kTileBytes / 2 * WN], name##3[kTileBytes / 2 * WN];                                            \
     const GemmStages name{{name##0, name##1, name##2, name##3}}
 
 // ---------------------------------------------------------------------------
@@ -328,6 +328,7 @@ __global__ __launch_bounds__(256) void pack_operands(const uint32_t* __restrict_
 // 1. conversion GEMM: G[4k+d][i] = sum_j digit_d(lambda*256^j mod p_k) * (byte_j(x_i)-128)
 //    then x_i*lambda mod p_k = REDC(sum_d 256^d G[4k+d][i] + off_k).
 // ---------------------------------------------------------------------------
+template <uint32_t WN>
 __device__ __forceinline__ void conversion_body(const int8_t* __restrict__ wtiles, const int8_t* __restrict__ packed,
                                                 const PrimeConst* __restrict__ consts, uint32_t* __restrict__ planes,
                                                 uint32_t n, uint32_t n_pad, uint32_t r, uint32_t r_pad,
@@ -335,20 +336,23 @@ __device__ __forceinline__ void conversion_body(const int8_t* __restrict__ wtile
                                                 uint32_t nops, uint32_t bid) {
     PM_GEMM_STAGES(stages);
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint32_t wm = wave / kWavesN, wn = wave % kWavesN;
+    const uint32_t wm = wave / WN, wn = wave % WN;
     const uint32_t ntiles = n_pad / kTile, num_m = conv_rows / kTile;
     uint32_t tm, tn;
-    tile_coords(bid, num_m, nops * ts.count, tm, tn);  // the set's coefficient tiles of nops operands
+    constexpr uint32_t kParts = 2 / WN;
+    tile_coords(bid, num_m, nops * ts.count * kParts, tm, tn);  // the set's coefficient tiles of nops operands
+    const uint32_t part = tn % kParts;                          // of the 256-coefficient tile
+    tn /= kParts;
     const uint32_t op = op0 + tn / ts.count, tcol = tile_at(ts, tn % ts.count);
     const int8_t* a_panel = wtiles + (size_t(op) * num_m + tm) * ksteps * kTileBytes;
-    const int8_t* b_panel = packed + (size_t(op) * ntiles + tcol) * ksteps * kTileBytes;
+    const int8_t* b_panel = packed + (size_t(op) * ntiles + tcol) * ksteps * kTileBytes + part * (kTileBytes / 2);
 
     v4i acc[kWaveM][kWaveN];
 #pragma unroll
     for (uint32_t mi = 0; mi < kWaveM; ++mi)
 #pragma unroll
         for (uint32_t ni = 0; ni < kWaveN; ++ni) acc[mi][ni] = v4i{0, 0, 0, 0};
-    gemm_mainloop(a_panel, b_panel, ksteps, stages, acc);
+    gemm_mainloop<WN>(a_panel, b_panel, ksteps, stages, acc);
 
     // Lane holds rows 4*(lane/16)+j (j = digit) of each 16-row tile: one prime.
     // The digit sum is sum_j c_j*(byte_j - 128) with |c_j| <= p/2 over 4L bytes,
@@ -357,7 +361,7 @@ __device__ __forceinline__ void conversion_body(const int8_t* __restrict__ wtile
     // Plans allow at most 16383 primes of < 32 bits covering (q-1)^2, so
     // q < 2^262144 and L <= 8192: 256*L <= 2^21.
     const DigitScales ds = digit_scales();
-    const uint32_t m0 = tm * kTile + wm * kWaveRows, c0 = tcol * kTile + wn * kWaveCols;
+    const uint32_t m0 = tm * kTile + wm * kWaveRows, c0 = tcol * kTile + (part + wn) * kWaveCols;
 #pragma unroll
     for (uint32_t mi = 0; mi < kWaveM; ++mi) {
         const uint32_t kp = (m0 + mi * 16) / 4 + (lane >> 4);
@@ -373,13 +377,14 @@ __device__ __forceinline__ void conversion_body(const int8_t* __restrict__ wtile
     }
 }
 
-__global__ __launch_bounds__(512) void conversion_gemm(const int8_t* __restrict__ wtiles,
+template <uint32_t WN>
+__global__ __launch_bounds__(256 * WN, 2) void conversion_gemm(const int8_t* __restrict__ wtiles,
                                                        const int8_t* __restrict__ packed,
                                                        const PrimeConst* __restrict__ consts,
                                                        uint32_t* __restrict__ planes, uint32_t n, uint32_t n_pad,
                                                        uint32_t r, uint32_t r_pad, uint32_t conv_rows,
                                                        uint32_t ksteps, TileSet ts, uint32_t op0, uint32_t nops) {
-    conversion_body(wtiles, packed, consts, planes, n, n_pad, r, r_pad, conv_rows, ksteps, ts, op0, nops, blockIdx.x);
+    conversion_body<WN>(wtiles, packed, consts, planes, n, n_pad, r, r_pad, conv_rows, ksteps, ts, op0, nops, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -532,29 +537,32 @@ __global__ __launch_bounds__(256, 3) void convert(const uint32_t* __restrict__ a
 //    words of 16 coefficients are 128-byte runs per coefficient, written one
 //    after another.
 // ---------------------------------------------------------------------------
+template <uint32_t WN>
 __device__ __forceinline__ void crt_body(const int8_t* __restrict__ wtiles, const int8_t* __restrict__ rtiles,
                                          int64_t* __restrict__ words, uint32_t n, uint32_t n_pad, uint32_t crt_rows,
-                                         uint32_t ksteps, uint32_t crt_words, uint32_t ws, TileSet ts,
-                                         uint32_t bid) {
+                                         uint32_t kstride, uint32_t ksteps, uint32_t crt_words, uint32_t ws,
+                                         TileSet ts, uint32_t bid) {
     PM_GEMM_STAGES(stages);
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint32_t wm = wave / kWavesN, wn = wave % kWavesN;
+    const uint32_t wm = wave / WN, wn = wave % WN;
     const uint32_t num_m = crt_rows / kTile;
     uint32_t tm, tn;
-    tile_coords(bid, num_m, ts.count, tm, tn);  // the set's coefficient tiles
-    tn = tile_at(ts, tn);
-    const int8_t* a_panel = wtiles + size_t(tm) * ksteps * kTileBytes;
-    const int8_t* b_panel = rtiles + size_t(tn) * ksteps * kTileBytes;
+    constexpr uint32_t kParts = 2 / WN;
+    tile_coords(bid, num_m, ts.count * kParts, tm, tn);  // the set's coefficient tiles
+    const uint32_t part = tn % kParts;                   // of the 256-coefficient tile
+    tn = tile_at(ts, tn / kParts);
+    const int8_t* a_panel = wtiles + size_t(tm) * kstride * kTileBytes;
+    const int8_t* b_panel = rtiles + size_t(tn) * kstride * kTileBytes + part * (kTileBytes / 2);
 
     v4i acc[kWaveM][kWaveN];
 #pragma unroll
     for (uint32_t mi = 0; mi < kWaveM; ++mi)
 #pragma unroll
         for (uint32_t ni = 0; ni < kWaveN; ++ni) acc[mi][ni] = v4i{0, 0, 0, 0};
-    gemm_mainloop(a_panel, b_panel, ksteps, stages, acc);
+    gemm_mainloop<WN>(a_panel, b_panel, ksteps, stages, acc);
 
     const DigitScales ds = digit_scales();
-    const uint32_t m0 = tm * kTile + wm * kWaveRows, c0 = tn * kTile + wn * kWaveCols;
+    const uint32_t m0 = tm * kTile + wm * kWaveRows, c0 = tn * kTile + (part + wn) * kWaveCols;
 #pragma unroll
     for (uint32_t ni = 0; ni < kWaveN; ++ni) {
         const uint32_t coef = c0 + ni * 16 + (lane & 15);
@@ -567,12 +575,94 @@ __device__ __forceinline__ void crt_body(const int8_t* __restrict__ wtiles, cons
     }
 }
 
-__global__ __launch_bounds__(512) void crt_gemm(const int8_t* __restrict__ wtiles,
+template <uint32_t WN>
+__global__ __launch_bounds__(256 * WN, 2) void crt_gemm(const int8_t* __restrict__ wtiles,
                                                 const int8_t* __restrict__ rtiles,
                                                 int64_t* __restrict__ words, uint32_t n, uint32_t n_pad,
-                                                uint32_t crt_rows, uint32_t ksteps, uint32_t crt_words,
-                                                uint32_t ws, TileSet ts) {
-    crt_body(wtiles, rtiles, words, n, n_pad, crt_rows, ksteps, crt_words, ws, ts, blockIdx.x);
+                                                uint32_t crt_rows, uint32_t kstride, uint32_t ksteps,
+                                                uint32_t crt_words, uint32_t ws, TileSet ts) {
+    crt_body<WN>(wtiles, rtiles, words, n, n_pad, crt_rows, kstride, ksteps, crt_words, ws, ts, blockIdx.x);
+}
+
+// ---------------------------------------------------------------------------
+// 5'. CRT GEMM for few coefficients: blocks of 64 weight rows (16 word sums) x
+// 64 coefficients, whose four waves each take every fourth K step, so that even
+// one tile's K loop is spread over a CU.  Both operands are read as MFMA
+// fragments straight from their tiles, two steps ahead, with no barrier until
+// the waves' sums meet in LDS; each wave then finishes a quarter of them.
+// Consecutive tiles of one XCD share their coefficients.  crt_gemm's three
+// blocks took 18.7 us at N = 128 with 128 limbs, this 6.4.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ void crt_small_body(const int8_t* __restrict__ wtiles, const int8_t* __restrict__ rtiles,
+                                               int64_t* __restrict__ words, uint32_t n, uint32_t kstride,
+                                               uint32_t ksteps, uint32_t crt_words, uint32_t ws, const TileSet& ts,
+                                               uint32_t bid) {
+    constexpr uint32_t NT = 4, T = 16 * NT;
+    __shared__ v4i part[4][3][NT][64];  // [wave that finishes][wave that summed][fragment][lane]
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t num_m = (crt_words + 15) / 16, total = num_m * ts.count * (kTile / T), per = total / 8;
+    const uint32_t logical = bid < per * 8 ? (bid % 8) * per + bid / 8 : bid;
+    const uint32_t m = logical % num_m, k0 = logical / num_m * T;
+    const uint32_t tile = tile_at(ts, k0 / kTile), i0 = tile * kTile + k0 % kTile;
+    if (i0 >= n) return;  // whole block
+    const uint32_t frag = (lane & 15) * kTK + (lane >> 4) * 16;
+    const v4i* ap = reinterpret_cast<const v4i*>(wtiles + size_t(m / 4) * kstride * kTileBytes + m % 4 * (kWaveRows * kTK) + frag);
+    const v4i* bp = reinterpret_cast<const v4i*>(rtiles + size_t(tile) * kstride * kTileBytes + k0 % kTile * kTK + frag);
+    v4i acc[kWaveM][NT], fa[2][kWaveM], fb[2][NT];
+#pragma unroll
+    for (uint32_t mi = 0; mi < kWaveM; ++mi)
+#pragma unroll
+        for (uint32_t ni = 0; ni < NT; ++ni) acc[mi][ni] = v4i{0, 0, 0, 0};
+    auto load = [&](uint32_t ks, v4i (&a)[kWaveM], v4i (&b)[NT]) {
+#pragma unroll
+        for (uint32_t mi = 0; mi < kWaveM; ++mi) a[mi] = ap[size_t(ks) * (kTileBytes / 16) + mi * 64];
+#pragma unroll
+        for (uint32_t ni = 0; ni < NT; ++ni) b[ni] = bp[size_t(ks) * (kTileBytes / 16) + ni * 64];
+    };
+    auto step = [&](const v4i (&a)[kWaveM], const v4i (&b)[NT]) {
+#pragma unroll
+        for (uint32_t mi = 0; mi < kWaveM; ++mi)
+#pragma unroll
+            for (uint32_t ni = 0; ni < NT; ++ni)
+                acc[mi][ni] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[mi], b[ni], acc[mi][ni], 0, 0, 0);
+    };
+    uint32_t ks = wave;
+    if (ks < ksteps) load(ks, fa[0], fb[0]);
+    if (ks + 4 < ksteps) load(ks + 4, fa[1], fb[1]);
+    for (; ks + 12 < ksteps; ks += 8) {
+        step(fa[0], fb[0]);
+        load(ks + 8, fa[0], fb[0]);
+        step(fa[1], fb[1]);
+        load(ks + 12, fa[1], fb[1]);
+    }
+    if (ks < ksteps) step(fa[0], fb[0]);
+    if (ks + 8 < ksteps) load(ks + 8, fa[0], fb[0]);
+    if (ks + 4 < ksteps) step(fa[1], fb[1]);
+    if (ks + 8 < ksteps) step(fa[0], fb[0]);
+    // wave w finishes row fragment mi = w
+#pragma unroll
+    for (uint32_t mi = 0; mi < kWaveM; ++mi)
+        if (mi != wave)
+#pragma unroll
+            for (uint32_t ni = 0; ni < NT; ++ni) part[mi][wave > mi ? wave - 1 : wave][ni][lane] = acc[mi][ni];
+    __syncthreads();
+    const DigitScales ds = digit_scales();
+    const uint32_t word = m * 16 + wave * 4 + (lane >> 4);
+#pragma unroll
+    for (uint32_t ni = 0; ni < NT; ++ni) {
+        v4i sum = wave == 0 ? acc[0][ni] : wave == 1 ? acc[1][ni] : wave == 2 ? acc[2][ni] : acc[3][ni];
+#pragma unroll
+        for (uint32_t w = 0; w < 3; ++w) sum += part[wave][w][ni][lane];
+        const uint32_t coef = i0 + ni * 16 + (lane & 15);
+        if (word < crt_words && coef < n) words[size_t(coef) * ws + word] = combine4(sum, ds);
+    }
+}
+
+__global__ __launch_bounds__(256, 3) void crt_small(const int8_t* __restrict__ wtiles,
+                                                    const int8_t* __restrict__ rtiles, int64_t* __restrict__ words,
+                                                    uint32_t n, uint32_t kstride, uint32_t ksteps,
+                                                    uint32_t crt_words, uint32_t ws, TileSet ts) {
+    crt_small_body(wtiles, rtiles, words, n, kstride, ksteps, crt_words, ws, ts, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -1810,7 +1900,7 @@ __global__ __launch_bounds__(256) void pack_group(GroupLaunch g) {
 __global__ __launch_bounds__(512) void conversion_group(GroupLaunch g) {
     uint32_t local;
     const GroupView& it = group_entry(g, local);
-    conversion_body(in_global(it.wconv), in_global(it.packed), in_global(it.consts), in_global(it.planes), it.n, it.n_pad, it.r, it.r_pad, it.conv_rows,
+    conversion_body<2>(in_global(it.wconv), in_global(it.packed), in_global(it.consts), in_global(it.planes), it.n, it.n_pad, it.r, it.r_pad, it.conv_rows,
                     it.conv_k / kTK, every_tile(it), 0, 2, local);
 }
 
@@ -1895,8 +1985,8 @@ __global__ __launch_bounds__(256) void inverse_tiles_group(GroupLaunch g) {
 __global__ __launch_bounds__(512) void crt_group(GroupLaunch g) {
     uint32_t local;
     const GroupView& it = group_entry(g, local);
-    crt_body(in_global(it.wcrt), in_global(it.rtiles), in_global(it.words), it.n, it.n_pad, it.crt_rows, it.crt_k / kTK, it.crt_words, it.ws,
-             every_tile(it), local);
+    crt_body<2>(in_global(it.wcrt), in_global(it.rtiles), in_global(it.words), it.n, it.n_pad, it.crt_rows,
+                it.crt_k / kTK, (it.r + 15) / 16, it.crt_words, it.ws, every_tile(it), local);
 }
 
 __global__ __launch_bounds__(256, 4) void crt_reconstruct_group(GroupLaunch g) {
@@ -2184,12 +2274,30 @@ void launch_pack(const Shape& s, const uint32_t* a, const uint32_t* b, int8_t* p
     check_launch("pack_operands");
 }
 
+namespace {
+
+// Whether a GEMM of `blocks` whole tiles takes halves (WN = 1).  A CU holds one
+// whole tile's block, or two halves, at a time; halves pay when they spread what
+// is left for the last round (up to 128 tiles on 256 CUs) over twice the CUs.
+// CRT GEMM, whole against halves: 128 tiles 31.7 / 22.1 us (N = 8192, 226
+// limbs), 80 tiles 62 / 42, 112 tiles 177 / 117 (N = 1024, 1747 limbs), but 224
+// tiles 202 / 219 and 256 tiles 36.2 / 37.5; conversion GEMM 336 tiles 66 / 55,
+// 456 tiles 190 / 195, 512 tiles 36.1 / 35.2.  With two full rounds and more the
+// last one matters less than the halves' extra weight traffic.
+bool gemm_halves(uint64_t blocks) { return blocks < 512 && (blocks - 1) % 256 < 128; }
+
+}  // namespace
+
 void launch_conversion(const Shape& s, const DeviceTables& t, const int8_t* packed, uint32_t* planes,
                        const TileSet& ts, uint32_t op0, uint32_t nops, hipStream_t stream) {
     check_tiles(s, ts, "conversion_gemm");
     const uint32_t blocks = (s.conv_rows / kTile) * nops * ts.count;
-    hipLaunchKernelGGL(conversion_gemm, dim3(blocks), dim3(kGemmThreads), 0, stream, t.wconv, packed,
-                       t.consts, planes, s.n, s.n_pad, s.r, s.r_pad, s.conv_rows, s.conv_k / kTK, ts, op0, nops);
+    if (gemm_halves(blocks))
+        hipLaunchKernelGGL(conversion_gemm<1>, dim3(2 * blocks), dim3(256), 0, stream, t.wconv, packed, t.consts,
+                           planes, s.n, s.n_pad, s.r, s.r_pad, s.conv_rows, s.conv_k / kTK, ts, op0, nops);
+    else
+        hipLaunchKernelGGL(conversion_gemm<2>, dim3(blocks), dim3(512), 0, stream, t.wconv, packed, t.consts, planes,
+                           s.n, s.n_pad, s.r, s.r_pad, s.conv_rows, s.conv_k / kTK, ts, op0, nops);
     check_launch("conversion_gemm");
 }
 
@@ -2334,12 +2442,34 @@ void launch_ntt_inverse_columns(const Shape& s, const DeviceTables& t, uint32_t*
     check_launch("ntt_columns_inverse_tiles");
 }
 
+namespace {
+
+// Whether the CRT GEMM has so few whole tiles that crt_small takes it.  Against
+// halves: 3 tiles 6.4 / 13 us (N = 128, 128 limbs), 8 tiles 12.9 / 30.3 (N =
+// 128, 500 limbs), 32 tiles 13.9 / 18.4 (N = 2048, 226 limbs), 28 tiles 68 / 98
+// (N = 128, 1747 limbs); 80 tiles 63.6 / 41.8, where every wave reading its own
+// operands from L2 starts to bound it.
+bool crt_few_blocks(uint32_t crt_rows, uint32_t tiles) { return crt_rows / kTile * tiles < 48; }
+
+}  // namespace
+
 void launch_crt(const Shape& s, const DeviceTables& t, const int8_t* rtiles, int64_t* words, const TileSet& ts,
                 hipStream_t stream) {
     check_tiles(s, ts, "crt_gemm");
+    if (crt_few_blocks(s.crt_rows, ts.count)) {
+        const dim3 grid((s.crt_words + 15) / 16 * ts.count * 4);
+        hipLaunchKernelGGL(crt_small, grid, dim3(256), 0, stream, t.wcrt, rtiles, words, s.n, s.crt_k / kTK,
+                           (s.r + 15) / 16, s.crt_words, word_stride(s), ts);
+        check_launch("crt_small");
+        return;
+    }
     const uint32_t blocks = (s.crt_rows / kTile) * ts.count;
-    hipLaunchKernelGGL(crt_gemm, dim3(blocks), dim3(kGemmThreads), 0, stream, t.wcrt, rtiles, words, s.n, s.n_pad,
-                       s.crt_rows, s.crt_k / kTK, s.crt_words, word_stride(s), ts);
+    if (gemm_halves(blocks))
+        hipLaunchKernelGGL(crt_gemm<1>, dim3(2 * blocks), dim3(256), 0, stream, t.wcrt, rtiles, words, s.n, s.n_pad,
+                           s.crt_rows, s.crt_k / kTK, (s.r + 15) / 16, s.crt_words, word_stride(s), ts);
+    else
+        hipLaunchKernelGGL(crt_gemm<2>, dim3(blocks), dim3(512), 0, stream, t.wcrt, rtiles, words, s.n, s.n_pad,
+                           s.crt_rows, s.crt_k / kTK, (s.r + 15) / 16, s.crt_words, word_stride(s), ts);
     check_launch("crt_gemm");
 }
 
@@ -2436,7 +2566,7 @@ namespace {
 // forward columns (four row-count classes), rows (one per row width and block
 // size n1, and the LDS kernel), inverse columns (four classes), CRT GEMM with
 // reconstruction, CRT GEMM, reconstruction (two kernels).
-constexpr size_t kGroupLaunches = 1 + 2 + 4 + 21 + 4 + 1 + 3;
+constexpr size_t kGroupLaunches = 1 + 2 + 4 + 21 + 4 + 1 + 1 + 2;
 
 enum GroupKind { kConvert, kPack, kConversion, kForward, kRowsReg, kRowsProduct, kInverse, kCrtRec, kCrt, kRecWide, kRecWave };
 
@@ -2522,7 +2652,7 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
             return row_kernel(it) == R && !skip ? uint64_t(it.row_width / 16) * (it.r_pad / 16) : 0;
         });
     add(kCrtRec, 0, [&](const GroupItem& it) { return it.crt_words <= kFusedWords ? 4 * ntiles(it) : 0; });
-    add(kCrt, 0, [&](const GroupItem& it) {
+    add(kCrt, 0, [&](const GroupItem& it) {  // whole tiles: the batch's products fill the GPU together
         return it.crt_words <= kFusedWords ? 0 : uint64_t(it.crt_rows / kTile) * ntiles(it);
     });
     add(kRecWide, 0, [&](const GroupItem& it) {
@@ -2546,7 +2676,7 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
                 hipLaunchKernelGGL(pack_group, grid, dim3(256), 0, stream, g);
                 break;
             case kConversion:
-                hipLaunchKernelGGL(conversion_group, grid, dim3(kGemmThreads), 0, stream, g);
+                hipLaunchKernelGGL(conversion_group, grid, dim3(512), 0, stream, g);
                 break;
             case kForward:
                 switch (L.variant) {
@@ -2582,7 +2712,7 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
                 hipLaunchKernelGGL(crt_reconstruct_group, grid, dim3(256), L.lds, stream, g);
                 break;
             case kCrt:
-                hipLaunchKernelGGL(crt_group, grid, dim3(kGemmThreads), 0, stream, g);
+                hipLaunchKernelGGL(crt_group, grid, dim3(512), 0, stream, g);
                 break;
             case kRecWide:
                 hipLaunchKernelGGL(reconstruct_wide_group, grid, dim3(256), 0, stream, g);
