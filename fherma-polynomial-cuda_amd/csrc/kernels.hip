@@ -416,7 +416,9 @@ __global__ __launch_bounds__(256 * WN, 2) void conversion_gemm(const int8_t* __r
 // 14.7 + 36.5): the 29 MB of limbs read and 60 MB of residues written, about
 // 18 us at a large copy's rate, with the MFMAs (7 us) and the reductions (5 us)
 // beside them.  At N = 131072 with 4 limbs 11.1 against 18.4 + 21.2 us, at
-// N = 128 with 128 limbs 4.8 against 2.9 + 12.0.  (Operand bytes in LDS and
+// N = 128 with 128 limbs 4.8 against 2.9 + 12.0, at N = 8192 with 226 41.8
+// against 7.9 + 37.5, at N = 65536 with 226 339 against 47 + 319.  Beyond 256
+// limbs a wave's registers hold too few coefficients to feed the MFMAs from LDS.  (Operand bytes in LDS and
 // weights straight from L2, one barrier per block: 37 us at N = 65536; the
 // weight fragments then come from L2 once per wave.)
 // ---------------------------------------------------------------------------
@@ -428,7 +430,10 @@ struct ConvertArgs {
     uint32_t op0;
 };
 
-constexpr uint32_t convert_stage_chunks(uint32_t ksteps) { return kConvertStage / (ksteps * kWaveRows * kTK); }
+constexpr uint32_t convert_stage_chunks(uint32_t ksteps) {
+    const uint32_t chunk = ksteps * kWaveRows * kTK;
+    return chunk < kConvertStage ? kConvertStage / chunk : 1;
+}
 
 // The staged weights, then the primes' constants.
 constexpr size_t convert_lds_bytes(uint32_t ksteps, uint32_t r) {
@@ -532,7 +537,7 @@ __device__ __forceinline__ void convert_body(const uint32_t* __restrict__ a, con
 }
 
 template <int KS, int NT>
-__global__ __launch_bounds__(256, 3) void convert(const uint32_t* __restrict__ a, const uint32_t* __restrict__ b,
+__global__ __launch_bounds__(256, KS * NT > 16 ? 2 : 3) void convert(const uint32_t* __restrict__ a, const uint32_t* __restrict__ b,
                                                   const int8_t* __restrict__ wtiles,
                                                   const PrimeConst* __restrict__ consts,
                                                   uint32_t* __restrict__ planes, ConvertArgs args) {
@@ -2319,6 +2324,9 @@ struct ConvertPlan {
     uint32_t ks, nt, split;
 };
 constexpr uint32_t kConvertBlocks = 512, kConvertGroupBlocks = 64;  // two per CU; a batch's share
+// Up to here a batch's products take the short conversion: 16 K steps in
+// registers would cost the shared kernel a third of its occupancy.
+constexpr uint32_t kGroupShortLimbs = 128;
 
 // `tiles` 256-coefficient tiles in all (of both operands).  Wide waves (NT 2 or
 // 4) read each weight from LDS for 32 or 64 coefficients; where they would
@@ -2330,8 +2338,8 @@ constexpr uint32_t kConvertBlocks = 512, kConvertGroupBlocks = 64;  // two per C
 // batch of 64 small products' conversions take 152 us in all, and 210 with each
 // product spread as if it were alone.
 ConvertPlan convert_plan(uint32_t r, uint32_t ksteps, uint32_t tiles, uint32_t want_blocks) {
-    const uint32_t chunks = (r + 15) / 16, ks = ksteps <= 1 ? 1 : ksteps <= 2 ? 2 : ksteps <= 4 ? 4 : 8;
-    uint32_t nt = ks == 8 ? 2 : 4;
+    const uint32_t chunks = (r + 15) / 16, ks = ksteps <= 1 ? 1 : ksteps <= 2 ? 2 : ksteps <= 4 ? 4 : ksteps <= 8 ? 8 : 16;
+    uint32_t nt = ks >= 8 ? 2 : 4;
     if (want_blocks == kConvertBlocks && tiles * (4 / nt) * chunks < want_blocks / 2) nt = 1;
     const uint32_t blocks = tiles * (4 / nt), want = (want_blocks + blocks - 1) / blocks;
     return ConvertPlan{ks, nt, chunks < want ? chunks : want};
@@ -2339,7 +2347,7 @@ ConvertPlan convert_plan(uint32_t r, uint32_t ksteps, uint32_t tiles, uint32_t w
 
 }  // namespace
 
-#define PM_CONVERT_VARIANTS(X) X(1, 1) X(2, 1) X(4, 1) X(8, 1) X(1, 4) X(2, 4) X(4, 4) X(8, 2)
+#define PM_CONVERT_VARIANTS(X) X(1, 1) X(2, 1) X(4, 1) X(8, 1) X(16, 1) X(1, 4) X(2, 4) X(4, 4) X(8, 2) X(16, 2)
 
 void launch_convert(const Shape& s, const DeviceTables& t, const uint32_t* a, const uint32_t* b, uint32_t* planes,
                     const TileSet& ts, uint32_t op0, uint32_t nops, hipStream_t stream) {
@@ -2632,13 +2640,13 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
     };
     auto ntiles = [](const GroupItem& it) { return uint64_t(it.n_pad / kTile); };
     add(kConvert, 0, [&](const GroupItem& it) {
-        return it.limbs <= kShortLimbs ? uint64_t(it.conv_split) * (8 / it.conv_nt) * ntiles(it) : 0;
+        return it.limbs <= kGroupShortLimbs ? uint64_t(it.conv_split) * (8 / it.conv_nt) * ntiles(it) : 0;
     });
     add(kPack, 0, [&](const GroupItem& it) {  // as launch_pack: 2 * ntiles * 256 rows
-        return it.limbs <= kShortLimbs ? 0 : 128 * ntiles(it) / pack_rows_per_wave(it.conv_k / kTK);
+        return it.limbs <= kGroupShortLimbs ? 0 : 128 * ntiles(it) / pack_rows_per_wave(it.conv_k / kTK);
     });
     add(kConversion, 0, [&](const GroupItem& it) {
-        return it.limbs <= kShortLimbs ? 0 : uint64_t(it.conv_rows / kTile) * 2 * ntiles(it);
+        return it.limbs <= kGroupShortLimbs ? 0 : uint64_t(it.conv_rows / kTile) * 2 * ntiles(it);
     });
     auto row_kernel = [](const GroupItem& it) { return it.rows < 8 ? 8 : it.rows; };
     for (uint32_t R = 8; R <= 64; R *= 2)

@@ -74,7 +74,7 @@ void launch_conversion(const Shape& s, const DeviceTables& t, const int8_t* pack
                        const TileSet& ts, uint32_t op0, uint32_t nops, hipStream_t stream);
 // Both of the above in one kernel that reads a and b itself (rows as launch_pack),
 // for q of up to kShortLimbs limbs.
-constexpr uint32_t kShortLimbs = 128;
+constexpr uint32_t kShortLimbs = 256;
 inline bool conversion_short(const Shape& s) { return s.limbs <= kShortLimbs; }
 void launch_convert(const Shape& s, const DeviceTables& t, const uint32_t* a, const uint32_t* b, uint32_t* planes,
                     const TileSet& ts, uint32_t op0, uint32_t nops, hipStream_t stream);

@@ -1,4 +1,4 @@
-"""The conversion that reads the limbs itself (q of up to 128 limbs) against the
+"""The conversion that reads the limbs itself (q of up to 256 limbs) against the
 oracle: residues exactly, for limb counts at the edges of its 64-byte K steps
 and of its range, N below, at and above a block, and prime counts of one, two
 and more 16-prime wave rows; then whole products, with enough coefficients for
@@ -16,7 +16,7 @@ def _case(workloads, n, limbs, seed):
     return q, workloads.uniform_below(q, n, rng), workloads.uniform_below(q, n, rng)
 
 
-@pytest.mark.parametrize("limbs", [1, 2, 7, 8, 15, 16, 17, 32, 33, 64, 127, 128, 129])
+@pytest.mark.parametrize("limbs", [1, 2, 7, 8, 15, 16, 17, 32, 33, 64, 127, 128, 129, 255, 256, 257])
 @pytest.mark.parametrize("n", [1, 64, 256])
 def test_residues(polymul, workloads, oracle, n, limbs):
     print("[gpu-case] short conversion residues", n, limbs, flush=True)
@@ -33,7 +33,8 @@ def test_residues(polymul, workloads, oracle, n, limbs):
         assert [int(v) for v in res[1, k]] == [beta[k] * x % p for x in bv], "beta*b mod p_%d" % k
 
 
-@pytest.mark.parametrize("n,limbs", [(16384, 3), (16384, 16), (32768, 30), (2048, 128), (16384, 129)])
+@pytest.mark.parametrize("n,limbs", [(16384, 3), (16384, 16), (32768, 30), (2048, 128), (16384, 129), (8192, 200),
+                                     (1024, 256), (1024, 257)])
 def test_products(polymul, workloads, oracle, device_memory, n, limbs):
     print("[gpu-case] short conversion products", n, limbs, flush=True)
     q, a, b = _case(workloads, n, limbs, 93000 + limbs)
