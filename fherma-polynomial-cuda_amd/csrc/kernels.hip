@@ -837,6 +837,8 @@ __global__ __launch_bounds__(256) void ntt_columns_inverse(uint32_t* __restrict_
 // ---------------------------------------------------------------------------
 // Register-resident NTT kernels for the usual shapes (rows <= 64, C = 2048).
 // ---------------------------------------------------------------------------
+constexpr uint32_t kRowWidth = 2048;  // C of every transform of more than one row
+
 // Cooley-Tukey: (a, b) -> (a + wb, a - wb).  a < p; b may be any 32-bit value
 // congruent to its residue.  With kReduce the outputs are below p; without,
 // below 2p, which is all the next level asks of the values it multiplies (b),
@@ -1671,6 +1673,12 @@ __global__ __launch_bounds__(256) void reconstruct_wide(const int64_t* __restric
 //    direct-to-LDS loads behind one barrier; the weights are read as MFMA
 //    fragments straight from global memory, two K steps ahead.  Only the K
 //    steps that hold primes run (the padded ones have zero weights).
+//    With up to 8 transform rows (ROWS > 0) there is no operand tile: the row
+//    stage's planes are read, the inverse column stages done in registers, one
+//    thread per (prime, column), and the residues written to LDS in its place
+//    (N = 16384 with 28 limbs: 9.2 us, where the inverse column kernel took 5.3
+//    and this one 6.6; a launch less).  Wider columns would need more
+//    coefficients per block than its accumulators hold.
 //  * The int64 word sums go to LDS, coefficient-major, over the operand bytes.
 //  * One lane per coefficient forms K and the Barrett estimate Qe, by the
 //    formulas of reconstruct_waves.
@@ -1691,7 +1699,7 @@ __global__ __launch_bounds__(256) void reconstruct_wide(const int64_t* __restric
 struct CrtFusedArgs {
     uint32_t n, limbs, t_words;
     uint32_t ksteps, kstride;  // K steps that hold primes; K steps of a residue tile
-    uint32_t r, ps;            // primes; plane row stride (residues read from the planes)
+    uint32_t r, ps, n2;        // primes; plane row stride, twiddles per prime (residues read from the planes)
     TileSet ts;                // output row k*256 + u is coefficient tile_at(ts, k)*256 + u
     uint32_t top_m, top_e, k_shift;
     uint64_t mu;
@@ -1707,10 +1715,12 @@ constexpr size_t fused_lds_bytes(uint32_t wm, uint32_t nw, uint32_t ksteps) {
     return operands > sums ? operands : sums;
 }
 
-template <int WM, int NW, bool kPlanes>
+template <int WM, int NW, int ROWS>
 __device__ __forceinline__ void crt_reconstruct_body(const int8_t* __restrict__ wtiles,
                                                      const int8_t* __restrict__ rtiles,
-                                                     const uint32_t* __restrict__ planes, uint32_t* __restrict__ c,
+                                                     const uint32_t* __restrict__ planes,
+                                                     const PrimeConst* __restrict__ consts,
+                                                     const uint2* __restrict__ twi, uint32_t* __restrict__ c,
                                                      const uint32_t* __restrict__ q,
                                                      const uint32_t* __restrict__ neg_p,
                                                      const uint32_t* __restrict__ corr_t,
@@ -1722,10 +1732,41 @@ __device__ __forceinline__ void crt_reconstruct_body(const int8_t* __restrict__ 
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t wm = wave % WM, wn = wave / WM;
     const uint32_t L = args.limbs, tw = args.t_words, ksteps = args.ksteps;
-    const uint32_t k0 = bx * T, tile = tile_at(args.ts, k0 / kTile), i0 = tile * kTile + k0 % kTile;
+    // The block's coefficients: 16 NW consecutive ones of the set, or (ROWS > 1)
+    // CW columns of the transform's [ROWS][2048] matrix, row after row.  Columns
+    // are 64 or 128 bytes wide: two blocks 8 ids apart, on one XCD, share the
+    // 128-byte lines (as in inverse_tiles_body).
+    constexpr uint32_t CW = ROWS > 1 ? T / ROWS : T;
+    const uint32_t cx = (bx & ~15u) | ((bx & 7u) << 1) | ((bx >> 3) & 1u);
+    const uint32_t k0 = ROWS > 1 ? cx * CW : bx * T;
+    const uint32_t tile = tile_at(args.ts, k0 / kTile), i0 = ROWS > 1 ? k0 : tile * kTile + k0 % kTile;
 
     // operand bytes, a row's chunk (16 bytes: four primes) swizzled as in swz
-    if constexpr (kPlanes) {  // thread -> coefficient tid % T, primes 4 (tid / T) .. + 3 of each K step
+    if constexpr (ROWS > 1) {
+        // inverse column stages: thread -> (prime, column), as inverse_tiles_body
+        for (uint32_t w = tid; w < ksteps * 16 * CW; w += NTH) {
+            const uint32_t k = w / CW, col = w % CW, kk = k < args.r ? k : args.r - 1;
+            const uint32_t p = consts[kk].p;
+            const uint32_t* src = planes + size_t(kk) * args.ps + k0 + col;
+            const uint2* tw = twi + size_t(kk) * args.n2;
+            uint32_t x[ROWS];
+#pragma unroll
+            for (int j = 0; j < ROWS; ++j) x[j] = src[j * kRowWidth];
+#pragma unroll
+            for (int m = ROWS / 2, half = 1; m >= 1; m /= 2, half *= 2)
+#pragma unroll
+                for (int g = 0; g < m; ++g) {
+                    const uint2 t = tw[m + g];
+#pragma unroll
+                    for (int jr = 0; jr < half; ++jr)
+                        gs_butterfly(x[2 * half * g + jr], x[2 * half * g + jr + half], t, p);
+                }
+#pragma unroll
+            for (int j = 0; j < ROWS; ++j)
+                *reinterpret_cast<u32_alias*>(lds + k / 16 * (T * kTK) + swz(j * CW + col, k % 16 / 4) + k % 4 * 4) =
+                    x[j] ^ 0x80808080u;
+        }
+    } else if constexpr (ROWS == 1) {  // thread -> coefficient tid % T, primes 4 (tid / T) .. + 3 of each K step
         const uint32_t cf = tid % T, chunk = tid / T;
         const uint32_t* src = planes + i0 + cf;
         for (uint32_t ks = 0; ks < ksteps; ++ks) {
@@ -1802,7 +1843,7 @@ __device__ __forceinline__ void crt_reconstruct_body(const int8_t* __restrict__ 
         uint32_t w[4];
         int64_t d[4];
         lw.sums(sums + cl * S, L, d);
-        lw.reconstruct(d, quotient[cl], multiple[cl], i0 + cl < args.n, w);
+        lw.reconstruct(d, quotient[cl], multiple[cl], ROWS > 1 || i0 + cl < args.n, w);
         // c over the coefficient's own sums (its lanes have read them all)
         u32_alias* cw = reinterpret_cast<u32_alias*>(lds + size_t(cl) * S * 8);
 #pragma unroll
@@ -1810,13 +1851,15 @@ __device__ __forceinline__ void crt_reconstruct_body(const int8_t* __restrict__ 
             if (4 * g + u < L) cw[4 * g + u] = w[u];
     }
     __syncthreads();
-    const uint32_t rows = i0 < args.n ? (args.n - i0 < T ? args.n - i0 : T) : 0;
+    const uint32_t rows = ROWS > 1 ? T : i0 < args.n ? (args.n - i0 < T ? args.n - i0 : T) : 0;
     uint32_t* out = c + size_t(k0) * L;
     const u32_alias* staged = reinterpret_cast<const u32_alias*>(lds);
     const uint32_t dq = NTH / L, dr = NTH % L;  // (row, column) of word k, stepped by NTH words
     uint32_t row = tid / L, col = tid % L;
     for (uint32_t k = tid; k < rows * L; k += NTH) {
-        out[k] = staged[row * (2 * S) + col];
+        // rows of one matrix row are consecutive coefficients
+        const size_t at = ROWS > 1 ? size_t(row / CW * (kRowWidth - CW)) * L + k : k;
+        out[at] = staged[row * (2 * S) + col];
         row += dq;
         col += dr;
         if (col >= L) {
@@ -1826,16 +1869,18 @@ __device__ __forceinline__ void crt_reconstruct_body(const int8_t* __restrict__ 
     }
 }
 
-template <int WM, int NW, bool kPlanes>
+template <int WM, int NW, int ROWS>
 __global__ __launch_bounds__(64 * NW, 4) void crt_reconstruct(const int8_t* __restrict__ wtiles,
                                                        const int8_t* __restrict__ rtiles,
-                                                       const uint32_t* __restrict__ planes, uint32_t* __restrict__ c,
+                                                       const uint32_t* __restrict__ planes,
+                                                       const PrimeConst* __restrict__ consts,
+                                                       const uint2* __restrict__ twi, uint32_t* __restrict__ c,
                                                        const uint32_t* __restrict__ q,
                                                        const uint32_t* __restrict__ neg_p,
                                                        const uint32_t* __restrict__ corr_t,
                                                        const uint32_t* __restrict__ corr_e, CrtFusedArgs args) {
     extern __shared__ __attribute__((aligned(16))) int8_t dyn_lds[];
-    crt_reconstruct_body<WM, NW, kPlanes>(wtiles, rtiles, planes, c, q, neg_p, corr_t, corr_e, args, blockIdx.x, dyn_lds);
+    crt_reconstruct_body<WM, NW, ROWS>(wtiles, rtiles, planes, consts, twi, c, q, neg_p, corr_t, corr_e, args, blockIdx.x, dyn_lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -2009,15 +2054,19 @@ __global__ __launch_bounds__(256, 4) void crt_reconstruct_group(GroupLaunch g) {
     uint32_t local;
     const GroupView& it = group_entry(g, local);
     const CrtFusedArgs args{it.n, it.limbs, it.t_words, (it.r + 15) / 16, it.r_pad / 16, it.r, it.n_pad,
-                            every_tile(it), it.top_m, it.top_e, it.k_shift, it.mu};
-    auto run = [&](auto wm, auto from_planes) {
-        crt_reconstruct_body<wm(), 4, from_planes()>(in_global(it.wcrt), in_global(it.rtiles), in_global(it.planes),
-                                                     in_global(it.c), in_global(it.q), in_global(it.neg_p),
+                            it.n2, every_tile(it), it.top_m, it.top_e, it.k_shift, it.mu};
+    auto run = [&](auto wm, auto rows) {
+        crt_reconstruct_body<wm(), 4, rows()>(in_global(it.wcrt), in_global(it.rtiles), in_global(it.planes),
+                                              in_global(it.consts), in_global(it.tw_inv), in_global(it.c), in_global(it.q), in_global(it.neg_p),
                                                      in_global(it.corr_t), in_global(it.corr_e), args, local, dyn_lds);
     };
     auto residues = [&](auto wm) {
-        if (it.rows == 1) run(wm, std::true_type());  // residues_from_planes
-        else run(wm, std::false_type());
+        switch (it.rows) {  // residues_from_planes, up to 4 rows
+            case 1: run(wm, std::integral_constant<int, 1>()); break;
+            case 2: run(wm, std::integral_constant<int, 2>()); break;
+            case 4: run(wm, std::integral_constant<int, 4>()); break;
+            default: run(wm, std::integral_constant<int, 0>()); break;
+        }
     };
     switch (fused_waves(it.crt_words)) {
         case 1: residues(std::integral_constant<int, 1>()); break;
@@ -2503,29 +2552,35 @@ void launch_crt_reconstruct(const Shape& s, const DeviceTables& t, const int8_t*
     check_tiles(s, ts, "crt_reconstruct");
     if (!reconstruct_fused(s)) throw std::logic_error("crt_reconstruct: more word sums than a block holds");
     const uint32_t top_m = barrett_top(s), ksteps = (s.r + 15) / 16, wm = fused_waves(s.crt_words);
-    const CrtFusedArgs args{s.n, s.limbs, s.t_words, ksteps, s.r_pad / 16, s.r, s.n_pad, ts, top_m, s.s_shift - 32 * top_m,
+    const CrtFusedArgs args{s.n, s.limbs, s.t_words, ksteps, s.r_pad / 16, s.r, s.n_pad, s.n2, ts, top_m, s.s_shift - 32 * top_m,
                             s.k_shift, s.mu};
 #define PM_FUSED(W, NW, P)                                                                                       \
     hipLaunchKernelGGL((crt_reconstruct<W, NW, P>), dim3(ts.count * (kTile / (16 * NW))), dim3(64 * NW),             \
-                       fused_lds_bytes(W, NW, ksteps), stream, t.wcrt, rtiles, planes, c, t.q, t.neg_p, t.corr_t,         \
+                       fused_lds_bytes(W, NW, ksteps), stream, t.wcrt, rtiles, planes, t.consts, t.tw_inv, c, t.q, t.neg_p, t.corr_t,         \
                        t.corr_e, args)
     // Blocks of eight waves read the weights half as often per coefficient (at
     // N = 65536 with 55 limbs 23.4 us against 29.2 us with four waves); below
     // 65536 coefficients there are too few of them, and smaller blocks start sooner.
     const bool wide = ts.count >= 256;
-    if (residues_from_planes(s)) {
-        if (wm == 1) PM_FUSED(1, 4, true);
-        else if (wm == 2) PM_FUSED(2, 4, true);
-        else PM_FUSED(4, 4, true);
-    } else if (wide) {
-        if (wm == 1) PM_FUSED(1, 8, false);
-        else if (wm == 2) PM_FUSED(2, 8, false);
-        else PM_FUSED(4, 8, false);
+#define PM_FUSED_WM(NW, R)                    \
+    do {                                      \
+        if (wm == 1) PM_FUSED(1, NW, R);      \
+        else if (wm == 2) PM_FUSED(2, NW, R); \
+        else PM_FUSED(4, NW, R);              \
+    } while (0)
+    if (!residues_from_planes(s, ts)) {
+        if (wide) PM_FUSED_WM(8, 0);
+        else PM_FUSED_WM(4, 0);
+    } else if (s.rows == 1) {
+        PM_FUSED_WM(4, 1);
+    } else if (s.rows == 2) {
+        PM_FUSED_WM(4, 2);
+    } else if (s.rows == 4) {
+        PM_FUSED_WM(4, 4);
     } else {
-        if (wm == 1) PM_FUSED(1, 4, false);
-        else if (wm == 2) PM_FUSED(2, 4, false);
-        else PM_FUSED(4, 4, false);
+        PM_FUSED_WM(8, 8);
     }
+#undef PM_FUSED_WM
 #undef PM_FUSED
     check_launch("crt_reconstruct");
 }
@@ -2666,7 +2721,7 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
     });
     for (uint32_t R = 8; R <= 64; R *= 2)
         add(kInverse, R, [&](const GroupItem& it) {
-            const bool skip = it.rows == 1 && it.crt_words <= kFusedWords;  // residues_from_planes
+            const bool skip = it.rows <= 4 && it.crt_words <= kFusedWords;  // crt_reconstruct_group does it
             return row_kernel(it) == R && !skip ? uint64_t(it.row_width / 16) * (it.r_pad / 16) : 0;
         });
     add(kCrtRec, 0, [&](const GroupItem& it) { return it.crt_words <= kFusedWords ? 4 * ntiles(it) : 0; });

@@ -41,9 +41,12 @@ struct DeviceWork {
 // crt_words rounded up to 16 (128-byte rows) above 64 words.
 constexpr uint32_t kFusedWords = 64;
 inline bool reconstruct_fused(const Shape& s) { return s.crt_words <= kFusedWords; }
-// One transform row: the inverse column stage would be a mere transpose into
-// the CRT operand tiles, which the fused kernel does on its way into LDS.
-inline bool residues_from_planes(const Shape& s) { return s.rows == 1 && reconstruct_fused(s); }
+// Up to 8 transform rows, and the whole product at once: the fused kernel reads
+// the row stage's results itself and does the inverse column stages (with one
+// row: none) on their way into its operand layout in LDS.
+inline bool residues_from_planes(const Shape& s, const TileSet& ts) {
+    return s.rows <= 8 && reconstruct_fused(s) && (s.rows == 1 || (ts.t0 == 0 && ts.w == ts.count && ts.count == s.n_pad / 256));
+}
 inline uint32_t word_stride(const Shape& s) { return s.t_words > 64 ? (s.crt_words + 15) / 16 * 16 : s.crt_words; }
 inline size_t word_sum_elements(const Shape& s) { return size_t(s.n_pad) * word_stride(s); }
 
@@ -103,7 +106,7 @@ void launch_crt(const Shape& s, const DeviceTables& t, const int8_t* rtiles, int
 // takes the residue tiles and writes each word of c once, so c may well be
 // pinned host memory; launch_reconstruct takes the word sums, and a coefficient
 // whose quotient estimate was off is written again by a later pass.
-// With residues_from_planes(s) it reads the row stage's results in `planes`
+// With residues_from_planes(s, ts) it reads the row stage's results in `planes`
 // itself, and no inverse column launch is needed.
 void launch_crt_reconstruct(const Shape& s, const DeviceTables& t, const int8_t* rtiles, const uint32_t* planes,
                             uint32_t* c, const TileSet& ts, hipStream_t stream);

@@ -338,7 +338,7 @@ struct pm_plan {
             }
             if (!chunks.strips) pm::launch_ntt_forward_columns(s, tables, work.planes, 0, nops, stream);
             pm::launch_ntt_rows_product(s, tables, work.planes, bplanes, stream);
-            if (!chunks.strips && !pm::residues_from_planes(s))
+            if (!chunks.strips && !pm::residues_from_planes(s, chunks.set[0]))
                 pm::launch_ntt_inverse_columns(s, tables, work.planes, work.rtiles, stream);
             // Output half, per chunk: the inverse column stages of the strips it
             // starts, its CRT GEMM, its reconstruction, then its D2H on the copy
@@ -554,7 +554,7 @@ struct pm_plan {
         mark(3);
         pm::launch_ntt_rows_product(s, tables, w.planes, bplanes, st);
         mark(4);
-        if (!pm::residues_from_planes(s) || last != PM_STAGE_OUTPUT)
+        if (!pm::residues_from_planes(s, all) || last != PM_STAGE_OUTPUT)
             pm::launch_ntt_inverse_columns(s, tables, w.planes, w.rtiles, st);
         mark(5);
         if (last == PM_STAGE_PRODUCT) return;

@@ -3,7 +3,8 @@ the edges of their variants.  The kernel that does the CRT GEMM too: 12, 28 and
 60 limbs are the widest q of one, two and four waves of word sums, 61 the
 narrowest that takes the separate kernels; of those, 124 and 252 limbs are the
 widest q of 32 and 64 lanes.  N below, at and above the blocks' coefficients,
-and enough of them for the separate kernels; q all ones, a power of two, one,
+enough of them for the separate kernels, and two, four and eight transform rows,
+whose inverse column stages the fused kernel does; q all ones, a power of two, one,
 and with zero limbs on top; operands random, all q-1 and zero.  Bit-exact, so
 there is no tolerance."""
 import sys
@@ -27,7 +28,8 @@ LIMBS = [1, 2, 6, 12, 13, 28, 29, 60, 61, 62, 63, 124, 125, 251, 252, 253]
 
 
 @pytest.mark.parametrize("n,limbs", [(n, limbs) for n in (1, 32, 64, 128, 1024) for limbs in LIMBS] +
-                         [(4096, limbs) for limbs in LIMBS if limbs > 60])
+                         [(4096, limbs) for limbs in LIMBS if limbs > 60] +
+                         [(n, limbs) for n in (4096, 8192, 16384) for limbs in (12, 28, 60)])
 def test_fused_reconstruction(polymul, workloads, oracle, n, limbs):
     rng = np.random.default_rng(91000 + 100 * limbs + n)
     for kind, q in _moduli(limbs, workloads, rng).items():
