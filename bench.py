@@ -452,7 +452,11 @@ SQ_COUNTERS = ["SQ_WAVE_CYCLES", "SQ_BUSY_CYCLES", "SQ_VALU_MFMA_BUSY_CYCLES", "
 
 
 def _short_kernel(name):
-    return name.replace("pm::", "").replace("(anonymous namespace)::", "").split("(")[0]
+    name = name.replace("pm::", "").replace("(anonymous namespace)::", "").split("(")[0]
+    for gemm in ("conversion_gemm", "crt_gemm"):  # whichever block tile the shape takes
+        if name.startswith("void %s<" % gemm):
+            return gemm
+    return name
 
 
 def _counters(path):
