@@ -236,13 +236,14 @@ pm_status pm_operand_create(pm_plan* plan, const uint32_t* b, pm_operand** out) 
         const size_t bytes = size_t(s.n) * s.limbs * sizeof(uint32_t);
         const pm::TileSet all = pm::all_tiles(s);
         hip_check(hipMemcpyAsync(plan->io_b, b, bytes, hipMemcpyHostToDevice, st), "copy b to device");
+        const bool columns = pm::conversion_columns(s, all);
         if (pm::conversion_short(s)) {
-            pm::launch_convert(s, plan->tables, nullptr, plan->io_b, plan->work.planes, all, 1, 1, st);
+            pm::launch_convert(s, plan->tables, nullptr, plan->io_b, plan->work.planes, all, 1, 1, columns, st);
         } else {
             pm::launch_pack(s, nullptr, plan->io_b, plan->work.packed, all, 1, 1, st);
             pm::launch_conversion(s, plan->tables, plan->work.packed, plan->work.planes, all, 1, 1, st);
         }
-        pm::launch_ntt_forward_columns(s, plan->tables, plan->work.planes, 1, 1, st);
+        if (!columns) pm::launch_ntt_forward_columns(s, plan->tables, plan->work.planes, 1, 1, st);
         hip_check(hipMemcpyAsync(op->planes, plan->b_planes(), plane_words * sizeof(uint32_t),
                                  hipMemcpyDeviceToDevice, st),
                   "keep b residues");

@@ -55,6 +55,8 @@ constexpr uint32_t kWaveM = 4, kWaveN = 8;    // 16x16 tiles per wave
 constexpr uint32_t kWaveRows = kWaveM * 16, kWaveCols = kWaveN * 16;
 constexpr uint32_t kGroupN = 4;               // raster group width (tiles)
 
+constexpr uint32_t kRowWidth = 2048;          // C of every transform of more than one row
+
 void check_launch(const char* what) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
@@ -101,6 +103,31 @@ __device__ __forceinline__ uint32_t redc_wide(uint64_t t, uint32_t p, uint32_t p
     hi = min(hi, hi - p);  // t - p*2^32, in redc's range, when that is not negative
     const uint32_t r = hi - mh;
     return min(r, r + p);
+}
+
+// Cooley-Tukey: (a, b) -> (a + wb, a - wb).  a < p; b may be any 32-bit value
+// congruent to its residue.  With kReduce the outputs are below p; without,
+// below 2p, which is all the next level asks of the values it multiplies (b),
+// and half of every level's outputs are that: 8 instead of 11 instructions.
+// (Primes just below 2^31 leave no room for Harvey's form, lazy in all of them.)
+template <bool kReduce>
+__device__ __forceinline__ void ct_butterfly(uint32_t& a, uint32_t& b, uint2 w, uint32_t p) {
+    const uint32_t v = mul_shoup(b, w.x, w.y, p);
+    if constexpr (kReduce) {
+        b = sub_mod(a, v, p);
+        a = add_mod(a, v, p);
+    } else {
+        b = a - v + p;
+        a = a + v;
+    }
+}
+
+// Gentleman-Sande: (a, b) -> (a + b, w (a - b)), all below p; the difference
+// goes into the product as it is, below 2p.
+__device__ __forceinline__ void gs_butterfly(uint32_t& a, uint32_t& b, uint2 w, uint32_t p) {
+    const uint32_t u = a, v = b;
+    a = add_mod(u, v, p);
+    b = mul_shoup(u - v + p, w.x, w.y, p);
 }
 
 __device__ __forceinline__ uint32_t mont(uint32_t a, uint32_t b, uint32_t p, uint32_t pinv) {
@@ -412,20 +439,23 @@ __global__ __launch_bounds__(256 * WN, 2) void conversion_gemm(const int8_t* __r
 //    gemm_mainloop; each chunk is multiplied, reduced and stored with no wait
 //    in between.
 //  * gridDim.y splits the primes over blocks when there are few coefficients.
+//  * ROWS > 1: a lane's fragments are the rows of whole columns, and it does the
+//    forward column stages before it stores (convert_plan).
 // What bounds it at N = 65536 with 55 limbs (30.7 us, packing and GEMM before:
 // 14.7 + 36.5): the 29 MB of limbs read and 60 MB of residues written, about
 // 18 us at a large copy's rate, with the MFMAs (7 us) and the reductions (5 us)
 // beside them.  At N = 131072 with 4 limbs 11.1 against 18.4 + 21.2 us, at
 // N = 128 with 128 limbs 4.8 against 2.9 + 12.0, at N = 8192 with 226 41.8
 // against 7.9 + 37.5, at N = 65536 with 226 339 against 47 + 319.  Beyond 256
-// limbs a wave's registers hold too few coefficients to feed the MFMAs from LDS.  (Operand bytes in LDS and
-// weights straight from L2, one barrier per block: 37 us at N = 65536; the
-// weight fragments then come from L2 once per wave.)
+// limbs a wave's registers hold too few coefficients to feed the MFMAs from
+// LDS.  (Operand bytes in LDS and weights straight from L2, one barrier per
+// block: 37 us at N = 65536; the weight fragments then come from L2 once per
+// wave.)
 // ---------------------------------------------------------------------------
 constexpr uint32_t kConvertStage = 48 << 10;  // LDS bytes of weights: three blocks per CU
 
 struct ConvertArgs {
-    uint32_t n, n_pad, limbs, r, r_pad, conv_rows, ksteps;
+    uint32_t n, n_pad, limbs, r, r_pad, conv_rows, ksteps, n2;
     TileSet ts;  // tile k's rows are rows k*256 .. of a and b (pack_body)
     uint32_t op0;
 };
@@ -435,30 +465,42 @@ constexpr uint32_t convert_stage_chunks(uint32_t ksteps) {
     return chunk < kConvertStage ? kConvertStage / chunk : 1;
 }
 
-// The staged weights, then the primes' constants.
-constexpr size_t convert_lds_bytes(uint32_t ksteps, uint32_t r) {
-    return size_t(convert_stage_chunks(ksteps)) * ksteps * kWaveRows * kTK + size_t(r) * sizeof(PrimeConst);
+// 16-prime chunks of one of `split` blocks that share the primes.
+__host__ __device__ constexpr uint32_t convert_share(uint32_t r, uint32_t split) {
+    return ((r + 15) / 16 + split - 1) / split;
+}
+
+// The staged weights, then the constants and (columns > 1) twiddles of a share's primes.
+constexpr size_t convert_lds_bytes(uint32_t ksteps, uint32_t r, uint32_t split, uint32_t columns) {
+    return size_t(convert_stage_chunks(ksteps)) * ksteps * kWaveRows * kTK +
+           size_t(convert_share(r, split)) * 16 * (sizeof(PrimeConst) + (columns > 1 ? columns * sizeof(uint2) : 0));
 }
 
 // Blocks (bx, by) of (., ny).
-template <int KS, int NT>
+template <int KS, int NT, int ROWS>
 __device__ __forceinline__ void convert_body(const uint32_t* __restrict__ a, const uint32_t* __restrict__ b,
                                              const int8_t* __restrict__ wtiles,
-                                             const PrimeConst* __restrict__ consts, uint32_t* __restrict__ planes,
+                                             const PrimeConst* __restrict__ consts,
+                                             const uint2* __restrict__ twf, uint32_t* __restrict__ planes,
                                              const ConvertArgs& args, uint32_t bx, uint32_t by, uint32_t ny,
                                              int8_t* lds) {
     typedef uint32_t v4u_word __attribute__((ext_vector_type(4), aligned(4)));  // 4-byte aligned
     constexpr uint32_t T = 64 * NT, kChunkStep = kWaveRows * kTK;                 // 4 KB: 64 rows of one K step
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t L = args.limbs, ksteps = args.ksteps;
-    const uint32_t per_op = args.ts.count * (kTile / T);
-    const uint32_t op = args.op0 + bx / per_op, k0 = bx % per_op * T;
-    const uint32_t i0 = tile_at(args.ts, k0 / kTile) * kTile + k0 % kTile;
-    const uint32_t rows = i0 < args.n ? (args.n - i0 < T ? args.n - i0 : T) : 0;
-    const uint32_t chunks = (args.r + 15) / 16, share = (chunks + ny - 1) / ny;
+    const uint32_t per_op = args.ts.count * kTile / T;
+    // The block's coefficients: T consecutive ones of the set, fragment ni of a
+    // wave 16 of them; or (ROWS > 1) T / ROWS columns of the transform's
+    // [ROWS][2048] matrix, fragment ni row ni % ROWS of 16 columns, so that a lane
+    // holds whole columns.
+    const uint32_t op = args.op0 + bx / per_op, k0 = bx % per_op * (T / ROWS);
+    const uint32_t i0 = ROWS > 1 ? k0 : tile_at(args.ts, k0 / kTile) * kTile + k0 % kTile;
+    const uint32_t rows = ROWS > 1 ? T : i0 < args.n ? (args.n - i0 < T ? args.n - i0 : T) : 0;
+    auto place = [](uint32_t ni) { return ni / ROWS * 16 + (ROWS > 1 ? ni % ROWS * kRowWidth : 0); };
+    const uint32_t chunks = (args.r + 15) / 16, share = convert_share(args.r, ny);
     const uint32_t c0 = by * share, c1 = c0 + share < chunks ? c0 + share : chunks;
     if (!rows || c0 >= c1) return;  // whole block
-    const uint32_t cl = wave * 16 * NT + (lane & 15);  // the lane's first coefficient of the block's
+    const uint32_t cl = wave * (16 * NT / ROWS) + (lane & 15);  // the lane's first coefficient of the block's
 
     v4i fb[KS][NT];
     {
@@ -468,7 +510,7 @@ __device__ __forceinline__ void convert_body(const uint32_t* __restrict__ a, con
         for (uint32_t ks = 0; ks < KS; ++ks)
 #pragma unroll
             for (uint32_t ni = 0; ni < NT; ++ni) {
-                const uint32_t row = cl + ni * 16 < rows ? cl + ni * 16 : rows - 1, w = ks * 16 + w0;
+                const uint32_t row = ROWS > 1 || cl + ni * 16 < rows ? cl + place(ni) : rows - 1, w = ks * 16 + w0;
                 const uint32_t* p = src + size_t(row) * L + w;
                 v4u x = {0, 0, 0, 0};
                 if (w + 4 <= L) {
@@ -484,6 +526,11 @@ __device__ __forceinline__ void convert_body(const uint32_t* __restrict__ a, con
     const uint32_t stage = convert_stage_chunks(ksteps), num_m = args.conv_rows / kTile;
     PrimeConst* pcs = reinterpret_cast<PrimeConst*>(lds + stage * ksteps * kChunkStep);
     for (uint32_t k = c0 * 16 + tid; k < args.r && k < c1 * 16; k += 256) pcs[k - c0 * 16] = consts[k];
+    // the column stages' twiddles, ROWS per prime (entry 0 unused)
+    uint2* tws = reinterpret_cast<uint2*>(pcs + share * 16);
+    if constexpr (ROWS > 1)
+        for (uint32_t k = c0 * 16 * ROWS + tid; k < args.r * ROWS && k < c1 * 16 * ROWS; k += 256)
+            tws[k - c0 * 16 * ROWS] = twf[size_t(k / ROWS) * args.n2 + k % ROWS];
     // thread tid fills slot tid of a chunk's K step: row tid>>2, chunk swizzled as in swz
     const uint32_t srow = tid >> 2, sbyte = srow * kTK + ((tid & 3) ^ ((srow >> 1) & 3)) * 16;
     const DigitScales ds = digit_scales();
@@ -527,22 +574,43 @@ __device__ __forceinline__ void convert_body(const uint32_t* __restrict__ a, con
                 const PrimeConst pc = pcs[kp - c0 * 16];
                 const int64_t off = int64_t(op ? pc.off_b : pc.off_a) + (int64_t(pc.p) << 31);
                 uint32_t* out = planes + (size_t(op) * args.r_pad + kp) * args.n_pad + i0 + cl;
+                uint32_t x[NT];
+#pragma unroll
+                for (uint32_t ni = 0; ni < NT; ++ni) x[ni] = redc(uint64_t(combine4(acc[mi][ni], ds, off)), pc.p, pc.pinv);
+                if constexpr (ROWS > 1) {  // the forward column stages (forward_reg_body)
+                    const uint2* tw = tws + (kp - c0 * 16) * ROWS;
+#pragma unroll
+                    for (int m = 1, half = ROWS / 2; m < ROWS; m *= 2, half /= 2)
+#pragma unroll
+                        for (int g = 0; g < m; ++g) {
+                            const uint2 t = tw[m + g];
+#pragma unroll
+                            for (int cg = 0; cg < NT / ROWS; ++cg)
+#pragma unroll
+                                for (int jr = 0; jr < half; ++jr) {
+                                    uint32_t &lo = x[cg * ROWS + 2 * half * g + jr],
+                                             &hi = x[cg * ROWS + 2 * half * g + jr + half];
+                                    if (half == 1 || !(jr & (half / 2))) ct_butterfly<true>(lo, hi, t, pc.p);
+                                    else ct_butterfly<false>(lo, hi, t, pc.p);
+                                }
+                        }
+                }
 #pragma unroll
                 for (uint32_t ni = 0; ni < NT; ++ni)
-                    if (cl + ni * 16 < rows)
-                        out[ni * 16] = redc(uint64_t(combine4(acc[mi][ni], ds, off)), pc.p, pc.pinv);
+                    if (ROWS > 1 || cl + ni * 16 < rows) out[place(ni)] = x[ni];
             }
         }
     }
 }
 
-template <int KS, int NT>
-__global__ __launch_bounds__(256, KS * NT > 16 ? 2 : 3) void convert(const uint32_t* __restrict__ a, const uint32_t* __restrict__ b,
+template <int KS, int NT, int ROWS>
+__global__ __launch_bounds__(256, KS * NT > 16 || NT == 8 ? 2 : 3) void convert(const uint32_t* __restrict__ a, const uint32_t* __restrict__ b,
                                                   const int8_t* __restrict__ wtiles,
                                                   const PrimeConst* __restrict__ consts,
-                                                  uint32_t* __restrict__ planes, ConvertArgs args) {
+                                                  const uint2* __restrict__ twf, uint32_t* __restrict__ planes,
+                                                  ConvertArgs args) {
     extern __shared__ __attribute__((aligned(16))) int8_t dyn_lds[];
-    convert_body<KS, NT>(a, b, wtiles, consts, planes, args, blockIdx.x, blockIdx.y, gridDim.y, dyn_lds);
+    convert_body<KS, NT, ROWS>(a, b, wtiles, consts, twf, planes, args, blockIdx.x, blockIdx.y, gridDim.y, dyn_lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -837,33 +905,6 @@ __global__ __launch_bounds__(256) void ntt_columns_inverse(uint32_t* __restrict_
 // ---------------------------------------------------------------------------
 // Register-resident NTT kernels for the usual shapes (rows <= 64, C = 2048).
 // ---------------------------------------------------------------------------
-constexpr uint32_t kRowWidth = 2048;  // C of every transform of more than one row
-
-// Cooley-Tukey: (a, b) -> (a + wb, a - wb).  a < p; b may be any 32-bit value
-// congruent to its residue.  With kReduce the outputs are below p; without,
-// below 2p, which is all the next level asks of the values it multiplies (b),
-// and half of every level's outputs are that: 8 instead of 11 instructions.
-// (Primes just below 2^31 leave no room for Harvey's form, lazy in all of them.)
-template <bool kReduce>
-__device__ __forceinline__ void ct_butterfly(uint32_t& a, uint32_t& b, uint2 w, uint32_t p) {
-    const uint32_t v = mul_shoup(b, w.x, w.y, p);
-    if constexpr (kReduce) {
-        b = sub_mod(a, v, p);
-        a = add_mod(a, v, p);
-    } else {
-        b = a - v + p;
-        a = a + v;
-    }
-}
-
-// Gentleman-Sande: (a, b) -> (a + b, w (a - b)), all below p; the difference
-// goes into the product as it is, below 2p.
-__device__ __forceinline__ void gs_butterfly(uint32_t& a, uint32_t& b, uint2 w, uint32_t p) {
-    const uint32_t u = a, v = b;
-    a = add_mod(u, v, p);
-    b = mul_shoup(u - v + p, w.x, w.y, p);
-}
-
 // Forward row-spanning stages: one thread per (operand, prime, column) holding
 // the column's ROWS values; the stage twiddles are uniform over the block.
 // Columns col0 + [0, 256 * gridDim.x).
@@ -1899,7 +1940,7 @@ __global__ __launch_bounds__(64 * NW, 4) void crt_reconstruct(const int8_t* __re
 struct GroupView {
     uint32_t n, n_pad, limbs, r, r_pad, conv_rows, conv_k, crt_rows, crt_k, crt_words, ws, t_words;
     uint32_t n1, n2, rows, row_width, s_shift, k_shift, top_m, top_e;
-    uint32_t conv_ks, conv_nt, conv_split;  // short conversion (launch_convert)
+    uint32_t conv_ks, conv_nt, conv_split, conv_columns;  // short conversion (launch_convert)
     uint64_t mu;
     const PM_GLOBAL PrimeConst* consts;
     const PM_GLOBAL int8_t* wconv;
@@ -1975,17 +2016,24 @@ __global__ __launch_bounds__(256, 3) void convert_group(GroupLaunch g) {
     uint32_t local;
     const GroupView& it = group_entry(g, local);
     const uint32_t nx = 2 * it.n_pad / (64 * it.conv_nt);
-    const ConvertArgs args{it.n, it.n_pad, it.limbs, it.r, it.r_pad, it.conv_rows, it.conv_k / kTK,
+    const ConvertArgs args{it.n, it.n_pad, it.limbs, it.r, it.r_pad, it.conv_rows, it.conv_k / kTK, it.n2,
                            every_tile(it), 0};
-    auto run = [&](auto ks, auto nt) {
-        convert_body<ks(), nt()>(in_global(it.a), in_global(it.b), in_global(it.wconv), in_global(it.consts),
-                                 in_global(it.planes), args, local % nx, local / nx, it.conv_split, dyn_lds);
+    auto run = [&](auto ks, auto nt, auto rows) {
+        convert_body<ks(), nt(), rows()>(in_global(it.a), in_global(it.b), in_global(it.wconv), in_global(it.consts),
+                                         in_global(it.tw_fwd), in_global(it.planes), args, local % nx, local / nx,
+                                         it.conv_split, dyn_lds);
+    };
+    using std::integral_constant;
+    auto columns = [&](auto ks, auto nt) {
+        if (it.conv_columns == 1) run(ks, nt, integral_constant<int, 1>());
+        else if (it.conv_columns == 2) run(ks, nt, integral_constant<int, 2>());
+        else if constexpr (nt() == 4) run(ks, nt, integral_constant<int, 4>());
     };
     switch (it.conv_ks) {  // convert_plan's wide waves
-        case 1: run(std::integral_constant<int, 1>(), std::integral_constant<int, 4>()); break;
-        case 2: run(std::integral_constant<int, 2>(), std::integral_constant<int, 4>()); break;
-        case 4: run(std::integral_constant<int, 4>(), std::integral_constant<int, 4>()); break;
-        default: run(std::integral_constant<int, 8>(), std::integral_constant<int, 2>()); break;
+        case 1: columns(integral_constant<int, 1>(), integral_constant<int, 4>()); break;
+        case 2: columns(integral_constant<int, 2>(), integral_constant<int, 4>()); break;
+        case 4: columns(integral_constant<int, 4>(), integral_constant<int, 4>()); break;
+        default: columns(integral_constant<int, 8>(), integral_constant<int, 2>()); break;
     }
 }
 
@@ -2368,9 +2416,10 @@ void launch_conversion(const Shape& s, const DeviceTables& t, const int8_t* pack
 namespace {
 
 // Variant of the short conversion: K steps held in registers (KS), 16-coefficient
-// fragments per wave (NT), splits of the primes over blocks.
+// fragments per wave (NT), transform rows whose column stages a lane does (1:
+// none), splits of the primes over blocks.
 struct ConvertPlan {
-    uint32_t ks, nt, split;
+    uint32_t ks, nt, rows, split;
 };
 constexpr uint32_t kConvertBlocks = 512, kConvertGroupBlocks = 64;  // two per CU; a batch's share
 // Up to here a batch's products take the short conversion: 16 K steps in
@@ -2386,30 +2435,52 @@ constexpr uint32_t kGroupShortLimbs = 128;
 // products fill the GPU, so there want_blocks is small and the waves wide: the
 // batch of 64 small products' conversions take 152 us in all, and 210 with each
 // product spread as if it were alone.
-ConvertPlan convert_plan(uint32_t r, uint32_t ksteps, uint32_t tiles, uint32_t want_blocks) {
-    const uint32_t chunks = (r + 15) / 16, ks = ksteps <= 1 ? 1 : ksteps <= 2 ? 2 : ksteps <= 4 ? 4 : ksteps <= 8 ? 8 : 16;
-    uint32_t nt = ks >= 8 ? 2 : 4;
-    if (want_blocks == kConvertBlocks && tiles * (4 / nt) * chunks < want_blocks / 2) nt = 1;
-    const uint32_t blocks = tiles * (4 / nt), want = (want_blocks + blocks - 1) / blocks;
-    return ConvertPlan{ks, nt, chunks < want ? chunks : want};
+//
+// `columns`: a lane takes the column stages where it holds whole columns, with
+// as many rows as fragments at most (8, with up to two K steps, is what the
+// registers hold; not in a batch, whose one kernel has three waves per SIMD).
+// That saves a pass over the residues and a launch, and is worth wide waves at
+// any number of blocks, whole products in us: N = 4096 with 1 limb 28.3 -> 25.8,
+// with 32 limbs 38.6 -> 36.0, with 125 65.9 -> 61.3, with 256 96.6 -> 89.4; N =
+// 8192 with 2 limbs 28.5 -> 26.3, with 64 64.7 -> 59.7; N = 16384 with 2 limbs
+// 29.2 -> 28.4, with 28 44.1 -> 41.7.
+ConvertPlan convert_plan(const Shape& s, uint32_t tiles, uint32_t want_blocks, bool columns) {
+    const uint32_t ksteps = s.conv_k / kTK, chunks = (s.r + 15) / 16;
+    const uint32_t ks = ksteps <= 1 ? 1 : ksteps <= 2 ? 2 : ksteps <= 4 ? 4 : ksteps <= 8 ? 8 : 16;
+    const bool batch = want_blocks == kConvertGroupBlocks;
+    const uint32_t wide = ks >= 8 ? 2 : 4, most = ks <= 2 && !batch ? 8 : wide;
+    const uint32_t rows = columns && s.rows <= most ? s.rows : 1;
+    uint32_t nt = rows > wide ? rows : wide;
+    if (rows == 1 && !batch && tiles * 4 / nt * chunks < want_blocks / 2) nt = 1;
+    const uint32_t blocks = tiles * 4 / nt, want = (want_blocks + blocks - 1) / blocks;
+    return ConvertPlan{ks, nt, rows, chunks < want ? chunks : want};
 }
 
 }  // namespace
 
-#define PM_CONVERT_VARIANTS(X) X(1, 1) X(2, 1) X(4, 1) X(8, 1) X(16, 1) X(1, 4) X(2, 4) X(4, 4) X(8, 2) X(16, 2)
+#define PM_CONVERT_VARIANTS(X)                                                                         \
+    X(1, 1, 1) X(2, 1, 1) X(4, 1, 1) X(8, 1, 1) X(16, 1, 1) X(1, 4, 1) X(2, 4, 1) X(4, 4, 1) X(8, 2, 1) \
+        X(16, 2, 1) X(1, 4, 2) X(2, 4, 2) X(4, 4, 2) X(8, 2, 2) X(16, 2, 2) X(1, 4, 4) X(2, 4, 4)       \
+            X(4, 4, 4) X(1, 8, 8) X(2, 8, 8)
+
+bool conversion_columns(const Shape& s, const TileSet& ts) {
+    if (!conversion_short(s) || ts.t0 != 0 || ts.w != ts.count || ts.count != s.n_pad / kTile) return false;
+    return convert_plan(s, ts.count, kConvertBlocks, true).rows > 1;
+}
 
 void launch_convert(const Shape& s, const DeviceTables& t, const uint32_t* a, const uint32_t* b, uint32_t* planes,
-                    const TileSet& ts, uint32_t op0, uint32_t nops, hipStream_t stream) {
+                    const TileSet& ts, uint32_t op0, uint32_t nops, bool columns, hipStream_t stream) {
     check_tiles(s, ts, "convert");
     if (!conversion_short(s)) throw std::logic_error("convert: operands wider than a wave holds");
+    if (columns && !conversion_columns(s, ts)) throw std::logic_error("convert: column stages not held by a lane");
     const uint32_t ksteps = s.conv_k / kTK;
-    const ConvertArgs args{s.n, s.n_pad, s.limbs, s.r, s.r_pad, s.conv_rows, ksteps, ts, op0};
-    const ConvertPlan cp = convert_plan(s.r, ksteps, nops * ts.count, kConvertBlocks);
-    const dim3 grid(nops * ts.count * (4 / cp.nt), cp.split);
-#define PM_CONVERT(K, N)                                                                                  \
-    if (cp.ks == K && cp.nt == N)                                                                         \
-        hipLaunchKernelGGL((convert<K, N>), grid, dim3(256), convert_lds_bytes(ksteps, s.r), stream, a, b, \
-                           t.wconv, t.consts, planes, args);
+    const ConvertArgs args{s.n, s.n_pad, s.limbs, s.r, s.r_pad, s.conv_rows, ksteps, s.n2, ts, op0};
+    const ConvertPlan cp = convert_plan(s, nops * ts.count, kConvertBlocks, columns);
+    const dim3 grid(nops * ts.count * 4 / cp.nt, cp.split);
+#define PM_CONVERT(K, N, R)                                                                              \
+    if (cp.ks == K && cp.nt == N && cp.rows == R)                                                        \
+        hipLaunchKernelGGL((convert<K, N, R>), grid, dim3(256), convert_lds_bytes(ksteps, s.r, cp.split, R), \
+                           stream, a, b, t.wconv, t.consts, t.tw_fwd, planes, args);
     PM_CONVERT_VARIANTS(PM_CONVERT)
 #undef PM_CONVERT
     check_launch("convert");
@@ -2614,8 +2685,9 @@ GroupItem group_item(const Shape& s, const DeviceTables& t, const DeviceWork& w,
     it.crt_words = s.crt_words, it.ws = word_stride(s), it.t_words = s.t_words;
     it.n1 = s.n1, it.n2 = s.n2, it.rows = s.rows, it.row_width = s.row_width;
     it.s_shift = s.s_shift, it.k_shift = s.k_shift;
-    const ConvertPlan cp = convert_plan(s.r, s.conv_k / kTK, 2 * s.n_pad / kTile, kConvertGroupBlocks);
+    const ConvertPlan cp = convert_plan(s, 2 * s.n_pad / kTile, kConvertGroupBlocks, true);
     it.conv_ks = cp.ks, it.conv_nt = cp.nt, it.conv_split = cp.split;
+    it.conv_columns = s.limbs <= kGroupShortLimbs ? cp.rows : 1;
     it.top_m = barrett_top(s);
     it.top_e = s.s_shift - 32 * it.top_m;
     it.mu = s.mu;
@@ -2685,7 +2757,7 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
             total += blocks(items[sel[j]]);
             const GroupItem& it = items[sel[j]];
             lds = std::max<size_t>(lds, kind == kCrtRec    ? fused_lds_bytes(fused_waves(it.crt_words), 4, (it.r + 15) / 16)
-                                        : kind == kConvert ? convert_lds_bytes(it.conv_k / kTK, it.r)
+                                        : kind == kConvert ? convert_lds_bytes(it.conv_k / kTK, it.r, it.conv_split, it.conv_columns)
                                                            : size_t(2) * it.row_width * 4);
         }
         if (total >= (uint64_t(1) << 31)) throw std::invalid_argument("launch_group: batch too large for one grid");
@@ -2706,7 +2778,7 @@ void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStre
     auto row_kernel = [](const GroupItem& it) { return it.rows < 8 ? 8 : it.rows; };
     for (uint32_t R = 8; R <= 64; R *= 2)
         add(kForward, R, [&](const GroupItem& it) {
-            return it.rows > 1 && row_kernel(it) == R ? uint64_t(it.row_width / 256) * it.r * 2 : 0;
+            return it.rows > 1 && it.conv_columns == 1 && row_kernel(it) == R ? uint64_t(it.row_width / 256) * it.r * 2 : 0;
         });
 #define PM_GROWS(LC, B)                                                                                        \
     add(kRowsReg, LC * 16 + B, [&](const GroupItem& it) {                                                      \

@@ -37,7 +37,8 @@ struct DeviceWork {
 
 // Up to 60 limbs (64 word sums) one kernel does the CRT GEMM and the
 // reconstruction, and the sums stay in LDS; wider q takes the GEMM, then one
-// wave per coefficient over coefficient-major sums [n_pad][ws] in memory, ws =
+// wave (up to 252 limbs and with more than 8 tiles 32 or 64 lanes, several words
+// each) per coefficient over coefficient-major sums [n_pad][ws] in memory, ws =
 // crt_words rounded up to 16 (128-byte rows) above 64 words.
 constexpr uint32_t kFusedWords = 64;
 inline bool reconstruct_fused(const Shape& s) { return s.crt_words <= kFusedWords; }
@@ -79,8 +80,12 @@ void launch_conversion(const Shape& s, const DeviceTables& t, const int8_t* pack
 // for q of up to kShortLimbs limbs.
 constexpr uint32_t kShortLimbs = 256;
 inline bool conversion_short(const Shape& s) { return s.limbs <= kShortLimbs; }
+// `columns` (only where conversion_columns says so: every tile at once, and two
+// to eight transform rows, fewer for wider q): the forward column stages too,
+// and launch_ntt_forward_columns must not follow.
+bool conversion_columns(const Shape& s, const TileSet& ts);
 void launch_convert(const Shape& s, const DeviceTables& t, const uint32_t* a, const uint32_t* b, uint32_t* planes,
-                    const TileSet& ts, uint32_t op0, uint32_t nops, hipStream_t stream);
+                    const TileSet& ts, uint32_t op0, uint32_t nops, bool columns, hipStream_t stream);
 // Forward row-spanning (column) stages of column strips [strip_begin,
 // strip_end) of 256 columns each, or of every column with the defaults; a strip
 // range needs the register-resident kernel (row_width a multiple of 256, 2 to
@@ -122,7 +127,7 @@ void launch_zero(uint32_t* c, size_t words, hipStream_t stream);
 struct GroupItem {
     uint32_t n, n_pad, limbs, r, r_pad, conv_rows, conv_k, crt_rows, crt_k, crt_words, ws, t_words;
     uint32_t n1, n2, rows, row_width, s_shift, k_shift, top_m, top_e;
-    uint32_t conv_ks, conv_nt, conv_split;  // short conversion (launch_convert)
+    uint32_t conv_ks, conv_nt, conv_split, conv_columns;  // short conversion (launch_convert)
     uint64_t mu;
     const PrimeConst* consts;
     const int8_t* wconv;

@@ -300,6 +300,7 @@ struct pm_plan {
             // 7.27 ms per product with one stream; N = 65536 with 1747 limbs,
             // ratio 0.64: 28.2 against 27.5 ms.)
             const bool two_streams = uint64_t(s.conv_rows) * s.conv_k < uint64_t(45600) * L;
+            const bool columns = !chunks.strips && pm::conversion_columns(s, chunks.set[0]);  // one chunk
             post(jobs[0]);
             for (uint32_t j = 0; j < njobs; ++j) {
                 const Job jb = jobs[j];
@@ -327,7 +328,7 @@ struct pm_plan {
                 const uint32_t* xa = io_a + base;  // pack reads the chunk's k-th tile at rows k*256..
                 const uint32_t* xb = xa + rows * L;
                 if (pm::conversion_short(s)) {
-                    pm::launch_convert(s, tables, xa, xb, work.planes, chunks.set[ch], 0, nops, stream);
+                    pm::launch_convert(s, tables, xa, xb, work.planes, chunks.set[ch], 0, nops, columns, stream);
                 } else {
                     pm::launch_pack(s, xa, xb, work.packed, chunks.set[ch], 0, nops, stream);
                     pm::launch_conversion(s, tables, work.packed, work.planes, chunks.set[ch], 0, nops, stream);
@@ -336,7 +337,7 @@ struct pm_plan {
                     pm::launch_ntt_forward_columns(s, tables, work.planes, 0, nops, stream, chunks.fwd_begin[ch],
                                                    chunks.fwd_end[ch]);
             }
-            if (!chunks.strips) pm::launch_ntt_forward_columns(s, tables, work.planes, 0, nops, stream);
+            if (!chunks.strips && !columns) pm::launch_ntt_forward_columns(s, tables, work.planes, 0, nops, stream);
             pm::launch_ntt_rows_product(s, tables, work.planes, bplanes, stream);
             if (!chunks.strips && !pm::residues_from_planes(s, chunks.set[0]))
                 pm::launch_ntt_inverse_columns(s, tables, work.planes, work.rtiles, stream);
@@ -543,14 +544,15 @@ struct pm_plan {
         const uint32_t nops = b ? 2 : 1;
         const uint32_t* bplanes = b ? b_planes(w) : bplanes_in;
         mark(0);
+        const bool columns = last != PM_STAGE_RESIDUES && pm::conversion_columns(s, all);
         const bool packed = !pm::conversion_short(s);  // else packing is part of the conversion's time
         if (packed) pm::launch_pack(s, a, b, w.packed, all, 0, nops, st);
         mark(1);
         if (packed) pm::launch_conversion(s, tables, w.packed, w.planes, all, 0, nops, st);
-        else pm::launch_convert(s, tables, a, b, w.planes, all, 0, nops, st);
+        else pm::launch_convert(s, tables, a, b, w.planes, all, 0, nops, columns, st);
         mark(2);
         if (last == PM_STAGE_RESIDUES) return;
-        pm::launch_ntt_forward_columns(s, tables, w.planes, 0, nops, st);
+        if (!columns) pm::launch_ntt_forward_columns(s, tables, w.planes, 0, nops, st);
         mark(3);
         pm::launch_ntt_rows_product(s, tables, w.planes, bplanes, st);
         mark(4);

@@ -54,3 +54,32 @@ def test_products(polymul, workloads, oracle, device_memory, n, limbs):
             for ptr in (pa, pb, pc):
                 device_memory.free(ptr)
         assert np.array_equal(got[1:].reshape(n, limbs), expect)
+
+
+@pytest.mark.parametrize("n,limbs", [(4096, 1), (4096, 17), (4096, 64), (4096, 65), (4096, 128), (4096, 129),
+                                     (4096, 256), (8192, 1), (8192, 32), (8192, 33), (8192, 64), (8192, 65), (16384, 1), (16384, 16),
+                                     (16384, 17), (16384, 32), (16384, 33)])
+def test_column_stages(polymul, workloads, oracle, device_memory, n, limbs):
+    """Two, four and eight transform rows, where the conversion does the forward
+    column stages too if a lane holds whole columns (8192 coefficients above 64
+    limbs and 16384 above 32, or in a batch: it does not): alone, with one
+    operand resident, and in a batch."""
+    print("[gpu-case] conversion with column stages", n, limbs, flush=True)
+    q, a, b = _case(workloads, n, limbs, 94000 + n + limbs)
+    a[: n // 2] = workloads.q_minus_one(q)
+    expect = oracle.kronecker_gmp(a, b, q)
+    with polymul.Plan(n, 32 * limbs, limbs, q) as plan, polymul.Plan(n, 32 * limbs, limbs, q) as other:
+        assert np.array_equal(plan.multiply(a, b), expect)
+        with plan.operand(b) as kept:
+            assert np.array_equal(plan.multiply_operand(a, kept), expect)
+        pa, pb = device_memory.upload(a), device_memory.upload(b)
+        pcs = [device_memory.upload(np.zeros_like(a)) for _ in range(2)]
+        try:
+            plan.multiply_device(pa, pb, pcs[0])
+            assert np.array_equal(device_memory.download(pcs[0], a.shape, np.uint32), expect)
+            polymul.multiply_device_batch([plan, other], [pa, pa], [pb, pb], pcs)
+            for pc in pcs:
+                assert np.array_equal(device_memory.download(pc, a.shape, np.uint32), expect)
+        finally:
+            for ptr in [pa, pb] + pcs:
+                device_memory.free(ptr)
