@@ -5,6 +5,7 @@
 //   1. conversion_gemm      limb bytes x signed byte weights on INT8 MFMA
 //                           (v_mfma_i32_16x16x64_i8), REDC -> residues mod p_k
 //                           [reference: tensor_product<true>, solve.cu:143-250]
+//   (0-2 in one kernel, convert: q of up to 256 limbs; 2 only for few rows)
 //   2. ntt_columns_forward  merged-twist negacyclic NTT stages whose butterfly
 //                           distance spans whole rows  [high_stages, solve.cu:280-382]
 //   3. ntt_rows_product     remaining forward stages, base-case product mod
@@ -19,6 +20,8 @@
 //   6. reconstruct          K = round(E/2^64), T += K*((-P) mod q), carries,
 //                           Barrett reduction by an arbitrary q
 //                           [reconstruct_direct, solve.cu:667-716, generalized]
+//   (5 and 6, and 4 for few rows, in one kernel, crt_reconstruct: q of up to 60
+//   limbs)
 //
 // Signed INT8 MFMA: data bytes u in [0,255] enter as u-128 (XOR 0x80); the
 // weights are signed base-256 digits; the constant 128*sum(weights) is folded
@@ -1300,7 +1303,7 @@ __global__ __launch_bounds__(256, LOGC < 8 ? 4 : 8) void ntt_rows_reg(uint32_t* 
 }
 
 // ---------------------------------------------------------------------------
-// 6'. reconstruction, one wave per coefficient (q wider than 62 limbs): the
+// 6'. reconstruction, one wave per coefficient (q wider than 60 limbs): the
 // coefficient's CRT word sums are coefficient-major (words[i][0 .. L+3]) and
 // each lane takes one of 64 consecutive words per round, so every round is one
 // 512-byte load and one 256-byte store, and N waves (not N lanes) keep the
