@@ -2440,18 +2440,19 @@ constexpr uint32_t kGroupShortLimbs = 128;
 // product spread as if it were alone.
 //
 // `columns`: a lane takes the column stages where it holds whole columns, with
-// as many rows as fragments at most (8, with up to two K steps, is what the
-// registers hold; not in a batch, whose one kernel has three waves per SIMD).
+// as many rows as fragments at most (8 with up to two K steps, 4 with up to
+// eight are what the registers hold; a batch, whose one kernel has three waves
+// per SIMD, keeps the wide waves' own).
 // That saves a pass over the residues and a launch, and is worth wide waves at
 // any number of blocks, whole products in us: N = 4096 with 1 limb 28.3 -> 25.8,
 // with 32 limbs 38.6 -> 36.0, with 125 65.9 -> 61.3, with 256 96.6 -> 89.4; N =
-// 8192 with 2 limbs 28.5 -> 26.3, with 64 64.7 -> 59.7; N = 16384 with 2 limbs
-// 29.2 -> 28.4, with 28 44.1 -> 41.7.
+// 8192 with 2 limbs 28.5 -> 26.3, with 64 64.7 -> 59.7, with 128 94.0 -> 90.9;
+// N = 16384 with 2 limbs 29.2 -> 28.4, with 28 44.1 -> 41.7.
 ConvertPlan convert_plan(const Shape& s, uint32_t tiles, uint32_t want_blocks, bool columns) {
     const uint32_t ksteps = s.conv_k / kTK, chunks = (s.r + 15) / 16;
     const uint32_t ks = ksteps <= 1 ? 1 : ksteps <= 2 ? 2 : ksteps <= 4 ? 4 : ksteps <= 8 ? 8 : 16;
     const bool batch = want_blocks == kConvertGroupBlocks;
-    const uint32_t wide = ks >= 8 ? 2 : 4, most = ks <= 2 && !batch ? 8 : wide;
+    const uint32_t wide = ks >= 8 ? 2 : 4, most = batch ? wide : ks <= 2 ? 8 : ks <= 8 ? 4 : 2;
     const uint32_t rows = columns && s.rows <= most ? s.rows : 1;
     uint32_t nt = rows > wide ? rows : wide;
     if (rows == 1 && !batch && tiles * 4 / nt * chunks < want_blocks / 2) nt = 1;
@@ -2464,7 +2465,7 @@ ConvertPlan convert_plan(const Shape& s, uint32_t tiles, uint32_t want_blocks, b
 #define PM_CONVERT_VARIANTS(X)                                                                         \
     X(1, 1, 1) X(2, 1, 1) X(4, 1, 1) X(8, 1, 1) X(16, 1, 1) X(1, 4, 1) X(2, 4, 1) X(4, 4, 1) X(8, 2, 1) \
         X(16, 2, 1) X(1, 4, 2) X(2, 4, 2) X(4, 4, 2) X(8, 2, 2) X(16, 2, 2) X(1, 4, 4) X(2, 4, 4)       \
-            X(4, 4, 4) X(1, 8, 8) X(2, 8, 8)
+            X(4, 4, 4) X(8, 4, 4) X(1, 8, 8) X(2, 8, 8)
 
 bool conversion_columns(const Shape& s, const TileSet& ts) {
     if (!conversion_short(s) || ts.t0 != 0 || ts.w != ts.count || ts.count != s.n_pad / kTile) return false;

@@ -57,13 +57,14 @@ def test_products(polymul, workloads, oracle, device_memory, n, limbs):
 
 
 @pytest.mark.parametrize("n,limbs", [(4096, 1), (4096, 17), (4096, 64), (4096, 65), (4096, 128), (4096, 129),
-                                     (4096, 256), (8192, 1), (8192, 32), (8192, 33), (8192, 64), (8192, 65), (16384, 1), (16384, 16),
-                                     (16384, 17), (16384, 32), (16384, 33)])
+                                     (4096, 256), (8192, 1), (8192, 32), (8192, 33), (8192, 64), (8192, 65),
+                                     (8192, 128), (8192, 129), (16384, 1), (16384, 16), (16384, 17), (16384, 32),
+                                     (16384, 33)])
 def test_column_stages(polymul, workloads, oracle, device_memory, n, limbs):
     """Two, four and eight transform rows, where the conversion does the forward
-    column stages too if a lane holds whole columns (8192 coefficients above 64
-    limbs and 16384 above 32, or in a batch: it does not): alone, with one
-    operand resident, and in a batch."""
+    column stages too if a lane holds whole columns (8192 coefficients above 128
+    limbs, or 64 in a batch, and 16384 above 32, or in a batch: it does not):
+    alone, with one operand resident, and in a batch."""
     print("[gpu-case] conversion with column stages", n, limbs, flush=True)
     q, a, b = _case(workloads, n, limbs, 94000 + n + limbs)
     a[: n // 2] = workloads.q_minus_one(q)
