@@ -1541,11 +1541,12 @@ struct QuotientWords {
 // of a reconstruction.  Whole waves call reconstruct together.
 template <int G>
 struct LaneWords {
-    uint32_t g;
+    uint32_t g, end;  // end: the lane of word L + 1, the last one that holds anything
     uint32_t ct[4], np[4], qv[6];  // qv[u + 2] = q[4g + u], two words below included
     __device__ __forceinline__ void load(const uint32_t* __restrict__ q, const uint32_t* __restrict__ neg_p,
                                          const uint32_t* __restrict__ corr_t, uint32_t L, uint32_t tw, uint32_t lane) {
         g = lane;
+        end = (L + 1) / 4;
         // (every load unconditional, its index clamped, the value selected after)
 #pragma unroll
         for (uint32_t u = 0; u < 4; ++u) {
@@ -1573,14 +1574,18 @@ struct LaneWords {
         return int32_t(t);
     }
     // Passes each lane's carry to the next lane of its group until none is left;
-    // the last lane's carries add up in `top` (0 on the other lanes).
+    // lane `end`'s carries add up in `top` (0 on the other lanes).  The lanes above
+    // it hold nothing and stay out: a coefficient's top words are often -1 until
+    // the carry from below arrives, and that borrow and its undoing would walk
+    // through every empty lane (128 limbs, 31 empty lanes of 64, N = 4096: 18.0
+    // us with the carries added up by the last lane, 5.8 so).
     __device__ __forceinline__ void settle(uint32_t (&w)[4], int32_t carry, int32_t& top) const {
         for (;;) {
-            if (g == G - 1) top += carry;
+            if (g == end) top += carry;
             int32_t cin;
             if constexpr (G <= 16) cin = __builtin_amdgcn_update_dpp(0, carry, 0x111, 0xF, 0xF, true);  // row_shr:1
             else cin = __shfl_up(carry, 1, 64);
-            if (g == 0) cin = 0;
+            if (g == 0 || g > end) cin = 0;
             if (!__ballot(cin != 0)) break;
             carry = add_carry(w, cin);
         }
@@ -1599,7 +1604,7 @@ struct LaneWords {
     // they are garbage, and so are the words.
     __device__ __forceinline__ void reconstruct(const int64_t (&d)[4], uint64_t qe, uint32_t k32, bool valid,
                                                 uint32_t (&w)[4]) const {
-        const uint32_t lane = threadIdx.x & 63, shift = lane & ~uint32_t(G - 1), last = lane | (G - 1);
+        const uint32_t lane = threadIdx.x & 63, shift = lane & ~uint32_t(G - 1), last = shift + end;
         constexpr uint64_t mask = G == 64 ? ~uint64_t(0) : (uint64_t(1) << (G & 63)) - 1;
         // R = T - Qe*q: this lane's four words and the carry out of them
         const uint64_t q0 = uint32_t(qe), q1 = uint32_t(qe >> 32);
