@@ -50,8 +50,6 @@ typedef uint32_t u32_alias __attribute__((may_alias));
 // waves, each owning a 64x128 slab = 4x8 MFMA 16x16 tiles (128 int32
 // accumulators per lane; two waves per SIMD).  WN is 2, or 1 where whole tiles
 // would leave CUs without a block (gemm_halves).
-constexpr uint32_t kTile = 256;
-constexpr uint32_t kTK = 64;
 constexpr uint32_t kTileBytes = kTile * kTK;  // one operand K step, 16 KB
 constexpr uint32_t kLoads = 2;                // 16-byte loads of B per thread and K step
 constexpr uint32_t kWaveM = 4, kWaveN = 8;    // 16x16 tiles per wave
@@ -1654,7 +1652,6 @@ struct LaneWords {
 // all 64 lanes: N = 8192 with 226 limbs 18.1 us, here 8.1; a
 // batch of 64 small products 70 us, here 25.
 // ---------------------------------------------------------------------------
-constexpr uint32_t kWideWords = 256;
 
 template <int G, int NP>
 __device__ __forceinline__ void reconstruct_wide_body(const int64_t* __restrict__ words, uint32_t* __restrict__ c,
@@ -1753,9 +1750,6 @@ struct CrtFusedArgs {
     uint32_t top_m, top_e, k_shift;
     uint64_t mu;
 };
-
-// Wave rows of the fused kernel: 16 word sums each.
-constexpr uint32_t fused_waves(uint32_t crt_words) { return crt_words <= 16 ? 1 : crt_words <= 32 ? 2 : 4; }
 
 constexpr uint32_t fused_row_words(uint32_t wm) { return 16 * wm + 2; }  // int64 per coefficient, 16-byte rows
 
@@ -2394,20 +2388,6 @@ void launch_pack(const Shape& s, const uint32_t* a, const uint32_t* b, int8_t* p
     check_launch("pack_operands");
 }
 
-namespace {
-
-// Whether a GEMM of `blocks` whole tiles takes halves (WN = 1).  A CU holds one
-// whole tile's block, or two halves, at a time; halves pay when they spread what
-// is left for the last round (up to 128 tiles on 256 CUs) over twice the CUs.
-// CRT GEMM, whole against halves: 128 tiles 31.7 / 22.1 us (N = 8192, 226
-// limbs), 80 tiles 62 / 42, 112 tiles 177 / 117 (N = 1024, 1747 limbs), but 224
-// tiles 202 / 219 and 256 tiles 36.2 / 37.5; conversion GEMM 336 tiles 66 / 55,
-// 456 tiles 190 / 195, 512 tiles 36.1 / 35.2.  With two full rounds and more the
-// last one matters less than the halves' extra weight traffic.
-bool gemm_halves(uint64_t blocks) { return blocks < 512 && (blocks - 1) % 256 < 128; }
-
-}  // namespace
-
 void launch_conversion(const Shape& s, const DeviceTables& t, const int8_t* packed, uint32_t* planes,
                        const TileSet& ts, uint32_t op0, uint32_t nops, hipStream_t stream) {
     check_tiles(s, ts, "conversion_gemm");
@@ -2421,62 +2401,6 @@ void launch_conversion(const Shape& s, const DeviceTables& t, const int8_t* pack
     check_launch("conversion_gemm");
 }
 
-namespace {
-
-// Variant of the short conversion: K steps held in registers (KS), 16-coefficient
-// fragments per wave (NT), transform rows whose column stages a lane does (1:
-// none), splits of the primes over blocks.
-struct ConvertPlan {
-    uint32_t ks, nt, rows, split;
-};
-constexpr uint32_t kConvertBlocks = 512, kConvertGroupBlocks = 64;  // two per CU; a batch's share
-// Up to here a batch's products take the short conversion: 16 K steps in
-// registers would cost the shared kernel a third of its occupancy.
-constexpr uint32_t kGroupShortLimbs = 128;
-
-// `tiles` 256-coefficient tiles in all (of both operands).  Wide waves (NT 2 or
-// 4) read each weight from LDS for 32 or 64 coefficients; where they would
-// leave most of the GPU idle (fewer than want_blocks / 2 blocks even with every
-// 16 primes in a block of their own) waves of 16 coefficients take over: N =
-// 1024 with 8 limbs 3.5 us against 4.3 with 64-coefficient blocks.  Then the
-// primes are split until there are want_blocks blocks.  In a batch the other
-// products fill the GPU, so there want_blocks is small and the waves wide: the
-// batch of 64 small products' conversions take 152 us in all, and 210 with each
-// product spread as if it were alone.
-//
-// `columns`: a lane takes the column stages where it holds whole columns, with
-// as many rows as fragments at most (8 with up to two K steps, 4 with up to
-// eight are what the registers hold; a batch, whose one kernel has three waves
-// per SIMD, keeps the wide waves' own).
-// That saves a pass over the residues and a launch, and is worth wide waves at
-// any number of blocks, whole products in us: N = 4096 with 1 limb 28.3 -> 25.8,
-// with 32 limbs 38.6 -> 36.0, with 125 65.9 -> 61.3, with 256 96.6 -> 89.4; N =
-// 8192 with 2 limbs 28.5 -> 26.3, with 64 64.7 -> 59.7, with 128 94.0 -> 90.9;
-// N = 16384 with 2 limbs 29.2 -> 28.4, with 28 44.1 -> 41.7.
-ConvertPlan convert_plan(const Shape& s, uint32_t tiles, uint32_t want_blocks, bool columns) {
-    const uint32_t ksteps = s.conv_k / kTK, chunks = (s.r + 15) / 16;
-    const uint32_t ks = ksteps <= 1 ? 1 : ksteps <= 2 ? 2 : ksteps <= 4 ? 4 : ksteps <= 8 ? 8 : 16;
-    const bool batch = want_blocks == kConvertGroupBlocks;
-    const uint32_t wide = ks >= 8 ? 2 : 4, most = batch ? wide : ks <= 2 ? 8 : ks <= 8 ? 4 : 2;
-    const uint32_t rows = columns && s.rows <= most ? s.rows : 1;
-    uint32_t nt = rows > wide ? rows : wide;
-    if (rows == 1 && !batch && tiles * 4 / nt * chunks < want_blocks / 2) nt = 1;
-    const uint32_t blocks = tiles * 4 / nt, want = (want_blocks + blocks - 1) / blocks;
-    return ConvertPlan{ks, nt, rows, chunks < want ? chunks : want};
-}
-
-}  // namespace
-
-#define PM_CONVERT_VARIANTS(X)                                                                         \
-    X(1, 1, 1) X(2, 1, 1) X(4, 1, 1) X(8, 1, 1) X(16, 1, 1) X(1, 4, 1) X(2, 4, 1) X(4, 4, 1) X(8, 2, 1) \
-        X(16, 2, 1) X(1, 4, 2) X(2, 4, 2) X(4, 4, 2) X(8, 2, 2) X(16, 2, 2) X(1, 4, 4) X(2, 4, 4)       \
-            X(4, 4, 4) X(8, 4, 4) X(1, 8, 8) X(2, 8, 8)
-
-bool conversion_columns(const Shape& s, const TileSet& ts) {
-    if (!conversion_short(s) || ts.t0 != 0 || ts.w != ts.count || ts.count != s.n_pad / kTile) return false;
-    return convert_plan(s, ts.count, kConvertBlocks, true).rows > 1;
-}
-
 void launch_convert(const Shape& s, const DeviceTables& t, const uint32_t* a, const uint32_t* b, uint32_t* planes,
                     const TileSet& ts, uint32_t op0, uint32_t nops, bool columns, hipStream_t stream) {
     check_tiles(s, ts, "convert");
@@ -2486,6 +2410,7 @@ void launch_convert(const Shape& s, const DeviceTables& t, const uint32_t* a, co
     const ConvertArgs args{s.n, s.n_pad, s.limbs, s.r, s.r_pad, s.conv_rows, ksteps, s.n2, ts, op0};
     const ConvertPlan cp = convert_plan(s, nops * ts.count, kConvertBlocks, columns);
     const dim3 grid(nops * ts.count * 4 / cp.nt, cp.split);
+    if (!convert_compiled(cp)) throw std::logic_error("convert: no kernel of the variant the shape takes");
 #define PM_CONVERT(K, N, R)                                                                              \
     if (cp.ks == K && cp.nt == N && cp.rows == R)                                                        \
         hipLaunchKernelGGL((convert<K, N, R>), grid, dim3(256), convert_lds_bytes(ksteps, s.r, cp.split, R), \
@@ -2501,6 +2426,7 @@ void launch_ntt_forward_columns(const Shape& s, const DeviceTables& t, uint32_t*
     if (s.rows < 2) return;
     const uint32_t ps = s.n_pad, r = s.r_pad, C = s.row_width;
     if (C % 256 == 0 && s.rows <= 64) {
+        if (!columns_compiled(s.rows)) throw std::logic_error("ntt_columns_forward: no kernel of this row count");
         const uint32_t s0 = whole ? 0 : strip_begin, s1 = whole ? C / 256 : strip_end;
         dim3 grid(s1 - s0, s.r, nops);
         switch (s.rows) {
@@ -2521,28 +2447,13 @@ void launch_ntt_forward_columns(const Shape& s, const DeviceTables& t, uint32_t*
     check_launch("ntt_columns_forward");
 }
 
-namespace {
-
-// log2 of the row width the register kernel takes, or 0 where the LDS kernel
-// runs: rows narrower than 128 values, and blocks wider than 8.
-uint32_t row_variant(uint32_t row_width, uint32_t n1) {
-    uint32_t logc = 0;
-    while ((1u << logc) < row_width) ++logc;
-    return logc >= 7 && n1 <= 8 ? logc : 0;
-}
-
-}  // namespace
-
-#define PM_ROWS_VARIANTS(X)                                                                                 \
-    X(7, 1) X(7, 2) X(7, 4) X(7, 8) X(8, 1) X(8, 2) X(8, 4) X(8, 8) X(9, 1) X(9, 2) X(9, 4) X(9, 8) X(10, 1) \
-        X(10, 2) X(10, 4) X(10, 8) X(11, 1) X(11, 2) X(11, 4) X(11, 8)
-
 void launch_ntt_rows_product(const Shape& s, const DeviceTables& t, uint32_t* planes, const uint32_t* bplanes,
                              hipStream_t stream) {
     const uint32_t ps = s.n_pad, r = s.r_pad, logc = row_variant(s.row_width, s.n1);
     if (logc) {
         const uint32_t per = kRowC >> logc;  // primes per block
         const dim3 grid(s.rows, (s.r + per - 1) / per);
+        if (!rows_compiled(logc, s.n1)) throw std::logic_error("ntt_rows_product: no kernel of the variant the shape takes");
 #define PM_ROWS(LC, B)                                                                                      \
     if (logc == LC && s.n1 == B)                                                                            \
         hipLaunchKernelGGL((ntt_rows_reg<LC, B>), grid, dim3(256), 0, stream, planes, bplanes, t.consts,     \
@@ -2562,6 +2473,7 @@ void launch_ntt_inverse_columns(const Shape& s, const DeviceTables& t, uint32_t*
     const bool whole = whole_columns(s, strip_begin, strip_end, "ntt_columns_inverse");
     const uint32_t ps = s.n_pad, ksteps = s.r_pad / 16;
     if (s.row_width % 16 == 0 && s.rows <= 64) {
+        if (!columns_compiled(s.rows)) throw std::logic_error("ntt_columns_inverse: no kernel of this row count");
         const uint32_t g0 = whole ? 0 : strip_begin * 16, g1 = whole ? s.row_width / 16 : strip_end * 16;
         dim3 grid(g1 - g0, s.r_pad / 16);
         switch (s.rows) {
@@ -2588,17 +2500,6 @@ void launch_ntt_inverse_columns(const Shape& s, const DeviceTables& t, uint32_t*
     }
     check_launch("ntt_columns_inverse_tiles");
 }
-
-namespace {
-
-// Whether the CRT GEMM has so few whole tiles that crt_small takes it.  Against
-// halves: 3 tiles 6.4 / 13 us (N = 128, 128 limbs), 8 tiles 12.9 / 30.3 (N =
-// 128, 500 limbs), 32 tiles 13.9 / 18.4 (N = 2048, 226 limbs), 28 tiles 68 / 98
-// (N = 128, 1747 limbs); 80 tiles 63.6 / 41.8, where every wave reading its own
-// operands from L2 starts to bound it.
-bool crt_few_blocks(uint32_t crt_rows, uint32_t tiles) { return crt_rows / kTile * tiles < 48; }
-
-}  // namespace
 
 void launch_crt(const Shape& s, const DeviceTables& t, const int8_t* rtiles, int64_t* words, const TileSet& ts,
                 hipStream_t stream) {
@@ -2674,15 +2575,15 @@ void launch_reconstruct(const Shape& s, const DeviceTables& t, const int64_t* wo
 #define PM_WIDE(G, NP)                                                                                              \
     hipLaunchKernelGGL((reconstruct_wide<G, NP>), dim3(ts.count * (kTile / (256 / G * NP))), dim3(256), 0, stream,   \
                        words, c, t.q, t.neg_p, t.corr_t, t.corr_e, args)
-    // Few coefficients leave the GPU idle either way, and a wave each is the
-    // shorter path: N = 128 with 128 limbs 4.1 us against 6.4.
-    const bool few = ts.count <= 8;
-    if (s.crt_words <= 128 && !few) PM_WIDE(32, 2);
-    else if (s.crt_words <= kWideWords && !few) PM_WIDE(64, 4);
+    switch (reconstruct_variant(s, ts.count)) {
+        case Reconstruction::kLanes32: PM_WIDE(32, 2); break;
+        case Reconstruction::kLanes64: PM_WIDE(64, 4); break;
+        case Reconstruction::kWave:
+            hipLaunchKernelGGL(reconstruct_waves, dim3(ts.count * 64), dim3(256), 0, stream, words, c, t.q, t.neg_p,
+                               t.corr_t, t.corr_e, args);
+            break;
+    }
 #undef PM_WIDE
-    else
-        hipLaunchKernelGGL(reconstruct_waves, dim3(ts.count * 64), dim3(256), 0, stream, words, c, t.q, t.neg_p,
-                           t.corr_t, t.corr_e, args);
     check_launch("reconstruct");
 }
 
@@ -2734,6 +2635,14 @@ size_t group_bytes(size_t count) { return group_item_bytes(count) + group_table_
 void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStream_t stream) {
     const uint32_t count = uint32_t(items.size());
     if (!count) return;
+    // A product none of whose variants the grouped kernels hold must not be skipped.
+    for (const GroupItem& it : items) {
+        const uint32_t logc = row_variant(it.row_width, it.n1);
+        const ConvertPlan cp{it.conv_ks, it.conv_nt, it.conv_columns, it.conv_split};
+        if (!columns_compiled(it.rows) || (logc && !rows_compiled(logc, it.n1)) ||
+            (it.limbs <= kGroupShortLimbs && !convert_group_compiled(cp)))
+            throw std::logic_error("launch_group: no kernel of the variant a product takes");
+    }
     const size_t item_bytes = group_item_bytes(count);
     const GroupView* dev_items = static_cast<const GroupView*>(dev_buffer);  // GroupItems, uploaded below
     uint32_t* dev_tables = reinterpret_cast<uint32_t*>(static_cast<char*>(dev_buffer) + item_bytes);

@@ -11,6 +11,7 @@
 #include "chunks.hpp"
 #include "plan.hpp"
 #include "polymul.h"
+#include "variants.hpp"
 
 namespace pm {
 
@@ -35,19 +36,8 @@ struct DeviceWork {
     int64_t* words = nullptr;    // CRT word sums [n_pad][ws] (q wider than 60 limbs, and the debug tap)
 };
 
-// Up to 60 limbs (64 word sums) one kernel does the CRT GEMM and the
-// reconstruction, and the sums stay in LDS; wider q takes the GEMM, then one
-// wave (up to 252 limbs and with more than 8 tiles 32 or 64 lanes, several words
-// each) per coefficient over coefficient-major sums [n_pad][ws] in memory, ws =
-// crt_words rounded up to 16 (128-byte rows) above 64 words.
-constexpr uint32_t kFusedWords = 64;
-inline bool reconstruct_fused(const Shape& s) { return s.crt_words <= kFusedWords; }
-// Up to 8 transform rows, and the whole product at once: the fused kernel reads
-// the row stage's results itself and does the inverse column stages (with one
-// row: none) on their way into its operand layout in LDS.
-inline bool residues_from_planes(const Shape& s, const TileSet& ts) {
-    return s.rows <= 8 && reconstruct_fused(s) && (s.rows == 1 || (ts.t0 == 0 && ts.w == ts.count && ts.count == s.n_pad / 256));
-}
+// Coefficient-major word sums: row stride of one coefficient's crt_words sums,
+// rounded up to 16 (128-byte rows) above 62 limbs.
 inline uint32_t word_stride(const Shape& s) { return s.t_words > 64 ? (s.crt_words + 15) / 16 * 16 : s.crt_words; }
 inline size_t word_sum_elements(const Shape& s) { return size_t(s.n_pad) * word_stride(s); }
 
@@ -77,13 +67,9 @@ void launch_pack(const Shape& s, const uint32_t* a, const uint32_t* b, int8_t* p
 void launch_conversion(const Shape& s, const DeviceTables& t, const int8_t* packed, uint32_t* planes,
                        const TileSet& ts, uint32_t op0, uint32_t nops, hipStream_t stream);
 // Both of the above in one kernel that reads a and b itself (rows as launch_pack),
-// for q of up to kShortLimbs limbs.
-constexpr uint32_t kShortLimbs = 256;
-inline bool conversion_short(const Shape& s) { return s.limbs <= kShortLimbs; }
-// `columns` (only where conversion_columns says so: every tile at once, and two
-// to eight transform rows, fewer for wider q): the forward column stages too,
-// and launch_ntt_forward_columns must not follow.
-bool conversion_columns(const Shape& s, const TileSet& ts);
+// where conversion_short(s).
+// `columns` (only where conversion_columns(s, ts)): the forward column stages
+// too, and launch_ntt_forward_columns must not follow.
 void launch_convert(const Shape& s, const DeviceTables& t, const uint32_t* a, const uint32_t* b, uint32_t* planes,
                     const TileSet& ts, uint32_t op0, uint32_t nops, bool columns, hipStream_t stream);
 // Forward row-spanning (column) stages of column strips [strip_begin,

@@ -1,0 +1,39 @@
+"""Kernel variants on the host (csrc/variants.hpp): every shape's rules name
+variants that are compiled, and a launch whose variant is not refuses instead of
+leaving its buffers unwritten."""
+import re
+import subprocess
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parents[1]
+CSRC = ROOT / "fherma-polynomial-cuda_amd" / "csrc"
+
+
+@pytest.fixture(scope="module")
+def variant_check(tmp_path_factory):
+    exe = tmp_path_factory.mktemp("variants") / "variant_check"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", str(CSRC), str(ROOT / "tests" / "variant_check.cpp"),
+                    "-o", str(exe)], check=True)
+    return lambda *args: subprocess.run([str(exe)] + [str(x) for x in args], check=True, capture_output=True,
+                                        text=True, timeout=100).stdout
+
+
+def test_every_shape_has_its_variants(variant_check):
+    out = variant_check().split()
+    assert out[0] == "ok" and int(out[1]) > 100000
+
+
+def test_every_list_of_variants_is_checked():
+    """Wherever the launch code expands a list of variants into `if`s, the
+    function throws first when the shape's variant is not in the list."""
+    text = (CSRC / "kernels.hip").read_text()
+    for launcher, check in (("launch_convert", "convert_compiled"), ("launch_ntt_rows_product", "rows_compiled"),
+                            ("launch_ntt_forward_columns", "columns_compiled"),
+                            ("launch_ntt_inverse_columns", "columns_compiled"),
+                            ("launch_group", "convert_group_compiled")):
+        body = text[text.index("\nvoid %s(" % launcher):]
+        body = body[:body.index("\n}\n")]
+        first = body.index("hipLaunchKernelGGL")
+        assert re.search(r"if \([^;]*!%s\([^;]*throw std::logic_error" % check, body[:first]), launcher
