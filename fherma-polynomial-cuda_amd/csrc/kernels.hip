@@ -1301,8 +1301,8 @@ __global__ __launch_bounds__(256, LOGC < 8 ? 4 : 8) void ntt_rows_reg(uint32_t* 
 }
 
 // ---------------------------------------------------------------------------
-// 6'. reconstruction, one wave per coefficient (q wider than 60 limbs): the
-// coefficient's CRT word sums are coefficient-major (words[i][0 .. L+3]) and
+// 6'. reconstruction, one wave per coefficient (q wider than 252 limbs, and some
+// widths with few coefficients, reconstruct_variant): the coefficient's CRT word sums are coefficient-major (words[i][0 .. L+3]) and
 // each lane takes one of 64 consecutive words per round, so every round is one
 // 512-byte load and one 256-byte store, and N waves (not N lanes) keep the
 // memory system busy.

@@ -132,9 +132,16 @@ constexpr uint32_t fused_waves(uint32_t crt_words) { return crt_words <= 16 ? 1 
 enum class Reconstruction { kLanes32, kLanes64, kWave };
 constexpr uint32_t kWideWords = 256;
 inline Reconstruction reconstruct_variant(const Shape& s, uint32_t tiles) {
-    // Few coefficients leave the GPU idle either way, and a wave each is the
-    // shorter path: N = 128 with 128 limbs 4.1 us against 6.4.
-    if (tiles <= 8 || s.crt_words > kWideWords) return Reconstruction::kWave;
+    if (s.crt_words > kWideWords) return Reconstruction::kWave;
+    // Up to 8 tiles leave the GPU idle, and the shorter path counts.  That is a
+    // wave each where q's limbs fill whole rounds of 64 words (the round with
+    // q's top words then has no empty words to carry a borrow through), whole
+    // products at N = 128 and 2048 in us, wave against lanes: 64 limbs 30.9 /
+    // 31.2 and 35.6 / 35.6, 127 limbs 1.6 and 1.3 shorter, 128 limbs 33.9 / 35.4
+    // and 48.6 / 50.0, 192 limbs 0.8 and 0.7 shorter.  Elsewhere the lanes are:
+    // 61 limbs 32.6 / 31.1 and 36.2 / 34.2, 100 limbs 33.9 / 32.3 and 41.3 / 39.5,
+    // 160 limbs 37.7 / 37.0 and 56.3 / 55.4, 252 limbs 39.9 / 39.2 and 67.3 / 66.1.
+    if (tiles <= 8 && (s.limbs + 1) % 64 <= 1) return Reconstruction::kWave;
     return s.crt_words <= 128 ? Reconstruction::kLanes32 : Reconstruction::kLanes64;
 }
 

@@ -2,7 +2,7 @@
 it several lanes: the lane of word L + 1 ends the chain, wherever in its four
 words that is, and the lanes above it stay out.  Limb counts on both sides of
 each lane's edge and of each lane count (4, 8, 16, 32 and 64 lanes), through a
-plan's own kernels (more than 8 tiles, or fused) and a batch's, with a q of all
+plan's own kernels (fused, or more than 8 tiles and up to 8) and a batch's, with a q of all
 ones, a power of two, one limb of many, and random, and operands that make the
 quotient estimate miss (q-1, zero).  Bit-exact, so there is no tolerance."""
 import numpy as np
@@ -22,10 +22,13 @@ def _moduli(limbs, workloads, rng):
             "power": power, "short": short}
 
 
-@pytest.mark.parametrize("limbs", LIMBS)
-def test_lane_ends(polymul, workloads, oracle, device_memory, limbs):
-    print("[gpu-case] lane carries", limbs, flush=True)
-    n = 4096 if limbs > 60 else 256
+# up to 8 tiles: a wave per coefficient at 63, 64, 127, 128, 191 and 192 limbs only
+FEW = [(n, limbs) for n in (128, 2048) for limbs in (62, 63, 64, 65, 126, 127, 128, 129, 190, 191, 192, 193)]
+
+
+@pytest.mark.parametrize("n,limbs", [(4096 if limbs > 60 else 256, limbs) for limbs in LIMBS] + FEW)
+def test_lane_ends(polymul, workloads, oracle, device_memory, n, limbs):
+    print("[gpu-case] lane carries", n, limbs, flush=True)
     rng = np.random.default_rng(97000 + limbs)
     for kind, q in _moduli(limbs, workloads, rng).items():
         used = max(i + 1 for i in range(limbs) if q[i])

@@ -25,6 +25,17 @@ def test_every_shape_has_its_variants(variant_check):
     assert out[0] == "ok" and int(out[1]) > 100000
 
 
+@pytest.mark.parametrize("n,limbs,primes,kernel", [
+    (128, 61, 127, "reconstruct_wide<32>"), (128, 63, 131, "reconstruct_waves"), (2048, 64, 133, "reconstruct_waves"),
+    (2048, 65, 135, "reconstruct_wide<32>"), (4096, 64, 133, "reconstruct_wide<32>"),
+    (2048, 124, 257, "reconstruct_wide<32>"), (2048, 125, 259, "reconstruct_wide<64>"),
+    (2048, 128, 265, "reconstruct_waves"), (4096, 128, 265, "reconstruct_wide<64>"),
+    (2048, 252, 521, "reconstruct_wide<64>"), (4096, 253, 523, "reconstruct_waves"),
+])
+def test_reconstruction_of_few_tiles(variant_check, n, limbs, primes, kernel):
+    assert variant_check(n, limbs, primes).splitlines()[-1] == kernel
+
+
 def test_every_list_of_variants_is_checked():
     """Wherever the launch code expands a list of variants into `if`s, the
     function throws first when the shape's variant is not in the list."""
