@@ -168,7 +168,7 @@ pm_status pm_multiply_device_batch(pm_plan* const* plans, const uint32_t* const*
                         hip_check(hipMalloc(&buf.ptr, need), "hipMalloc");
                         buf.bytes = need;
                     }
-                    pm::launch_group(items, buf.ptr, st);
+                    pm::launch_group(std::move(items), buf.ptr, st);
                     hip_check(hipStreamSynchronize(st), "multiply batch");
                 } catch (...) {
                     (void)hipStreamSynchronize(st);

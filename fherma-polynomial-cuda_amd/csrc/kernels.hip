@@ -2596,7 +2596,7 @@ GroupItem group_item(const Shape& s, const DeviceTables& t, const DeviceWork& w,
     it.n1 = s.n1, it.n2 = s.n2, it.rows = s.rows, it.row_width = s.row_width;
     it.s_shift = s.s_shift, it.k_shift = s.k_shift;
     const ConvertPlan cp = convert_plan(s, 2 * s.n_pad / kTile, kConvertGroupBlocks, true);
-    it.conv_ks = cp.ks, it.conv_nt = cp.nt, it.conv_split = cp.split;
+    it.conv_ks = cp.ks, it.conv_nt = cp.nt;  // conv_split: launch_group
     it.conv_columns = s.limbs <= kGroupShortLimbs ? cp.rows : 1;
     it.top_m = barrett_top(s);
     it.top_e = s.s_shift - 32 * it.top_m;
@@ -2632,9 +2632,15 @@ size_t group_table_words(size_t count) { return kGroupLaunches * (2 * count + 1)
 
 size_t group_bytes(size_t count) { return group_item_bytes(count) + group_table_words(count) * sizeof(uint32_t); }
 
-void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStream_t stream) {
+void launch_group(std::vector<GroupItem> items, void* dev_buffer, hipStream_t stream) {
     const uint32_t count = uint32_t(items.size());
     if (!count) return;
+    uint64_t conv_blocks = 0;
+    for (const GroupItem& it : items)
+        if (it.limbs <= kGroupShortLimbs) conv_blocks += convert_group_blocks(it.n, it.conv_nt);
+    for (GroupItem& it : items)
+        if (it.limbs <= kGroupShortLimbs)
+            it.conv_split = convert_group_split((it.r + 15) / 16, convert_group_blocks(it.n, it.conv_nt), conv_blocks);
     // A product none of whose variants the grouped kernels hold must not be skipped.
     for (const GroupItem& it : items) {
         const uint32_t logc = row_variant(it.row_width, it.n1);

@@ -141,10 +141,11 @@ bool groupable(const Shape& s);
 // Bytes of device memory a batch of `count` products needs: the items, then
 // the launches' work lists.
 size_t group_bytes(size_t count);
-// Runs the stages of every item, in order, on `stream`, after copying the items
+// Sets each item's conv_split for the batch, and runs the stages of every item,
+// in order, on `stream`, after copying the items
 // and the work lists (one copy) into `dev_buffer` (group_bytes(items.size())
 // bytes, unused by any launch still queued).
-void launch_group(const std::vector<GroupItem>& items, void* dev_buffer, hipStream_t stream);
+void launch_group(std::vector<GroupItem> items, void* dev_buffer, hipStream_t stream);
 
 // Plan-time table construction on the device (plans built with Tables::kDevice):
 // beta_k, the merged-twist twiddles, both conversion weight matrices and their

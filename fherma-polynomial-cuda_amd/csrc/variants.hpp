@@ -35,7 +35,7 @@ struct ConvertPlan {
     X(1, 4, 1) X(2, 4, 1) X(4, 4, 1) X(8, 2, 1) X(1, 4, 2) X(2, 4, 2) X(4, 4, 2) X(8, 2, 2) X(1, 4, 4) \
         X(2, 4, 4) X(4, 4, 4)
 
-constexpr uint32_t kConvertBlocks = 512, kConvertGroupBlocks = 64;  // two per CU; a batch's share
+constexpr uint32_t kConvertBlocks = 512, kConvertGroupBlocks = 64;  // two per CU; a batch's share at least
 // Up to here a batch's products take the short conversion: 16 K steps in
 // registers would cost the shared kernel a third of its occupancy.
 constexpr uint32_t kGroupShortLimbs = 128;
@@ -45,10 +45,8 @@ constexpr uint32_t kGroupShortLimbs = 128;
 // leave most of the GPU idle (fewer than want_blocks / 2 blocks even with every
 // 16 primes in a block of their own) waves of 16 coefficients take over: N =
 // 1024 with 8 limbs 3.5 us against 4.3 with 64-coefficient blocks.  Then the
-// primes are split until there are want_blocks blocks.  In a batch the other
-// products fill the GPU, so there want_blocks is small and the waves wide: the
-// batch of 64 small products' conversions take 152 us in all, and 210 with each
-// product spread as if it were alone.
+// primes are split until there are want_blocks blocks.  In a batch the waves are
+// wide, and convert_group_split splits the primes.
 //
 // `columns`: a lane takes the column stages where it holds whole columns, with
 // as many rows as fragments at most (8 with up to two K steps, 4 with up to
@@ -70,6 +68,24 @@ inline ConvertPlan convert_plan(const Shape& s, uint32_t tiles, uint32_t want_bl
     const uint32_t blocks = tiles * 4 / nt, want = (want_blocks + blocks - 1) / blocks;
     return ConvertPlan{ks, nt, rows, chunks < want ? chunks : want};
 }
+
+// Splits of a batch product's primes, from its blocks without splits (the ones
+// that hold coefficients) and those of all the batch's products.  Where the
+// others fill the GPU a product needs no more than kConvertGroupBlocks: the batch
+// of 64 small products' conversions took 152 us in all (in four launches then),
+// and 210 with each product spread as if it were alone.  A few products do not fill it, and are spread as
+// far as one alone; in brackets with kConvertGroupBlocks each all the same: one
+// product of N = 4096 with 128 limbs 18.0 us (43.0), two of N = 2048 16.3 (25.6),
+// one of N = 2048 with 100 limbs 9.7 (18.8).  Twice kConvertBlocks was up to 4 %
+// slower (8 products of N = 2048 with 128 limbs) and nowhere faster by more than
+// runs differ.
+inline uint32_t convert_group_split(uint32_t chunks, uint32_t blocks, uint64_t batch_blocks) {
+    const uint64_t own = (kConvertGroupBlocks + blocks - 1) / blocks;
+    const uint64_t fill = (kConvertBlocks + batch_blocks - 1) / batch_blocks;
+    const uint64_t want = own > fill ? own : fill;
+    return uint32_t(want < chunks ? want : chunks);
+}
+inline uint32_t convert_group_blocks(uint32_t n, uint32_t nt) { return 2 * ((n + 64 * nt - 1) / (64 * nt)); }
 
 // Whether the short conversion of the tiles of `ts` takes the forward column
 // stages too: every tile at once, and two to eight transform rows, fewer for

@@ -86,7 +86,17 @@ int main(int argc, char** argv) {
                     }
                     if (limbs > pm::kGroupShortLimbs) continue;
                     const pm::ConvertPlan p = pm::convert_plan(s, 2 * tiles, pm::kConvertGroupBlocks, true);
-                    if (!pm::convert_group_compiled(p) || !p.split) fail("batch", p);
+                    if (!pm::convert_group_compiled(p)) fail("batch", p);
+                    // a batch's product: spread over the GPU where it is alone,
+                    // kConvertGroupBlocks or what one split gives among many
+                    const uint32_t chunks = (r + 15) / 16, blocks = pm::convert_group_blocks(s.n, p.nt);
+                    const uint32_t alone = pm::convert_group_split(chunks, blocks, blocks);
+                    const uint32_t among = pm::convert_group_split(chunks, blocks, 1 << 20);
+                    if (blocks > 2 * tiles * (pm::kTile / (64 * p.nt))) fail("batch blocks", p);
+                    if (alone < 1 || alone > chunks || (alone < chunks && blocks * alone < pm::kConvertBlocks))
+                        fail("alone in a batch", p);
+                    if (among < 1 || among > alone || (among > 1 && blocks * (among - 1) >= pm::kConvertGroupBlocks))
+                        fail("among many in a batch", p);
                 }
     // variants that no rule may name
     for (pm::ConvertPlan p : {pm::ConvertPlan{3, 4, 1, 1}, pm::ConvertPlan{16, 2, 4, 1}, pm::ConvertPlan{8, 8, 8, 1}})
