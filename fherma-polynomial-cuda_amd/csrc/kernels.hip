@@ -27,8 +27,8 @@
 // weights are signed base-256 digits; the constant 128*sum(weights) is folded
 // into per-prime offsets (conversion) and a fixed big-integer correction (CRT).
 //
-// Planes, word sums and scratch use a row stride of n_pad = N rounded up to
-// 256, so every GEMM tile load is in bounds and 16-byte aligned.
+// Planes have a row stride of n_pad = N rounded up to 256, and word sums n_pad
+// rows, so every GEMM tile load is in bounds and 16-byte aligned.
 #include "kernels.hpp"
 
 #include <algorithm>
@@ -301,18 +301,15 @@ __device__ __forceinline__ void gemm_mainloop(const int8_t* __restrict__ a_panel
 // ---------------------------------------------------------------------------
 // 0. operand packing: [N][L] u32 -> [2][n_pad/256][conv_k/64][256][64] bytes,
 //    each byte XOR 0x80 (u -> u-128 as int8); padding words (beyond L, or rows
-//    beyond N) hold the value 0.  One wave per coefficient row (two or four
-//    short rows per wave, below): lane l moves words l, l+64, ... of the row,
-//    so every load reads 256 contiguous bytes and each 128-byte line of the
-//    input is consumed by one wave (a block holds consecutive rows, so only
-//    lines at block edges are shared).
+//    beyond N) hold the value 0.  16 lanes per coefficient row: lane l moves
+//    words l, l+16, ... of the row (a block holds consecutive rows, so only
+//    128-byte lines at block edges are shared).
 // ---------------------------------------------------------------------------
 // Rows of one wave: four rows of 16 lanes each, so that a store instruction
 // writes four consecutive coefficients' 64-byte K-step chunks, 256 contiguous
 // bytes of the packed tile (with one row per wave, it wrote four chunks 16 KB
-// apart: 0.391 against 0.370 ms at N = 65536 with 1747 limbs).  Rows of two K
-// steps (L of 9 to 16 limbs) go two at a time: 32 lanes cover their 32 words.
-constexpr uint32_t pack_rows_per_wave(uint32_t ksteps) { return ksteps == 2 ? 2 : 4; }
+// apart: 0.391 against 0.370 ms at N = 65536 with 1747 limbs).
+constexpr uint32_t kPackRows = 4, kPackSpan = 64 / kPackRows;  // lanes per row
 
 // Packs the tiles of `ts` of operands op0 .. op0+nops-1.  The k-th tile's rows
 // are read from rows k*256 .. k*256+255 of a (or b): the caller passes the
@@ -321,11 +318,11 @@ __device__ __forceinline__ void pack_body(const uint32_t* __restrict__ a, const 
                                           uint32_t* __restrict__ packed, uint32_t n, uint32_t limbs,
                                           uint32_t ksteps, uint32_t ntiles, TileSet ts, uint32_t op0,
                                           uint32_t nops, uint32_t bx) {
-    const uint32_t rpw = pack_rows_per_wave(ksteps), span = 64 / rpw;  // lanes per row
+    constexpr uint32_t span = kPackSpan;
     const uint32_t lane = (threadIdx.x & 63) % span;
     const uint32_t per_op = ts.count * kTile;
     // row over all operands of the launch
-    const uint32_t gr = (bx * 4 + (threadIdx.x >> 6)) * rpw + (threadIdx.x & 63) / span;
+    const uint32_t gr = (bx * 4 + (threadIdx.x >> 6)) * kPackRows + (threadIdx.x & 63) / span;
     if (gr >= nops * per_op) return;
     const uint32_t op = op0 + gr / per_op, rr = gr % per_op;
     const uint32_t tn = tile_at(ts, rr / kTile), row = rr % kTile, coef = tn * kTile + row;
@@ -623,7 +620,7 @@ __global__ __launch_bounds__(256, KS * NT > 16 || NT == 8 ? 2 : 3) void convert(
 // ---------------------------------------------------------------------------
 template <uint32_t WN>
 __device__ __forceinline__ void crt_body(const int8_t* __restrict__ wtiles, const int8_t* __restrict__ rtiles,
-                                         int64_t* __restrict__ words, uint32_t n, uint32_t n_pad, uint32_t crt_rows,
+                                         int64_t* __restrict__ words, uint32_t n, uint32_t crt_rows,
                                          uint32_t kstride, uint32_t ksteps, uint32_t crt_words, uint32_t ws,
                                          TileSet ts, uint32_t bid) {
     PM_GEMM_STAGES(stages);
@@ -662,10 +659,10 @@ __device__ __forceinline__ void crt_body(const int8_t* __restrict__ wtiles, cons
 template <uint32_t WN>
 __global__ __launch_bounds__(256 * WN, 2) void crt_gemm(const int8_t* __restrict__ wtiles,
                                                 const int8_t* __restrict__ rtiles,
-                                                int64_t* __restrict__ words, uint32_t n, uint32_t n_pad,
-                                                uint32_t crt_rows, uint32_t kstride, uint32_t ksteps,
+                                                int64_t* __restrict__ words, uint32_t n, uint32_t crt_rows,
+                                                uint32_t kstride, uint32_t ksteps,
                                                 uint32_t crt_words, uint32_t ws, TileSet ts) {
-    crt_body<WN>(wtiles, rtiles, words, n, n_pad, crt_rows, kstride, ksteps, crt_words, ws, ts, blockIdx.x);
+    crt_body<WN>(wtiles, rtiles, words, n, crt_rows, kstride, ksteps, crt_words, ws, ts, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -869,7 +866,7 @@ __global__ __launch_bounds__(256) void ntt_rows_product(uint32_t* __restrict__ p
                                                         const uint2* __restrict__ twf,
                                                         const uint2* __restrict__ twi, uint32_t ps,
                                                         uint32_t n1, uint32_t n2, uint32_t C,
-                                                        uint32_t rows, uint32_t r) {
+                                                        uint32_t rows) {
     extern __shared__ uint32_t lds32[];
     rows_product_body(planes, bplanes, consts, twf, twi, ps, n1, n2, C, rows, lds32, blockIdx.x, blockIdx.y);
 }
@@ -1941,7 +1938,7 @@ __global__ __launch_bounds__(64 * NW, 4) void crt_reconstruct(const int8_t* __re
 #endif
 struct GroupView {
     uint32_t n, n_pad, limbs, r, r_pad, conv_rows, conv_k, crt_rows, crt_k, crt_words, ws, t_words;
-    uint32_t n1, n2, rows, row_width, s_shift, k_shift, top_m, top_e;
+    uint32_t n1, n2, rows, row_width, k_shift, top_m, top_e;
     uint32_t conv_ks, conv_nt, conv_split, conv_columns;  // short conversion (launch_convert)
     uint64_t mu;
     const PM_GLOBAL PrimeConst* consts;
@@ -2095,7 +2092,7 @@ __global__ __launch_bounds__(256) void inverse_tiles_group(GroupLaunch g) {
 __global__ __launch_bounds__(512) void crt_group(GroupLaunch g) {
     uint32_t local;
     const GroupView& it = group_entry(g, local);
-    crt_body<2>(in_global(it.wcrt), in_global(it.rtiles), in_global(it.words), it.n, it.n_pad, it.crt_rows,
+    crt_body<2>(in_global(it.wcrt), in_global(it.rtiles), in_global(it.words), it.n, it.crt_rows,
                 it.crt_k / kTK, (it.r + 15) / 16, it.crt_words, it.ws, every_tile(it), local);
 }
 
@@ -2380,8 +2377,8 @@ void launch_pack(const Shape& s, const uint32_t* a, const uint32_t* b, int8_t* p
                  uint32_t op0, uint32_t nops, hipStream_t stream) {
     check_tiles(s, ts, "pack_operands");
     const uint32_t ksteps = s.conv_k / kTK, ntiles = s.n_pad / kTile;
-    const size_t rows = size_t(nops) * ts.count * kTile;  // 4 waves per block, 1, 2 or 4 rows per wave
-    const uint32_t per_block = 4 * pack_rows_per_wave(ksteps);
+    const size_t rows = size_t(nops) * ts.count * kTile;  // 4 waves per block
+    const uint32_t per_block = 4 * kPackRows;
     dim3 grid(uint32_t((rows + per_block - 1) / per_block));
     hipLaunchKernelGGL(pack_operands, grid, dim3(256), 0, stream, a, b, reinterpret_cast<uint32_t*>(packed), s.n,
                        s.limbs, ksteps, ntiles, ts, op0, nops);
@@ -2449,7 +2446,7 @@ void launch_ntt_forward_columns(const Shape& s, const DeviceTables& t, uint32_t*
 
 void launch_ntt_rows_product(const Shape& s, const DeviceTables& t, uint32_t* planes, const uint32_t* bplanes,
                              hipStream_t stream) {
-    const uint32_t ps = s.n_pad, r = s.r_pad, logc = row_variant(s.row_width, s.n1);
+    const uint32_t ps = s.n_pad, logc = row_variant(s.row_width, s.n1);
     if (logc) {
         const uint32_t per = kRowC >> logc;  // primes per block
         const dim3 grid(s.rows, (s.r + per - 1) / per);
@@ -2463,7 +2460,7 @@ void launch_ntt_rows_product(const Shape& s, const DeviceTables& t, uint32_t* pl
     } else {
         const dim3 grid(s.rows, s.r);
         hipLaunchKernelGGL(ntt_rows_product, grid, dim3(256), size_t(2) * s.row_width * 4, stream, planes, bplanes,
-                           t.consts, t.tw_fwd, t.tw_inv, ps, s.n1, s.n2, s.row_width, s.rows, r);
+                           t.consts, t.tw_fwd, t.tw_inv, ps, s.n1, s.n2, s.row_width, s.rows);
     }
     check_launch("ntt_rows_product");
 }
@@ -2513,10 +2510,10 @@ void launch_crt(const Shape& s, const DeviceTables& t, const int8_t* rtiles, int
     }
     const uint32_t blocks = (s.crt_rows / kTile) * ts.count;
     if (gemm_halves(blocks))
-        hipLaunchKernelGGL(crt_gemm<1>, dim3(2 * blocks), dim3(256), 0, stream, t.wcrt, rtiles, words, s.n, s.n_pad,
+        hipLaunchKernelGGL(crt_gemm<1>, dim3(2 * blocks), dim3(256), 0, stream, t.wcrt, rtiles, words, s.n,
                            s.crt_rows, s.crt_k / kTK, (s.r + 15) / 16, s.crt_words, word_stride(s), ts);
     else
-        hipLaunchKernelGGL(crt_gemm<2>, dim3(blocks), dim3(512), 0, stream, t.wcrt, rtiles, words, s.n, s.n_pad,
+        hipLaunchKernelGGL(crt_gemm<2>, dim3(blocks), dim3(512), 0, stream, t.wcrt, rtiles, words, s.n,
                            s.crt_rows, s.crt_k / kTK, (s.r + 15) / 16, s.crt_words, word_stride(s), ts);
     check_launch("crt_gemm");
 }
@@ -2594,7 +2591,7 @@ GroupItem group_item(const Shape& s, const DeviceTables& t, const DeviceWork& w,
     it.conv_rows = s.conv_rows, it.conv_k = s.conv_k, it.crt_rows = s.crt_rows, it.crt_k = s.crt_k;
     it.crt_words = s.crt_words, it.ws = word_stride(s), it.t_words = s.t_words;
     it.n1 = s.n1, it.n2 = s.n2, it.rows = s.rows, it.row_width = s.row_width;
-    it.s_shift = s.s_shift, it.k_shift = s.k_shift;
+    it.k_shift = s.k_shift;
     const ConvertPlan cp = convert_plan(s, 2 * s.n_pad / kTile, kConvertGroupBlocks, true);
     it.conv_ks = cp.ks, it.conv_nt = cp.nt;  // conv_split: launch_group
     it.conv_columns = s.limbs <= kGroupShortLimbs ? cp.rows : 1;
@@ -2694,7 +2691,7 @@ void launch_group(std::vector<GroupItem> items, void* dev_buffer, hipStream_t st
         return it.limbs <= kGroupShortLimbs ? uint64_t(it.conv_split) * (8 / it.conv_nt) * ntiles(it) : 0;
     });
     add(kPack, 0, [&](const GroupItem& it) {  // as launch_pack: 2 * ntiles * 256 rows
-        return it.limbs <= kGroupShortLimbs ? 0 : 128 * ntiles(it) / pack_rows_per_wave(it.conv_k / kTK);
+        return it.limbs <= kGroupShortLimbs ? 0 : 128 * ntiles(it) / kPackRows;
     });
     add(kConversion, 0, [&](const GroupItem& it) {
         return it.limbs <= kGroupShortLimbs ? 0 : uint64_t(it.conv_rows / kTile) * 2 * ntiles(it);

@@ -112,7 +112,7 @@ void launch_zero(uint32_t* c, size_t words, hipStream_t stream);
 // them for product item[j] with that product's parameters.
 struct GroupItem {
     uint32_t n, n_pad, limbs, r, r_pad, conv_rows, conv_k, crt_rows, crt_k, crt_words, ws, t_words;
-    uint32_t n1, n2, rows, row_width, s_shift, k_shift, top_m, top_e;
+    uint32_t n1, n2, rows, row_width, k_shift, top_m, top_e;
     uint32_t conv_ks, conv_nt, conv_split, conv_columns;  // short conversion (launch_convert)
     uint64_t mu;
     const PrimeConst* consts;
