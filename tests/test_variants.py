@@ -1,6 +1,7 @@
 """Kernel variants on the host (csrc/variants.hpp): every shape's rules name
 variants that are compiled, and a launch whose variant is not refuses instead of
 leaving its buffers unwritten."""
+import importlib.util
 import re
 import subprocess
 from pathlib import Path
@@ -34,6 +35,21 @@ def test_every_shape_has_its_variants(variant_check):
 ])
 def test_reconstruction_of_few_tiles(variant_check, n, limbs, primes, kernel):
     assert variant_check(n, limbs, primes).splitlines()[-1] == kernel
+
+
+def test_gpu_cases_reach_the_gemm_tiles_they_name(variant_check, polymul):
+    """tests/test_gpu_gemm_variants.py: each case's kernels, and together every
+    variant of the two GEMMs."""
+    spec = importlib.util.spec_from_file_location("gemm_variants", ROOT / "tests" / "test_gpu_gemm_variants.py")
+    cases = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(cases)
+    reached = set()
+    for n, limbs, kernels in cases.CASES:
+        with polymul.Plan(n, 32 * limbs, limbs, cases.case_modulus(limbs), device=False) as plan:
+            taken = variant_check(n, limbs, len(plan.primes())).splitlines()
+        assert set(kernels) <= set(taken), (n, limbs, taken)
+        reached |= {k.split()[0] for k in kernels}
+    assert reached == {"conversion_gemm<1>", "conversion_gemm<2>", "crt_gemm<1>", "crt_gemm<2>", "crt_small"}
 
 
 def test_every_list_of_variants_is_checked():
