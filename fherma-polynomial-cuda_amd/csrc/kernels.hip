@@ -672,7 +672,8 @@ __global__ __launch_bounds__(256 * WN, 2) void crt_gemm(const int8_t* __restrict
 // fragments straight from their tiles, two steps ahead, with no barrier until
 // the waves' sums meet in LDS; each wave then finishes a quarter of them.
 // Consecutive tiles of one XCD share their coefficients.  crt_gemm's three
-// blocks took 18.7 us at N = 128 with 128 limbs, this 6.4.
+// blocks took 18.7 us at N = 128 with 128 limbs, this 6.4.  (Three waves per
+// SIMD leave it 5 registers short: 24 bytes of scratch a lane.)
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void crt_small_body(const int8_t* __restrict__ wtiles, const int8_t* __restrict__ rtiles,
                                                int64_t* __restrict__ words, uint32_t n, uint32_t kstride,
@@ -1646,8 +1647,8 @@ struct LaneWords {
 // NP passes of 256 / G coefficients, whose sums are all loaded ahead; K and Qe
 // by one lane per coefficient as in the fused kernel.
 // reconstruct_waves spends a whole wave on every 64 words and forms K and Qe in
-// all 64 lanes: N = 8192 with 226 limbs 18.1 us, here 8.1; a
-// batch of 64 small products 70 us, here 25.
+// all 64 lanes: N = 8192 with 226 limbs 18.1 us, here 8.4; a
+// batch of 64 small products 70 us, here 23.
 // ---------------------------------------------------------------------------
 
 template <int G, int NP>
@@ -2096,6 +2097,9 @@ __global__ __launch_bounds__(512) void crt_group(GroupLaunch g) {
                 it.crt_k / kTK, (it.r + 15) / 16, it.crt_words, it.ws, every_tile(it), local);
 }
 
+// The variants' quotient arrays add up to 9 KB of LDS here (768 bytes in a kernel
+// of one variant), so that a CU holds three blocks of the widest, not four, and
+// the registers are 12 short (20 bytes of scratch a lane).
 __global__ __launch_bounds__(256, 4) void crt_reconstruct_group(GroupLaunch g) {
     extern __shared__ __attribute__((aligned(16))) int8_t dyn_lds[];
     uint32_t local;

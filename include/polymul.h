@@ -243,7 +243,11 @@ pm_status pm_multiply_batch(const pm_request* requests, size_t count, uint64_t d
  * (0: operand packing, 1: conversion GEMM, 2: forward column NTT, 3: row NTT +
  * product + inverse row NTT, 4: inverse column NTT + CRT tiling, 5: CRT GEMM,
  * 6: reconstruction, 7: total), measured with HIP events on the stream the
- * kernels run on. */
+ * kernels run on.  Where one kernel does several stages its time is one entry's,
+ * and the others are the near-zero time between two events: with q of up to 256
+ * limbs entry 1 includes the packing (0), and with 2 to 8 transform rows of 2048,
+ * fewer for wider q, the forward columns (2); with q of up to 60 limbs entry 5
+ * includes the reconstruction (6), and with up to 8 rows the inverse columns (4). */
 pm_status pm_set_profiling(pm_plan* plan, int enabled);
 pm_status pm_get_stage_times(const pm_plan* plan, float* ms, int count);
 
