@@ -73,12 +73,12 @@ inline ConvertPlan convert_plan(const Shape& s, uint32_t tiles, uint32_t want_bl
 // that hold coefficients) and those of all the batch's products.  Where the
 // others fill the GPU a product needs no more than kConvertGroupBlocks: the batch
 // of 64 small products' conversions took 152 us in all (in four launches then),
-// and 210 with each product spread as if it were alone.  A few products do not fill it, and are spread as
-// far as one alone; in brackets with kConvertGroupBlocks each all the same: one
-// product of N = 4096 with 128 limbs 18.0 us (43.0), two of N = 2048 16.3 (25.6),
-// one of N = 2048 with 100 limbs 9.7 (18.8).  Twice kConvertBlocks was up to 4 %
-// slower (8 products of N = 2048 with 128 limbs) and nowhere faster by more than
-// runs differ.
+// and 210 with each product spread as if it were alone.  A few products do not
+// fill it and are spread as far as one alone, in us (in brackets: split for
+// kConvertGroupBlocks each): one of N = 4096 with 128 limbs 18.0 (43.0), two of
+// N = 2048 16.3 (25.6), one of N = 2048 with 100 limbs 9.7 (18.8).  Twice
+// kConvertBlocks was up to 4 % slower (8 products of N = 2048 with 128 limbs) and
+// nowhere faster by more than runs differ.
 inline uint32_t convert_group_split(uint32_t chunks, uint32_t blocks, uint64_t batch_blocks) {
     const uint64_t own = (kConvertGroupBlocks + blocks - 1) / blocks;
     const uint64_t fill = (kConvertBlocks + batch_blocks - 1) / batch_blocks;
